@@ -126,13 +126,13 @@ void potrf_run(const PotrfPlan &p)
             /* POTRF(k) and the TRSM of the tiles below in one launch */
             double f = nk * (nk * nk / 3.0 + nk / 2.0 + 1.0 / 6.0);
             for (int m = k + 1; m < NT; ++m) f += tsz(m) * nbd * nbd;
-            const int ND = ldt / 64;
             int epoch = 0;
-            int *flags = lane_flags(L, ND * ND, 1, &epoch);
+            int *flags = lane_flags(L, k::panel_flags(ldt), 1, &epoch);
             unsigned *ctr = lane_counters(L);
+            double *ws = lane_panel_scratch(L, k::panel_scratch(ldt));
             timed(CHAMAMD_KERNEL_PANEL, f, sm, [&] {
                 k::panel_factor(tile(k, k), tile(std::min(k + 1, NT - 1), k), (long long)ts, NT - k - 1, ldt, dk,
-                                flags, ctr, epoch, p.d_info, p.nb * k, nvalid, sm);
+                                ws, flags, ctr, epoch, p.d_info, p.nb * k, nvalid, sm);
             });
             if (k + 1 < NT && p.lp_mode >= 0) demote(k);
             return;

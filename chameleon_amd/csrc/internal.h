@@ -83,6 +83,8 @@ struct Lane {
     int flags_n = 0;
     int epoch = 0;
     unsigned *panel_ctr = nullptr;
+    double *panel_ws = nullptr;         /* what the fused panel kernel's workgroups hand one another */
+    size_t panel_ws_n = 0;
 };
 Lane *main_lane();
 hipEvent_t lane_event(Lane *L, size_t i);
@@ -91,6 +93,7 @@ int *lane_flags(Lane *L, int n, int launches, int *epoch);
 /* four counters: [0..1] the fused panel kernel's tickets, [2] the strip
  * solves' task ticket */
 unsigned *lane_counters(Lane *L);
+double *lane_panel_scratch(Lane *L, size_t n);   /* at least n doubles */
 void lane_release(Lane *L);         /* frees flags, counters and events (not the streams) */
 
 struct Context {
@@ -295,8 +298,12 @@ void lacpy_tiles(const double *src, double *dst, int mt, int nt, int ldt, int wd
                  int uplo, hipStream_t s);
 /* chol.hip */
 void potrf_diag(double *Akk, int ldt, double *dinv, int iinfo, int nvalid, int *info, int waves, hipStream_t s);
-void panel_factor(double *T, double *P, long long ts, int S, int ldt, double *dinv, int *flags, unsigned *ctr,
-                  int epoch, int *info, int iinfo, int nvalid, hipStream_t s);
+/* scratch: panel_scratch doubles, flags: panel_flags of them, used by one
+ * panel at a time */
+void panel_factor(double *T, double *P, long long ts, int S, int ldt, double *dinv, double *scratch, int *flags,
+                  unsigned *ctr, int epoch, int *info, int iinfo, int nvalid, hipStream_t s);
+size_t panel_scratch(int ldt);
+int panel_flags(int ldt);
 void trsm_right_lower_trans(double *panel, int ntiles, size_t tile_stride, int ldt, const double *Lkk,
                             const double *dinv, const int *info, hipStream_t s);
 void trsm_right_lower_trans_batched(double *P0, int ntiles, long long pstride, int ldt, const double *L0,

@@ -116,30 +116,6 @@ __device__ __forceinline__ void block16_potrf(double (&a)[16], int lane, int &fa
     }
 }
 
-/* One 16-column step of a 64-row column panel by one wavefront: lanes
- * 0-15 hold the rows of the 16 x 16 diagonal block, lanes 16-63 the rows
- * below it, a[] their 16 columns.  The right-looking Cholesky steps that
- * factor the diagonal block (pivots and column entries read from lanes
- * 0-15) turn the rows below into X = P L16^-T at the same time.  Entries
- * above the diagonal of lanes 0-15 end up meaningless (never read).  rd =
- * 1 / L(l,l) on lanes l < 16; `fail` as in block16_potrf. */
-__device__ __forceinline__ void block16_panel(double (&a)[16], int lane, int &fail, double &rd)
-{
-    fail = 0;
-    rd = 0.0;
-#pragma unroll
-    for (int j = 0; j < 16; ++j) {
-        const double d = readlane_f64(a[j], j);
-        if (fail == 0 && !(d > 0.0)) fail = j + 1;
-        const double r = rsqrt_f64(d);
-        const double lij = a[j] * r;
-        if (lane == j) rd = r;
-        a[j] = lij;
-#pragma unroll
-        for (int k = j + 1; k < 16; ++k) a[k] -= lij * readlane_f64(lij, k);
-    }
-}
-
 /* Column (lane % 16) of the inverse of the lower triangular 16 x 16 block
  * L(r,p) = Ls[r * lds + p], by forward substitution, with the reciprocal
  * diagonal rdiag[r] = 1 / L(r,r). */
@@ -746,36 +722,72 @@ void trsm_right_lower_trans(double *panel, int ntiles, size_t tile_stride, int l
  * in one launch, spread over 64-row units so that the panel is not bounded
  * by one compute unit.
  *
- * Units (one workgroup of 4 wavefronts each, numbered in the order the
- * workgroups start, through a ticket counter):
- *   r < ND      owner of row block r of the diagonal tile (ND = ldt / 64)
- *   r >= ND     one 64-row block of a tile below
- * Every unit walks the 64-column blocks C of the panel left-looking:
- *   R = A(u, C) - sum_{p<C} X(u, p) X(C, p)^T      X(C, .) published by owner C
- *   X(u, C) = R Linv_C^T                           Linv_C published by owner C
- * and owner r, after its blocks C < r, factors its diagonal block
- *   L(r, r) L(r, r)^T = A(r, r) - sum_{p<r} X(r, p) X(r, p)^T
- * and publishes L(r, r)'s inverse.  The SYRK part over p < r-1 is formed
- * before the wait for Linv_{r-1}, so the chain per column block is one
- * 64 x 64 product, one rank-64 update and the 64 x 64 factorisation.
+ * What bounds it is the chain of 64 x 64 diagonal factorisations, so one
+ * workgroup, the chain, makes all of them and nothing on the way from one
+ * to the next goes to another workgroup and back.  Units (one workgroup of 4
+ * wavefronts each, ND = ldt / 64 column blocks, in ticket order):
+ *   chain       for C = 0 .. ND-1, from D(C) and R(C), which hold A(C, C) and
+ *               A(C, C-1) less the products of the column blocks p < C-1:
+ *                 X(C, C-1) = R(C) L(C-1, C-1)^-T          (C > 0)
+ *                 L(C, C) L(C, C)^T = D(C) - X(C, C-1) X(C, C-1)^T
+ *   block (r, C), C < r-1, of the diagonal tile:
+ *                 X(r, C) = (A(r, C) - sum_{p<C} X(r, p) X(C, p)^T) L(C, C)^-T
+ *               taking each product as its operands are published
+ *   R(r), D(r)  the chain's inputs, published while it is on block r-1
+ *   the others  one 64-row block below: X(u, C) for every C, left-looking
+ * L(C, C) travels as M(C): its 16 x 16 blocks below the diagonal, and the
+ * inverses of its four diagonal 16 x 16 blocks.  A product with L(C, C)^-T is
+ * then a block substitution on MFMAs whose results stay in registers (the
+ * result layout of one product is the operand layout of the next): as many
+ * products as with the 64 x 64 inverse, which therefore is off the chain.  It
+ * is still wanted (dinv) by the solves: the unit of R(r) forms block r-1's.
  *
- * Publication: flag F[r * ND + C] set to this launch's epoch once owner r
- * stored X(r, C) (C < r) or L(r, r) and Linv_r (C = r), after a
- * device-scope release.  Published blocks are read with device-scope
- * loads (past the non-coherent L2 of other XCDs).  A unit only waits for
- * flags of owners, and owners only for owners with smaller tickets, which
- * have started: the waits end.  A wait also ends when the info flag is
- * set (a failed pivot) or after a bounded number of polls.             */
+ * Measured on MI355X, the launch alone, against one owner per 64 rows with two
+ * exchanges per link and the 64 x 64 inverse on the chain (us; tile size, tiles
+ * below): 128, 0: 50 -> 37; 256, 27: 109 -> 70; 320, 12: 132 -> 86; 512, 0: 207 ->
+ * 125; 512, 30: 227 -> 166; 512, 63: 301 -> 256.  One link is 14 us (was 25): 1.3
+ * the substitution, 1.0 the first products, 4 x 1.2 the columns, the rest LDS
+ * round trips and barriers between the steps.  With many tiles below, the
+ * FP64 MFMAs are the bound (36 products of 64^3 per row unit, 1.9 us each).
+ *
+ * Publication: a flag set to this launch's epoch after the data was written
+ * with device-scope (coherent) stores, every wave has waited for its stores
+ * to complete and the workgroup has met at a barrier; readers poll the flag
+ * and read with device-scope loads, past the non-coherent L2 of other XCDs
+ * (a release fence would write back the whole L2 at each link).  Everything
+ * published goes through scratch, packed so that 64 units reading one block
+ * spread over the memory channels (the tile's 512-byte column pieces, a power
+ * of two apart, met on a few of them); the tile's own lines are each
+ * touched by one unit of the launch only.
+ *
+ * Every wait ends.  The units go by level (R(L+1), D(L+1) and the blocks
+ * (r, L) for L = 0, 1, ..., then the rows below); the workgroups with tickets
+ * 1 .. nw take every nw-th unit of the diagonal tile in that order, and tickets
+ * are taken in the order in which workgroups start.  A unit of level L waits
+ * for units of lower levels and for the chain's blocks <= L, the chain's block
+ * C for units of levels < C: with the chain and the workgroup of the lowest
+ * unfinished unit resident one of them can go on, and a workgroup that has not
+ * started yet only needs a place that some finished one leaves.  A wait also
+ * ends when the info flag is set (a failed pivot) or after a bounded number
+ * of polls.                                                                */
 
 #define PF_SPIN_LIMIT (1 << 22)
+#define PF_BLK 256                       /* one 16 x 16 block, element (i, j) at i + 16 j   */
+#define PF_LOW (10 * PF_BLK)             /* lower blocks of a 64 x 64 block, packed by rows */
+#define PF_W (2 * PF_LOW + 4096)         /* scratch of one row block: M | D | R             */
+#define PF_X 4096                        /* a published X(r, C), element (i, k) at i + 64 k  */
 
 struct PanelArgs {
     double *T;           /* diagonal tile                                         */
     double *P;           /* first tile below it; tile t at P + t * ts             */
     long long ts;
     int S, ldt, ND;
+    int nw;              /* workgroups that share the units of the diagonal tile   */
     double *dinv;        /* Linv_C at dinv + C * 4096, column-major 64 x 64        */
-    int *flags;          /* ND x ND publication flags                              */
+    double *W;           /* published M, D and R of row block r at W + r * PF_W    */
+    double *XW;          /* published X(r, C) at XW + (r (r - 1) / 2 + C) * PF_X   */
+    int *flags;          /* X(r, C) at r ND + C, M(r) at r ND + r, R(r) at r
+                          * (r > 0), D(r) at ND + r (r > 1)                        */
     unsigned *ctr;       /* [0] tickets taken, [1] workgroups finished (both zero
                           * between launches: the last workgroup clears them)      */
     int epoch;
@@ -786,42 +798,55 @@ struct PanelArgs {
 /* Buffer accesses relative to a tile: one per-lane offset register, the
  * uniform part of each address in a scalar offset.  aux 16 sets sc1, a
  * device-scope (coherent) access, the form of a relaxed device-scope
- * atomic load. */
+ * atomic load or store. */
 typedef __amdgpu_buffer_rsrc_t rsrc_t;
 __device__ __forceinline__ rsrc_t pf_rsrc(const double *p)
 {
     return __builtin_amdgcn_make_buffer_rsrc(const_cast<double *>(p), 0, 0x7fffffff, 0x00020000);
 }
+template <bool DEV = false>
 __device__ __forceinline__ double pf_ld(rsrc_t r, int vo, int so)
 {
-    return __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(r, vo, so, 0));
+    return __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(r, vo, so, DEV ? 16 : 0));
 }
-__device__ __forceinline__ double pf_ld_dev(rsrc_t r, int vo, int so)
-{
-    return __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(r, vo, so, 16));
-}
+template <bool DEV = false>
 __device__ __forceinline__ void pf_st(double v, rsrc_t r, int vo, int so)
 {
     typedef unsigned int u2 __attribute__((ext_vector_type(2)));
-    __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u2, v), r, vo, so, 0);
+    __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u2, v), r, vo, so, DEV ? 16 : 0);
 }
 
-/* Wait for flag idx of this launch; false if the factorisation failed
- * meanwhile (or the poll limit was reached).  Uniform over the workgroup. */
-__device__ bool pf_wait(const PanelArgs &a, int idx, int tid, int *s_bad)
+/* Packed lower blocks.  A block below the diagonal: lane (li, lk) slot s of an
+ * MFMA operand, element (li, lk + 4s), is at block + 64 s + lane.  The inverse
+ * of a diagonal block has element (r, c) at (r ^ c) + 16 c, so that lanes on
+ * consecutive columns (as pf_col16 leaves it) meet different banks too. */
+__device__ __forceinline__ constexpr int pf_low(int i, int j) { return (i * (i + 1) / 2 + j) * PF_BLK; }
+__device__ __forceinline__ int pf_inv(int r, int c) { return (r ^ c) + 16 * c; }
+
+/* One wave's wait for flag idx of this launch; false if the factorisation
+ * failed meanwhile (or the poll limit was reached).  The rows below, hundreds
+ * of units on one flag, poll more rarely (SLEEP x 64 cycles between polls). */
+template <int SLEEP = 1>
+__device__ __forceinline__ bool pf_wave_wait(const PanelArgs &a, int idx)
 {
-    if (tid == 0) {
-        int bad = 0, n = 0;
-        while (__hip_atomic_load(&a.flags[idx], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != a.epoch) {
-            if (__hip_atomic_load(a.info, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0) { bad = 1; break; }
-            if (++n > PF_SPIN_LIMIT) {
-                atomicCAS(a.info, 0, PANEL_STALLED);
-                bad = 1;
-                break;
-            }
-            __builtin_amdgcn_s_sleep(2);
+    for (int n = 0;; ++n) {
+        if (__hip_atomic_load(&a.flags[idx], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == a.epoch) return true;
+        if ((n & 7) == 7 && __hip_atomic_load(a.info, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0) return false;
+        if (n > PF_SPIN_LIMIT) {
+            atomicCAS(a.info, 0, PANEL_STALLED);
+            return false;
         }
-        *s_bad = bad;
+        __builtin_amdgcn_s_sleep(SLEEP);
+    }
+}
+
+/* The same for the workgroup (uniform result), for one or two flags. */
+template <int SLEEP = 1>
+__device__ __forceinline__ bool pf_wait(const PanelArgs &a, int idx, int tid, int *s_bad, int idx2 = -1)
+{
+    if (tid < 64) {
+        const bool ok = pf_wave_wait<SLEEP>(a, idx) && (idx2 < 0 || pf_wave_wait<SLEEP>(a, idx2));
+        if (tid == 0) *s_bad = !ok;
     }
     __syncthreads();
     const int bad = *s_bad;
@@ -829,263 +854,554 @@ __device__ bool pf_wait(const PanelArgs &a, int idx, int tid, int *s_bad)
     return bad == 0;
 }
 
+__device__ __forceinline__ void pf_stores_done() { __builtin_amdgcn_s_waitcnt(0x0F70); }   /* vmcnt(0) */
+__device__ __forceinline__ void pf_set(const PanelArgs &a, int idx)
+{
+    __hip_atomic_store(&a.flags[idx], a.epoch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
 __device__ __forceinline__ void pf_publish(const PanelArgs &a, int idx, int tid)
 {
+    pf_stores_done();
     __syncthreads();
-    if (tid == 0) {
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
-        __hip_atomic_store(&a.flags[idx], a.epoch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (tid == 0) pf_set(a, idx);
+}
+
+/* acc[f] += X[16w + i, k] Y[16f + j, k]^T over one 64-column block (wave w,
+ * lane (i, j) of the result layout): x[q] = X(16w + li, 4q + lk) in
+ * registers, Ys = Y as [k][row] in LDS.  The operands of a step are read
+ * while the step before multiplies, and the order is held: left to itself the
+ * compiler reads them where they are used, an LDS latency in every two
+ * products. */
+__device__ __forceinline__ void pf_mma(const double *Ys, int lane, const double (&x)[16], v4d (&acc)[4])
+{
+    const double *y0 = Ys + (lane >> 4) * 64 + (lane & 15);
+    double y[2][4];
+#pragma unroll
+    for (int f = 0; f < 4; ++f) y[0][f] = y0[16 * f];
+#pragma unroll
+    for (int q = 0; q < 16; ++q) {
+        if (q < 15) {
+#pragma unroll
+            for (int f = 0; f < 4; ++f) y[(q + 1) & 1][f] = y0[256 * (q + 1) + 16 * f];
+        }
+#pragma unroll
+        for (int f = 0; f < 4; ++f) acc[f] = mfma_f64(y[q & 1][f], x[q], acc[f]);
+    }
+    __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);      /* two LDS reads of two operands each, */
+#pragma unroll
+    for (int q = 0; q < 16; ++q) {
+        if (q < 15) __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
+        __builtin_amdgcn_sched_group_barrier(0x008, 4, 0);  /* four products */
     }
 }
 
-/* acc[f] += X[16w + i, 0:64n] Y[16f + j, 0:64n]^T (wave w, lane (i, j) of
- * the result layout).  X: the unit's own rows (plain loads); Y: 64 rows
- * read with device-scope loads and staged in LDS once per 64-column block;
- * the next block is loaded while the current one is multiplied.  */
-__device__ void pf_kloop(const double *X, const double *Y, int ldt, int n, double *Ys, int tid, int wave, int lane,
-                         v4d (&acc)[4])
+/* y <- y L^-T for this wave's 16 rows: slot s of y[f] is column 16f + lk + 4s
+ * of row li on entry and return; Ms holds M (packed). */
+__device__ __forceinline__ void pf_subst(const double *Ms, int lane, v4d (&y)[4])
 {
     const int li = lane & 15, lk = lane >> 4;
-    const rsrc_t rx = pf_rsrc(X), ry = pf_rsrc(Y);
-    const int vx = (16 * wave + li + lk * ldt) * 8;            /* X(16w + li, lk)          */
-    const int vy = ((tid & 63) + (tid >> 6) * ldt) * 8;        /* Y(tid % 64, tid / 64)    */
-    const int c4 = 4 * ldt * 8;                                 /* four columns, in bytes   */
-    double x[16], yst[16];
 #pragma unroll
-    for (int q = 0; q < 16; ++q) x[q] = pf_ld(rx, vx, q * c4);
+    for (int f = 0; f < 4; ++f) {
+        v4d t = y[f];
+        if (f > 0) {
+            v4d acc = zero4d();
 #pragma unroll
-    for (int h = 0; h < 16; ++h) yst[h] = pf_ld_dev(ry, vy, h * c4);
-    for (int p = 0; p < n; ++p) {
-        __syncthreads();
+            for (int i = 0; i < f; ++i)
 #pragma unroll
-        for (int h = 0; h < 16; ++h) Ys[tid + 256 * h] = yst[h];
-        __syncthreads();
-        const bool more = p + 1 < n;
-        const int o = (p + 1) * 16 * c4;
-        if (more) {
-#pragma unroll
-            for (int h = 0; h < 16; ++h) yst[h] = pf_ld_dev(ry, vy, o + h * c4);
+                for (int s = 0; s < 4; ++s) acc = mfma_f64(Ms[pf_low(f, i) + 64 * s + lane], y[i][s], acc);
+            t = t - acc;
         }
-        /* x[q] is consumed by its four products, then refilled with the
-         * next block's value */
+        v4d x = zero4d();
 #pragma unroll
-        for (int q = 0; q < 16; ++q) {
-            const double xq = x[q];
-            if (more) x[q] = pf_ld(rx, vx, o + q * c4);
-#pragma unroll
-            for (int f = 0; f < 4; ++f) acc[f] = mfma_f64(Ys[(4 * q + lk) * 64 + 16 * f + li], xq, acc[f]);
-        }
+        for (int s = 0; s < 4; ++s) x = mfma_f64(Ms[pf_low(f, f) + pf_inv(li, lk + 4 * s)], t[s], x);
+        y[f] = x;
     }
 }
 
-/* Factor the 64 x 64 block in Ld (lower part, zeros above) in place and
- * build its inverse in Lv, by 16-column steps: (1) columns [c0, c0+16)
- * of rows [c0, 64) take the earlier steps' products (MFMA), (2) one
- * wavefront factors that 16-column panel in registers (block16_panel:
- * the diagonal block and, in the same steps, the rows below).  The
- * 16 x 16 inverses are only needed for the 64 x 64 inverse, so the four
- * are formed after the loop, one per wavefront, off the column-to-column
- * chain.  Rd holds 1 / L(i,i) of all 64 columns.  Returns the 1-based
- * column of the first non-positive pivot, 0 if none (uniform). */
-__device__ int pf_factor64(double (*Ld)[OBP], double (*Lb)[16][17], double (*Lv)[OBP], double *Rd, int *s_fail,
-                           int wave, int lane)
+/* d - (block (i, j) of X X^T), X in LDS as Xs[k][row]: lane (li, lk) slot s
+ * is element (li, lk + 4s) of the block. */
+__device__ __forceinline__ v4d pf_syrk(const double *Xs, int i, int j, int lane, v4d d)
+{
+    const double *row = Xs + (lane >> 4) * 64 + (lane & 15);
+#pragma unroll
+    for (int q = 0; q < 16; ++q) d = mfma_f64(-row[256 * q + 16 * j], row[256 * q + 16 * i], d);
+    return d;
+}
+
+/* Sixteen right-looking columns by one wavefront, rows across the lanes:
+ * lanes 0-15 hold the 16 x 16 diagonal block (lower part), the others rows
+ * below it or rows of the identity, which turn into P L16^-T and L16^-T.
+ * The update of column k by column j is a[k] -= (a[j] / d) a_kj with the
+ * pivot d and the unscaled a_kj read from the diagonal lanes: only the
+ * reciprocal (estimate, two Newton steps) is between a pivot and the next,
+ * and the other lane reads go on beside it; the square roots scale all
+ * columns at the end.  Returns the 1-based index of the first non-positive
+ * pivot, 0 if none. */
+__device__ __forceinline__ int pf_col16(double (&a)[16], int lane)
+{
+    double dv = 1.0;                     /* lane j: pivot j */
+#pragma unroll
+    for (int j = 0; j < 16; ++j) {
+        const double d = readlane_f64(a[j], j);
+        double r = __builtin_amdgcn_rcp(d);
+        double s[16];
+#pragma unroll
+        for (int k = j + 1; k < 16; ++k) s[k] = readlane_f64(a[j], k);
+        dv = lane == j ? a[j] : dv;
+        r = fma(fma(-d, r, 1.0), r, r);
+        r = fma(fma(-d, r, 1.0), r, r);
+        const double w = -(a[j] * r);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int k = j + 1; k < 16; ++k) a[k] = fma(w, s[k], a[k]);
+    }
+    const unsigned long long bad = __ballot(!(dv > 0.0));
+    const double rs = rsqrt_f64(dv);
+#pragma unroll
+    for (int j = 0; j < 16; ++j) a[j] *= readlane_f64(rs, j);
+    return __builtin_ffsll((long long)bad);
+}
+
+/* The 64 x 64 inverse from M, into dinv (column-major, zeros above the
+ * diagonal): Z(J, J) = Lb(J), Z(I, J) = -Lb(I) sum_{J<=P<I} L(I, P) Z(P, J);
+ * wave J forms block column J in registers.  Xs: 32 KB of LDS. */
+__device__ __forceinline__ void pf_inverse(const double *Ms, double *Xs, double *dinv, int tid, int wave, int lane)
 {
     const int li = lane & 15, lk = lane >> 4;
-    const int tid = threadIdx.x;
-    if (tid == 0) *s_fail = 0;
-    __syncthreads();
-    for (int cb = 0; cb < 4; ++cb) {
-        const int c0 = 16 * cb;
-        if (cb > 0) {
-            const int rb = wave;
-            if (rb < 4 - cb) {
-                const int r0 = c0 + 16 * rb;
-                v4d acc = zero4d();
-                for (int p = 0; p < c0; p += 4) acc = mfma_f64(Ld[c0 + li][p + lk], Ld[r0 + li][p + lk], acc);
+    v4d z[4];
 #pragma unroll
-                for (int s = 0; s < 4; ++s) {
-                    const int c = lk + 4 * s;
-                    if (rb > 0 || li >= c) Ld[r0 + li][c0 + c] -= acc[s];
-                }
+    for (int I = 0; I < 4; ++I) {
+        z[I] = zero4d();
+        if (I == wave) {
+#pragma unroll
+            for (int s = 0; s < 4; ++s) z[I][s] = Ms[pf_low(I, I) + pf_inv(lk + 4 * s, li)];
+        } else if (I > wave) {
+            v4d t = zero4d();
+#pragma unroll
+            for (int P = 0; P < I; ++P)
+#pragma unroll
+                for (int s = 0; s < 4; ++s) t = mfma_f64(Ms[pf_low(I, P) + 64 * s + lane], z[P][s], t);
+#pragma unroll
+            for (int s = 0; s < 4; ++s) z[I] = mfma_f64(-Ms[pf_low(I, I) + pf_inv(li, lk + 4 * s)], t[s], z[I]);
+        }
+    }
+    __syncthreads();
+    /* element (r, c) at r + 64 c, the row XORed with the column's low bits */
+#pragma unroll
+    for (int I = 0; I < 4; ++I)
+#pragma unroll
+        for (int s = 0; s < 4; ++s) Xs[((16 * I + lk + 4 * s) ^ li) + 64 * (16 * wave + li)] = z[I][s];
+    __syncthreads();
+    for (int e = tid; e < 4096; e += 256) dinv[e] = Xs[e ^ ((e >> 6) & 15)];
+}
+
+/* M(C) from its scratch into LDS (whole workgroup; barriers by the caller) */
+__device__ __forceinline__ void pf_load_m(const double *W, double *Ms, int tid)
+{
+    const rsrc_t r = pf_rsrc(W);
+    double v[10];
+#pragma unroll
+    for (int b = 0; b < 10; ++b) v[b] = pf_ld<true>(r, tid * 8, b * PF_BLK * 8);
+#pragma unroll
+    for (int b = 0; b < 10; ++b) Ms[b * PF_BLK + tid] = v[b];
+}
+
+__device__ __forceinline__ double *pf_xw(const PanelArgs &a, int r, int C)
+{
+    return a.XW + ((size_t)(r * (r - 1) / 2) + C) * PF_X;
+}
+
+struct PanelLds {
+    double Xs[4096];
+    double B[2][PF_LOW];
+    int s_int, s_fail;
+};
+
+/* the chain (see above) */
+__device__ __forceinline__ void panel_chain(const PanelArgs &a, PanelLds &L)
+{
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int li = lane & 15, lk = lane >> 4;
+    const int ldt = a.ldt, ND = a.ND;
+    double *const Xs = L.Xs;
+    if (tid == 0) L.s_fail = L.s_int = 0;
+    /* R(C) and D(C): rv this wave's rows of R, dcol block (wave, 0) of D, drest
+     * blocks (wave, 1) and the wave-th of (2,2), (3,2), (3,3); block rows 0 and
+     * 1 come from the tile, the others from their units */
+    v4d rv[4], dcol = zero4d(), drest[2] = {zero4d(), zero4d()};
+    const int r2i = wave == 1 ? 2 : 3, r2j = wave == 3 ? 3 : 2;
+    const int vt = (li + lk * ldt) * 8;
+    auto tile_at = [&](int i, int j) { return (16 * i + 16 * j * ldt) * 8; };
+    int cur = 0;
+    for (int C = 0; C < ND; ++C, cur ^= 1) {
+        /* Ms: M(C-1), then R(C+1)'s and D(C+1)'s values for wave 0, and from Ld
+         * on the diagonal 16 x 16 blocks of L(C, C) */
+        double *const Db = L.B[cur], *const Ms = L.B[cur ^ 1], *const Ld = Ms + PF_LOW - 4 * PF_BLK;
+        const rsrc_t rM = pf_rsrc(a.W + (size_t)C * PF_W);
+        const rsrc_t rD = pf_rsrc(a.T + 64 * C + (size_t)64 * C * ldt);     /* the diagonal block in the tile */
+        if (C == 0) {
+            double d[10];
+            const int vo = ((tid & 15) + (tid >> 4) * ldt) * 8;
+#pragma unroll
+            for (int b = 0; b < 10; ++b) {
+                const int i = b < 1 ? 0 : b < 3 ? 1 : b < 6 ? 2 : 3, j = b - i * (i + 1) / 2;
+                d[b] = pf_ld(rD, vo, tile_at(i, j));
             }
+#pragma unroll
+            for (int b = 0; b < 10; ++b) Db[b * PF_BLK + tid] = d[b];
             __syncthreads();
-        }
-        if (wave == 0) {
-            /* lane (g, i): row c0 + 16 g + i of the panel, g = 0 the diagonal block */
-            const int row = c0 + 16 * lk + li;
-            const bool valid = row < OB;
-            double a[16];
+        } else {
+            if (wave == 0) {
+                /* fetched by the other waves while this one was factoring */
 #pragma unroll
-            for (int q = 0; q < 16; ++q) a[q] = (valid && (lk > 0 || q <= li)) ? Ld[row][c0 + q] : 0.0;
-            int fail;
-            double rd;
-            block16_panel(a, lane, fail, rd);
-            if (lk == 0) {
+                for (int q = 0; q < 16; ++q) rv[q >> 2][q & 3] = Db[q * 64 + lane];
 #pragma unroll
-                for (int q = 0; q < 16; ++q) Ld[row][c0 + q] = (q <= li) ? a[q] : 0.0;
-                Rd[c0 + li] = rd;
-            } else if (valid) {
-#pragma unroll
-                for (int q = 0; q < 16; ++q) Ld[row][c0 + q] = a[q];
+                for (int s = 0; s < 4; ++s) dcol[s] = Db[(16 + s) * 64 + lane];
             }
-            if (lane == 0 && fail && *s_fail == 0) *s_fail = c0 + fail;
-        }
-        __syncthreads();
-        if (*s_fail) return *s_fail;
-    }
-    /* the four 16 x 16 inverses, one per wavefront */
-    {
-        double col[16];
-        block16_inverse_col(&Ld[16 * wave][16 * wave], OBP, &Rd[16 * wave], lane, col);
-        if (lane < 16) {
-#pragma unroll
-            for (int q = 0; q < 16; ++q) Lb[wave][q][li] = col[q];
-        }
-    }
-    __syncthreads();
-    assemble_inverse(Ld, Lb, Lv, 4, wave, lane);
-    return 0;
-}
-
-__device__ __forceinline__ void panel_unit(const PanelArgs &a, int t, double *Ys, double (*Ld)[OBP],
-                                           double (*Lb)[16][17], double *Rd, int *s_int)
-{
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int li = lane & 15, lk = lane >> 4;
-    const int ND = a.ND, ldt = a.ldt;
-    const bool owner = t < ND;
-    const int r = owner ? t : (t - ND) % ND;
-    double *R = owner ? a.T + 64 * r : a.P + (size_t)((t - ND) / ND) * a.ts + 64 * r;
-    const int nsteps = owner ? r : ND;
-    const int rowo = 16 * wave + li;
-    const rsrc_t rR = pf_rsrc(R);
-    const int vr = (rowo + lk * ldt) * 8;          /* R(rowo, lk) */
-    /* owner r keeps A(r, r) - sum_{p<=C} X(r, p) X(r, p)^T of its diagonal
-     * block in Ld ([row][col]): each X block just published is folded in
-     * while the next one is awaited */
-    for (int C = 0; C < nsteps; ++C) {
-        v4d acc[4] = {zero4d(), zero4d(), zero4d(), zero4d()};
-        if (C > 0) {
-            if (!pf_wait(a, C * ND + C - 1, tid, s_int)) return;
-            pf_kloop(R, a.T + 64 * C, ldt, C, Ys, tid, wave, lane, acc);
-        }
-        double av[4][4];
-#pragma unroll
-        for (int f = 0; f < 4; ++f)
-#pragma unroll
-            for (int s = 0; s < 4; ++s) av[f][s] = pf_ld(rR, vr, (64 * C + 16 * f + 4 * s) * ldt * 8) - acc[f][s];
-        if (!pf_wait(a, C * ND + C, tid, s_int)) return;
-        const rsrc_t rL = pf_rsrc(a.dinv + (size_t)C * 4096);
-        double lv[16];
-#pragma unroll
-        for (int h = 0; h < 16; ++h) lv[h] = pf_ld_dev(rL, tid * 8, h * 2048);
-#pragma unroll
-        for (int h = 0; h < 16; ++h) Ys[tid + 256 * h] = lv[h];
-        __syncthreads();
-        v4d xo[4];
-#pragma unroll
-        for (int f = 0; f < 4; ++f) {
-            xo[f] = zero4d();
-#pragma unroll
-            for (int kq = 0; kq < 16; ++kq)
-                if (kq < 4 * (f + 1)) xo[f] = mfma_f64(Ys[(4 * kq + lk) * 64 + 16 * f + li], av[kq >> 2][kq & 3], xo[f]);
-        }
-#pragma unroll
-        for (int f = 0; f < 4; ++f)
-#pragma unroll
-            for (int s = 0; s < 4; ++s) pf_st(xo[f][s], rR, vr, (64 * C + 16 * f + 4 * s) * ldt * 8);
-        if (owner) {
-            pf_publish(a, r * ND + C, tid);
-            /* at the first column block the diagonal block starts from A(r, r):
-             * its 16 values per lane requested together, ahead of the
-             * products (a load per value behind a run-time test put a
-             * wait after each one) */
-            double base0[4][4];
-            if (C == 0) {
-#pragma unroll
-                for (int f = 0; f < 4; ++f)
-#pragma unroll
-                    for (int s = 0; s < 4; ++s) base0[f][s] = pf_ld(rR, vr, (64 * r + 16 * f + 4 * s) * ldt * 8);
-            }
-            /* rank-64 term X(r, C) X(r, C)^T of the diagonal block: the block
-             * through LDS ([k][row]) as the shared operand */
+            pf_subst(Ms, lane, rv);
 #pragma unroll
             for (int f = 0; f < 4; ++f)
 #pragma unroll
-                for (int s = 0; s < 4; ++s) Ys[(16 * f + lk + 4 * s) * 64 + rowo] = xo[f][s];
+                for (int s = 0; s < 4; ++s) Xs[(16 * f + lk + 4 * s) * 64 + 16 * wave + li] = rv[f][s];
             __syncthreads();
-            v4d a2[4] = {zero4d(), zero4d(), zero4d(), zero4d()};
+            {
+                const v4d x = pf_syrk(Xs, wave, 0, lane, dcol);
 #pragma unroll
-            for (int q = 0; q < 16; ++q) {
-                const double xq = xo[q >> 2][q & 3];
-#pragma unroll
-                for (int f = 0; f < 4; ++f) a2[f] = mfma_f64(Ys[(4 * q + lk) * 64 + 16 * f + li], xq, a2[f]);
+                for (int s = 0; s < 4; ++s) Db[pf_low(wave, 0) + 64 * s + lane] = x[s];
             }
-#pragma unroll
-            for (int f = 0; f < 4; ++f)
-#pragma unroll
-                for (int s = 0; s < 4; ++s) {
-                    const int c = 16 * f + lk + 4 * s;
-                    const double base = C == 0 ? base0[f][s] : Ld[rowo][c];
-                    Ld[rowo][c] = base - a2[f][s];
-                }
+            __syncthreads();
         }
-    }
-    if (!owner) return;
-
-    /* diagonal block of owner r: A(r, r) - sum_p X(r, p) X(r, p)^T, lower part */
-    double (*Lv)[OBP] = reinterpret_cast<double (*)[OBP]>(Ys);
-    __syncthreads();
-    if (r == 0) {
-        /* owner 0 starts the chain from A(0, 0): all 16 loads in flight */
-        double v0[4][4];
+        /* factor the 64 x 64 block in Db, by 16-column steps: wave 0 the
+         * columns, the others what comes after them and the traffic */
+#pragma unroll 1
+        for (int cb = 0; cb < 4; ++cb) {
+            /* wave 3 repeats the first block during the second step, for its
+             * inverse: in the first there is no lane left for the identity */
+            if (wave == 0 || (wave == 3 && cb == 1)) {
+                /* row group lk: block (c + lk, c), lk < nr, then identity rows */
+                const int c = wave == 0 ? cb : 0, nr = wave == 0 ? 4 - cb : 1;
+                const bool row = lk < nr;
+                double *const blk = Db + pf_low(row ? c + lk : c, c);
+                double v[16];
 #pragma unroll
-        for (int f = 0; f < 4; ++f)
+                for (int q = 0; q < 16; ++q) {
+                    const double x = blk[li + 16 * q];
+                    v[q] = row ? x : (q == li ? 1.0 : 0.0);
+                }
+                const int fail = pf_col16(v, lane);
+                if (lk == 0) {
 #pragma unroll
-            for (int s = 0; s < 4; ++s) v0[f][s] = pf_ld(rR, vr, (16 * f + 4 * s) * ldt * 8);
+                    for (int q = 0; q < 16; ++q)
+                        if (cb > 0) Ld[c * PF_BLK + li + 16 * q] = v[q];       /* L(c, c), for the tile */
+                } else if (row) {
 #pragma unroll
-        for (int f = 0; f < 4; ++f)
+                    for (int q = 0; q < 16; ++q) blk[li + 16 * q] = v[q];
+                } else if (lk == nr) {
 #pragma unroll
-            for (int s = 0; s < 4; ++s) {
-                const int c = 16 * f + lk + 4 * s;
-                Ld[rowo][c] = (rowo >= c) ? v0[f][s] : 0.0;
+                    for (int q = 0; q < 16; ++q) blk[pf_inv(q, li)] = q >= li ? v[q] : 0.0;
+                }
+                /* (the padding's own pivots do not count) */
+                const int col = 64 * C + 16 * c + fail;
+                if (lane == 0 && fail && col - 1 < a.nvalid) L.s_fail = col;
+            } else if (cb == 0) {
+                if (C > 0) {
+                    /* publish X(C, C-1) (R(C+1) waits for it), element (row lane, column k) */
+                    const rsrc_t rP = pf_rsrc(pf_xw(a, C, C - 1));
+#pragma unroll
+                    for (int u = 0; u < 22; ++u) {
+                        const int k = min(3 * u + wave - 1, 63);
+                        pf_st<true>(Xs[64 * k + lane], rP, lane * 8, k * 512);
+                    }
+                    /* the products of the columns factored later */
+#pragma unroll
+                    for (int u = 0; u < 2; ++u) {
+                        const int i = u ? r2i : wave, j = u ? r2j : 1;
+                        const v4d x = pf_syrk(Xs, i, j, lane, drest[u]);
+#pragma unroll
+                        for (int s = 0; s < 4; ++s) Db[pf_low(i, j) + 64 * s + lane] = x[s];
+                    }
+                }
+            } else {
+                if (cb == 1 && C > 0) {
+                    if (wave == 1 && lane == 0) pf_set(a, C * ND + C - 1);
+                    /* X(C, C-1) to the tile */
+                    const rsrc_t rX = pf_rsrc(a.T + 64 * C + (size_t)64 * (C - 1) * ldt);
+#pragma unroll 8
+                    for (int k = 32 * (wave - 1); k < 32 * wave; ++k) pf_st(Xs[64 * k + lane], rX, lane * 8, k * ldt * 8);
+                }
+                if (cb < 3) {
+                    /* what step cb-1 takes off the columns after cb: (2,2),
+                     * (3,2), (3,3), then (3,3) */
+                    for (int u = wave - 1; u < (cb == 1 ? 3 : 1); u += 2) {
+                        const int i = u == 0 && cb == 1 ? 2 : 3, j = u == 2 || cb == 2 ? 3 : 2;
+                        v4d x;
+#pragma unroll
+                        for (int s = 0; s < 4; ++s) x[s] = Db[pf_low(i, j) + 64 * s + lane];
+#pragma unroll
+                        for (int s = 0; s < 4; ++s)
+                            x = mfma_f64(-Db[pf_low(j, cb - 1) + 64 * s + lane], Db[pf_low(i, cb - 1) + 64 * s + lane], x);
+#pragma unroll
+                        for (int s = 0; s < 4; ++s) Db[pf_low(i, j) + 64 * s + lane] = x[s];
+                    }
+                }
+                /* publish the finished columns of M and store them to the
+                 * tile: 0 and 1 beside step 2 (waves 2 and 3), 2 beside step 3 */
+                const int j = cb == 2 ? wave - 2 : cb == 3 && wave == 1 ? 2 : -1;
+                if (j >= 0) {
+                    for (int i = j; i < 4; ++i) {
+#pragma unroll
+                        for (int s = 0; s < 4; ++s) {
+                            const double x = Db[pf_low(i, j) + 64 * s + lane];
+                            pf_st<true>(x, rM, lane * 8, (pf_low(i, j) + 64 * s) * 8);
+                            const double y = i == j ? Ld[j * PF_BLK + 64 * s + lane] : x;
+                            if (i > j || li >= lk + 4 * s) pf_st(y, rD, vt, tile_at(i, j) + 32 * s * ldt);
+                        }
+                    }
+                }
+                if (cb == 3 && C + 1 < ND) {
+                    /* R(C+1) and D(C+1), wave 0's share among them */
+                    bool ok = true;
+                    rsrc_t rr, rd;
+                    int vo, sr, sd;      /* strides of one slot */
+                    if (C == 0) {                /* no products yet: from the tile */
+                        rr = pf_rsrc(a.T + 64);
+                        rd = pf_rsrc(a.T + 64 + (size_t)64 * ldt);
+                        vo = vt; sr = sd = 32 * ldt;
+                    } else {
+                        ok = pf_wave_wait(a, C + 1) && pf_wave_wait(a, ND + C + 1);
+                        rr = pf_rsrc(a.W + (size_t)(C + 1) * PF_W + 2 * PF_LOW);
+                        rd = pf_rsrc(a.W + (size_t)(C + 1) * PF_W + PF_LOW);
+                        vo = lane * 8; sr = sd = 512;
+                    }
+                    auto at_r = [&](int w) { return C == 0 ? 128 * w : w * 16 * 512; };
+                    auto at_d = [&](int i, int j) { return C == 0 ? tile_at(i, j) : pf_low(i, j) * 8; };
+                    if (ok) {
+#pragma unroll
+                        for (int q = 0; q < 16; ++q) rv[q >> 2][q & 3] = pf_ld<true>(rr, vo, at_r(wave) + q * sr);
+#pragma unroll
+                        for (int s = 0; s < 4; ++s) {
+                            dcol[s] = pf_ld<true>(rd, vo, at_d(wave, 0) + s * sd);
+                            drest[0][s] = pf_ld<true>(rd, vo, at_d(wave, 1) + s * sd);
+                            drest[1][s] = pf_ld<true>(rd, vo, at_d(r2i, r2j) + s * sd);
+                        }
+                        double t[7];
+#pragma unroll
+                        for (int u = 0; u < 7; ++u) {
+                            const int q = (wave - 1) * 7 + u;
+                            t[u] = q < 16 ? pf_ld<true>(rr, vo, at_r(0) + q * sr)
+                                          : pf_ld<true>(rd, vo, at_d(0, 0) + (q < 20 ? q - 16 : 0) * sd);
+                        }
+#pragma unroll
+                        for (int u = 0; u < 7; ++u) Ms[((wave - 1) * 7 + u) * 64 + lane] = t[u];
+                    } else if (lane == 0) {
+                        L.s_int = 1;
+                    }
+                }
             }
-    } else {
+            if (cb == 0 || cb == 3) pf_stores_done();       /* X(C, C-1); M's columns */
+            __syncthreads();
+            if (L.s_fail) break;
+            if (cb < 3) {
+                /* column cb+1 takes off step cb: block (cb + 1 + wave, cb + 1) */
+                const int i = cb + 1 + wave;
+                if (i < 4) {
+                    v4d x;
 #pragma unroll
-        for (int f = 0; f < 4; ++f)
+                    for (int s = 0; s < 4; ++s) x[s] = Db[pf_low(i, cb + 1) + 64 * s + lane];
 #pragma unroll
-            for (int s = 0; s < 4; ++s) {
-                const int c = 16 * f + lk + 4 * s;
-                if (rowo < c) Ld[rowo][c] = 0.0;
+                    for (int s = 0; s < 4; ++s)
+                        x = mfma_f64(-Db[pf_low(cb + 1, cb) + 64 * s + lane], Db[pf_low(i, cb) + 64 * s + lane], x);
+#pragma unroll
+                    for (int s = 0; s < 4; ++s) Db[pf_low(i, cb + 1) + 64 * s + lane] = x[s];
+                }
+                __syncthreads();
             }
-    }
-    __syncthreads();
-    const int fail = pf_factor64(Ld, Lb, Lv, Rd, s_int, wave, lane);
-    if (fail) {
-        const int col = 64 * r + fail;
-        if (col - 1 < a.nvalid) {
-            if (tid == 0 && __hip_atomic_load(a.info, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 0)
-                __hip_atomic_store(a.info, a.iinfo + col, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+        if (L.s_fail) {
+            if (tid == 0) atomicCAS(a.info, 0, a.iinfo + L.s_fail);
             return;
         }
+        if (L.s_int) return;
+        if (wave == 1) {
+#pragma unroll
+            for (int s = 0; s < 4; ++s)
+                pf_st<true>(Db[pf_low(3, 3) + 64 * s + lane], rM, lane * 8, (pf_low(3, 3) + 64 * s) * 8);
+            pf_stores_done();
+            if (lane == 0) pf_set(a, C * (ND + 1));
+        } else if (wave == 2) {
+#pragma unroll
+            for (int s = 0; s < 4; ++s) {
+                const double y = Ld[3 * PF_BLK + 64 * s + lane];
+                if (li >= lk + 4 * s) pf_st(y, rD, vt, tile_at(3, 3) + 32 * s * ldt);
+            }
+        }
     }
-    double *Tr = a.T + 64 * r + (size_t)(64 * r) * ldt;
-    double *Dv = a.dinv + (size_t)r * 4096;
-    for (int e = tid; e < OB * OB; e += 256) {
-        const int rr = e % OB, cc = e / OB;
-        if (rr >= cc) Tr[rr + (size_t)cc * ldt] = Ld[rr][cc];
-        Dv[e] = Lv[rr][cc];
-    }
-    pf_publish(a, r * ND + r, tid);
+    pf_inverse(L.B[cur ^ 1], Xs, a.dinv + (size_t)(ND - 1) * 4096, tid, wave, lane);
 }
+
+/* Block (r, C) of the diagonal tile below its diagonal blocks; for C = r-1 it
+ * is R(r), left to the chain's substitution, and the 64 x 64 inverse of block
+ * r-1 is formed after it. */
+__device__ __forceinline__ void panel_block(const PanelArgs &a, PanelLds &L, int r, int C)
+{
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int li = lane & 15, lk = lane >> 4;
+    const int ldt = a.ldt, ND = a.ND;
+    const bool is_r = C == r - 1;
+    const rsrc_t rx = pf_rsrc(a.T + 64 * r + (size_t)64 * C * ldt);
+    const int vx = (16 * wave + li + lk * ldt) * 8, c4 = 4 * ldt * 8;
+    const int vp = (16 * wave + li + 64 * lk) * 8;      /* (16w + li, lk) of a published block */
+    v4d y[4];
+    if (r > 1) {
+        double av[16];
+#pragma unroll
+        for (int q = 0; q < 16; ++q) av[q] = pf_ld(rx, vx, q * c4);
+        v4d acc[4] = {zero4d(), zero4d(), zero4d(), zero4d()};
+        for (int p = 0; p < C; ++p) {
+            if (!pf_wait(a, r * ND + p, tid, &L.s_int, C * ND + p)) return;
+            double x[16], yst[16];
+#pragma unroll
+            for (int h = 0; h < 16; ++h) yst[h] = pf_ld<true>(pf_rsrc(pf_xw(a, C, p)), tid * 8, h * 2048);
+#pragma unroll
+            for (int q = 0; q < 16; ++q) x[q] = pf_ld<true>(pf_rsrc(pf_xw(a, r, p)), vp, q * 2048);
+#pragma unroll
+            for (int h = 0; h < 16; ++h) L.Xs[tid + 256 * h] = yst[h];
+            __syncthreads();
+            pf_mma(L.Xs, lane, x, acc);
+        }
+#pragma unroll
+        for (int q = 0; q < 16; ++q) y[q >> 2][q & 3] = av[q] - acc[q >> 2][q & 3];
+    }
+    if (is_r) {
+        if (r > 1) {
+            const rsrc_t rW = pf_rsrc(a.W + (size_t)r * PF_W + 2 * PF_LOW);
+#pragma unroll
+            for (int q = 0; q < 16; ++q) pf_st<true>(y[q >> 2][q & 3], rW, lane * 8, (16 * wave + q) * 512);
+            pf_publish(a, r, tid);
+        }
+    }
+    if (!pf_wait(a, C * (ND + 1), tid, &L.s_int)) return;
+    pf_load_m(a.W + (size_t)C * PF_W, L.B[0], tid);
+    __syncthreads();
+    if (is_r) {
+        pf_inverse(L.B[0], L.Xs, a.dinv + (size_t)C * 4096, tid, wave, lane);
+        return;
+    }
+    pf_subst(L.B[0], lane, y);
+#pragma unroll
+    for (int q = 0; q < 16; ++q) {
+        pf_st<true>(y[q >> 2][q & 3], pf_rsrc(pf_xw(a, r, C)), vp, q * 2048);
+        pf_st(y[q >> 2][q & 3], rx, vx, q * c4);
+    }
+    pf_publish(a, r * ND + C, tid);
+}
+
+/* D(r) = A(r, r) - sum_{p < r-1} X(r, p) X(r, p)^T, lower blocks */
+__device__ __forceinline__ void panel_diag(const PanelArgs &a, PanelLds &L, int r)
+{
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int li = lane & 15, lk = lane >> 4;
+    const int ldt = a.ldt, ND = a.ND;
+    const rsrc_t rx = pf_rsrc(a.T + 64 * r + (size_t)64 * r * ldt);
+    v4d d[3];
+#pragma unroll
+    for (int u = 0; u < 3; ++u) {
+        const int b = min(4 * u + wave, 9), i = b < 1 ? 0 : b < 3 ? 1 : b < 6 ? 2 : 3, j = b - i * (i + 1) / 2;
+#pragma unroll
+        for (int s = 0; s < 4; ++s) d[u][s] = pf_ld(rx, (16 * i + li + lk * ldt) * 8, (16 * j + 4 * s) * ldt * 8);
+    }
+    for (int p = 0; p < r - 1; ++p) {
+        if (!pf_wait(a, r * ND + p, tid, &L.s_int)) return;
+        double yst[16];
+#pragma unroll
+        for (int h = 0; h < 16; ++h) yst[h] = pf_ld<true>(pf_rsrc(pf_xw(a, r, p)), tid * 8, h * 2048);
+#pragma unroll
+        for (int h = 0; h < 16; ++h) L.Xs[tid + 256 * h] = yst[h];
+        __syncthreads();
+#pragma unroll
+        for (int u = 0; u < 3; ++u) {
+            const int b = min(4 * u + wave, 9), i = b < 1 ? 0 : b < 3 ? 1 : b < 6 ? 2 : 3, j = b - i * (i + 1) / 2;
+            d[u] = pf_syrk(L.Xs, i, j, lane, d[u]);
+        }
+    }
+    const rsrc_t rW = pf_rsrc(a.W + (size_t)r * PF_W + PF_LOW);
+#pragma unroll
+    for (int u = 0; u < 3; ++u)
+        if (4 * u + wave < 10) {
+#pragma unroll
+            for (int s = 0; s < 4; ++s) pf_st<true>(d[u][s], rW, lane * 8, ((4 * u + wave) * PF_BLK + 64 * s) * 8);
+        }
+    pf_publish(a, ND + r, tid);
+}
+
+/* X(u, C) of the 64 rows at Rw in a tile below, every C, left-looking.  The
+ * published blocks X(C, p) go through two LDS buffers, one barrier per block;
+ * the loads of a block (and of the unit's own X(u, p)) are issued before the
+ * products of the one before.  64-row blocks per product: 1.7 us of MFMAs. */
+__device__ __forceinline__ void panel_rows(const PanelArgs &a, PanelLds &L, double *Rw)
+{
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int li = lane & 15, lk = lane >> 4;
+    const int ldt = a.ldt, ND = a.ND;
+    const rsrc_t rR = pf_rsrc(Rw);
+    const int vr = (16 * wave + li + lk * ldt) * 8, c4 = 4 * ldt * 8;
+    for (int C = 0; C < ND; ++C) {
+        v4d acc[4] = {zero4d(), zero4d(), zero4d(), zero4d()}, y[4];
+        double av[16];
+#pragma unroll
+        for (int q = 0; q < 16; ++q) av[q] = pf_ld(rR, vr, (16 * C + q) * c4);
+        if (C > 0) {
+            const rsrc_t ry = pf_rsrc(pf_xw(a, C, 0));
+            double x[16], yst[16];
+#pragma unroll
+            for (int q = 0; q < 16; ++q) x[q] = pf_ld(rR, vr, q * c4);
+            /* X(C, C-2) is published after every X(C, p) before it; X(C, C-1)
+             * comes last, from the chain */
+            if (!pf_wait<16>(a, C * ND + max(C - 2, 0), tid, &L.s_int)) return;
+#pragma unroll
+            for (int h = 0; h < 16; ++h) yst[h] = pf_ld<true>(ry, tid * 8, h * 2048);
+#pragma unroll
+            for (int h = 0; h < 16; ++h) L.Xs[tid + 256 * h] = yst[h];
+            __syncthreads();
+            for (int p = 0; p < C; ++p) {
+                double *const cur = p & 1 ? L.B[0] : L.Xs, *const nxt = p & 1 ? L.Xs : L.B[0];
+                double xn[16];
+                if (p + 1 < C) {
+                    if (p + 2 == C && !pf_wait<16>(a, C * ND + C - 1, tid, &L.s_int)) return;
+#pragma unroll
+                    for (int h = 0; h < 16; ++h) yst[h] = pf_ld<true>(ry, tid * 8, (p + 1) * PF_X * 8 + h * 2048);
+#pragma unroll
+                    for (int q = 0; q < 16; ++q) xn[q] = pf_ld(rR, vr, (16 * (p + 1) + q) * c4);
+                }
+                pf_mma(cur, lane, x, acc);
+                if (p + 1 < C) {
+#pragma unroll
+                    for (int h = 0; h < 16; ++h) nxt[tid + 256 * h] = yst[h];
+#pragma unroll
+                    for (int q = 0; q < 16; ++q) x[q] = xn[q];
+                }
+                __syncthreads();
+            }
+        }
+#pragma unroll
+        for (int q = 0; q < 16; ++q) y[q >> 2][q & 3] = av[q] - acc[q >> 2][q & 3];
+        if (!pf_wait<16>(a, C * (ND + 1), tid, &L.s_int)) return;
+        pf_load_m(a.W + (size_t)C * PF_W, L.B[0], tid);
+        __syncthreads();
+        pf_subst(L.B[0], lane, y);
+#pragma unroll
+        for (int q = 0; q < 16; ++q) pf_st(y[q >> 2][q & 3], rR, vr, (16 * C + q) * c4);
+    }
+}
+
+/* units of the diagonal tile besides the chain: level L < ND-1 holds R(L+1),
+ * D(L+1) (L > 0) and the blocks (r, L), r > L+1 */
+__host__ __device__ __forceinline__ int panel_units(int ND) { return ND > 1 ? ND * (ND - 1) / 2 + ND - 2 : 0; }
 
 __global__ __launch_bounds__(256, 2) void panel_factor_kernel(PanelArgs a)
 {
-    __shared__ double Ys[OB * OBP];       /* Y blocks, Linv_C, the inverse being built */
-    __shared__ double Ld[OB][OBP];        /* diagonal block, the last X block          */
-    __shared__ double Lb[4][16][17];
-    __shared__ double Rd[64];
-    __shared__ int s_int, s_ticket, s_info;
+    __shared__ PanelLds L;
+    __shared__ int s_ticket, s_info;
     const int tid = threadIdx.x;
     __builtin_amdgcn_s_setprio(2);        /* critical path: win issue next to update waves */
     if (tid == 0) {
@@ -1093,11 +1409,28 @@ __global__ __launch_bounds__(256, 2) void panel_factor_kernel(PanelArgs a)
         s_info = __hip_atomic_load(a.info, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
     __syncthreads();
+    const int t = __builtin_amdgcn_readfirstlane(s_ticket), nu = panel_units(a.ND);
     /* a ticket past the grid would mean the counters were not cleared */
-    if (s_ticket >= a.ND * (a.S + 1)) {
+    if (t >= (int)gridDim.x) {
         if (tid == 0) atomicCAS(a.info, 0, PANEL_STALLED);
     } else if (s_info == 0) {
-        panel_unit(a, s_ticket, Ys, Ld, Lb, Rd, &s_int);
+        if (t == 0) {
+            panel_chain(a, L);
+        } else if (t <= a.nw) {
+            for (int i = t - 1; i < nu; i += a.nw) {
+                int u = i, lev = 0;
+                for (int len = a.ND - 1; u >= len; len = a.ND - lev) {
+                    u -= len;
+                    ++lev;
+                }
+                __syncthreads();         /* the last unit is done with the LDS */
+                if (lev > 0 && u == 1) panel_diag(a, L, lev + 1);
+                else panel_block(a, L, lev + 1 + (u > 1 ? u - (lev > 0) : u), lev);
+            }
+        } else {
+            const int u = t - 1 - a.nw;
+            panel_rows(a, L, a.P + (size_t)(u / a.ND) * a.ts + 64 * (u % a.ND));
+        }
     }
     __syncthreads();
     if (tid == 0 && atomicAdd(&a.ctr[1], 1u) == gridDim.x - 1) {
@@ -1106,14 +1439,37 @@ __global__ __launch_bounds__(256, 2) void panel_factor_kernel(PanelArgs a)
     }
 }
 
-void panel_factor(double *T, double *P, long long ts, int S, int ldt, double *dinv, int *flags, unsigned *ctr,
-                  int epoch, int *info, int iinfo, int nvalid, hipStream_t s)
+size_t panel_scratch(int ldt)
+{
+    const size_t n = ldt / 64;
+    return n * PF_W + n * (n - 1) / 2 * PF_X;
+}
+int panel_flags(int ldt) { return (ldt / 64) * (ldt / 64) + 1; }
+
+void panel_factor(double *T, double *P, long long ts, int S, int ldt, double *dinv, double *scratch, int *flags,
+                  unsigned *ctr, int epoch, int *info, int iinfo, int nvalid, hipStream_t s)
 {
     PanelArgs a;
     a.T = T; a.P = P; a.ts = ts; a.S = S; a.ldt = ldt; a.ND = ldt / 64;
-    a.dinv = dinv; a.flags = flags; a.ctr = ctr; a.epoch = epoch;
+    a.dinv = dinv; a.W = scratch; a.XW = scratch + (size_t)a.ND * PF_W; a.flags = flags; a.ctr = ctr; a.epoch = epoch;
     a.info = info; a.iinfo = iinfo; a.nvalid = nvalid;
-    const int grid = a.ND * (S + 1);
+    /* As many workgroups as there are units of the diagonal tile, but no more
+     * than leave every 64-row unit below a compute unit of its own, or where
+     * those are too many a place of its own (two on a compute unit), as long
+     * as there are seven: two row units on one compute unit take twice as
+     * long, and one that starts when another has ended doubles the launch
+     * (512-column tile, 30 tiles below: 225 us with 33 workgroups, 166 with
+     * 15; 63 tiles below: 340 us with 33, 256 with 7). */
+    static const int ncu = [] {
+        int dev = 0, n = 0;
+        CHX_HIP(hipGetDevice(&dev));
+        CHX_HIP(hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev));
+        return n;
+    }();
+    const int nu = panel_units(a.ND), least = nu < 7 ? nu : 7, rows = 1 + a.ND * S;
+    const int room = rows + least <= ncu ? ncu - rows : rows + least <= 2 * ncu ? 2 * ncu - rows : nu;
+    a.nw = nu < room ? nu : room;
+    const int grid = 1 + a.nw + a.ND * S;
     hipLaunchKernelGGL(panel_factor_kernel, dim3(grid), dim3(256), 0, s, a);
 }
 

@@ -95,14 +95,28 @@ unsigned *lane_counters(Lane *L)
     return L->panel_ctr;
 }
 
+double *lane_panel_scratch(Lane *L, size_t n)
+{
+    if (n > L->panel_ws_n) {
+        CHX_HIP(hipStreamSynchronize(L->sm));   /* no launch still uses the old one */
+        if (L->panel_ws) CHX_HIP(hipFree(L->panel_ws));
+        CHX_HIP(hipMalloc(&L->panel_ws, n * sizeof(double)));
+        L->panel_ws_n = n;
+    }
+    return L->panel_ws;
+}
+
 void lane_release(Lane *L)
 {
     for (hipEvent_t e : L->events) CHX_HIP(hipEventDestroy(e));
     L->events.clear();
     if (L->flags) CHX_HIP(hipFree(L->flags));
     if (L->panel_ctr) CHX_HIP(hipFree(L->panel_ctr));
+    if (L->panel_ws) CHX_HIP(hipFree(L->panel_ws));
     L->flags = nullptr;
     L->panel_ctr = nullptr;
+    L->panel_ws = nullptr;
+    L->panel_ws_n = 0;
     L->flags_n = 0;
     L->epoch = 0;
 }
