@@ -780,80 +780,92 @@ static void narrow_launch(const NarrowArgs &a, hipStream_t s)
         hipLaunchKernelGGL((strip_narrow_kernel<NCV, true>), dim3(grid), dim3(512), 0, s, a);
 }
 
+/* 64 x 64 products of the two kernels below, P = X Y with X(i, k) at X[i*xi + k*xk]
+ * and Y(k, j) at Y[k*yk + j*yj] in LDS: one wave forms the 16 x 16 block (g, f)
+ * over the 16-column pieces [k0, k1) of k.  Lane (li, lk) slot s is element
+ * (16 g + li, 16 f + lk + 4 s). */
+__device__ __forceinline__ v4d block_product(const double *X, int xi, int xk, const double *Y, int yk, int yj, int g,
+                                             int f, int k0, int k1, int lane)
+{
+    const int li = lane & 15, lk = lane >> 4;
+    const double *x = X + (16 * g + li) * xi + lk * xk, *y = Y + lk * yk + (16 * f + li) * yj;
+    v4d acc = zero4d();
+#pragma unroll
+    for (int q = 0; q < 16; ++q)
+        if (q >= 4 * k0 && q < 4 * k1) acc = mfma_f64(y[4 * q * yk], x[4 * q * xk], acc);
+    return acc;
+}
+
+#define BLD 65           /* leading dimension of a 64 x 64 block in LDS */
+
+/* a 64 x 64 block (leading dimension ld) in registers, then in LDS; `lower`:
+ * its upper triangle taken as zero */
+__device__ __forceinline__ void block_load(const double *src, int ld, int tid, double (&v)[16])
+{
+#pragma unroll
+    for (int h = 0; h < 16; ++h) v[h] = src[(tid & 63) + (size_t)((tid >> 6) + 4 * h) * ld];
+}
+__device__ __forceinline__ void block_store(double *dst, int tid, const double (&v)[16], bool lower)
+{
+    const int i = tid & 63;
+#pragma unroll
+    for (int h = 0; h < 16; ++h) {
+        const int k = (tid >> 6) + 4 * h;
+        dst[i + k * BLD] = !lower || i >= k ? v[h] : 0.0;
+    }
+}
+
 /* D128 of strip s (rows 128 s .. 128 s + 127, inside diagonal tile
  * tm = s / (ldt/128)) from the 64 x 64 inverses Da, Db of its two halves
  * and the factor block L_ba between them:
  *     [ L_aa   0   ]^-1   [ Da               0  ]
  *     [ L_ba  L_bb ]    = [ -Db (L_ba Da)    Db ]
- * The inverses' upper triangles are taken as zero.  One workgroup per
- * strip, each thread a 4 x 4 block of the two 64 x 64 products. */
+ * The inverses' upper triangles are taken as zero.  One workgroup per strip.
+ * It is one link of every narrow solve, and its length is its own: three
+ * loads at once, two times 40 FP64 MFMAs per wave (the triangular halves are
+ * not multiplied; each wave has as many).  With a 4 x 4 block of FMAs per
+ * thread, every operand an LDS read, it took 30 us for a short factor (now 10), 37 at N = 32768 (14). */
 __global__ __launch_bounds__(256) void dinv128_kernel(const double *A, const double *D, long long dts,
                                                       long long doff, int ldd, int NT, int ldt, double *D128)
 {
-    __shared__ double X[64 * 65], Y[64 * 65];
-    const int s = blockIdx.x, tid = threadIdx.x;
+    __shared__ double X[64 * BLD], Y[64 * BLD], Z[64 * BLD];
+    const int s = blockIdx.x, tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int li = lane & 15, lk = lane >> 4;
     const int q = ldt / NSR, tm = s / q, rs = (s % q) * NSR;
     const int qa = ldt / 64, sa = 2 * s, sb = 2 * s + 1;
     const size_t ts = (size_t)ldt * ldt;
-    const double *Da = D + (size_t)(sa / qa) * dts + (size_t)(sa % qa) * doff;
-    const double *Db = D + (size_t)(sb / qa) * dts + (size_t)(sb % qa) * doff;
-    const double *Lba = A + ((size_t)tm * NT + tm) * ts + (rs + 64) + (size_t)rs * ldt;
     double *O = D128 + (size_t)s * NSR * NSR;
-    for (int e = tid; e < 4096; e += 256) {
-        const int i = e & 63, k = e >> 6;
-        X[i + k * 65] = Lba[i + (size_t)k * ldt];
-        Y[i + k * 65] = i >= k ? Da[i + (size_t)k * ldd] : 0.0;
-    }
+    double va[16], vb[16], vl[16];
+    block_load(D + (size_t)(sa / qa) * dts + (size_t)(sa % qa) * doff, ldd, tid, va);
+    block_load(A + ((size_t)tm * NT + tm) * ts + (rs + 64) + (size_t)rs * ldt, ldt, tid, vl);
+    block_load(D + (size_t)(sb / qa) * dts + (size_t)(sb % qa) * doff, ldd, tid, vb);
+    block_store(Y, tid, va, true);
+    block_store(X, tid, vl, false);
+    block_store(Z, tid, vb, true);
     __syncthreads();
-    const int i0 = (tid & 15) * 4, j0 = (tid >> 4) * 4;
-    double g[4][4] = {};
-    for (int k = 0; k < 64; ++k) {
-        double x[4], y[4];
+    /* G = L_ba Da, row group `wave`; Da(k, c) is zero for k < c */
+    v4d g[4];
 #pragma unroll
-        for (int u = 0; u < 4; ++u) {
-            x[u] = X[(i0 + u) + k * 65];
-            y[u] = Y[k + (j0 + u) * 65];
-        }
-#pragma unroll
-        for (int u = 0; u < 4; ++u)
-#pragma unroll
-            for (int v = 0; v < 4; ++v) g[u][v] = fma(x[u], y[v], g[u][v]);
-    }
-    /* top half of the result: [Da 0] */
+    for (int f = 0; f < 4; ++f) g[f] = block_product(X, 1, BLD, Y, 1, BLD, wave, f, f, 4, lane);
+    /* [Da 0] and Db beside it */
     for (int e = tid; e < 64 * NSR; e += 256) {
         const int i = e & 63, j = e >> 6;
-        O[i + (size_t)j * NSR] = j < 64 ? Y[i + j * 65] : 0.0;
+        O[i + (size_t)j * NSR] = j < 64 ? Y[i + j * BLD] : 0.0;
+        if (j < 64) O[(64 + i) + (size_t)(64 + j) * NSR] = Z[i + j * BLD];
     }
     __syncthreads();
 #pragma unroll
-    for (int u = 0; u < 4; ++u)
+    for (int f = 0; f < 4; ++f)
 #pragma unroll
-        for (int v = 0; v < 4; ++v) X[(i0 + u) + (j0 + v) * 65] = g[u][v];
-    for (int e = tid; e < 4096; e += 256) {
-        const int i = e & 63, k = e >> 6;
-        Y[i + k * 65] = i >= k ? Db[i + (size_t)k * ldd] : 0.0;
-    }
+        for (int e = 0; e < 4; ++e) X[16 * wave + li + (16 * f + lk + 4 * e) * BLD] = g[f][e];
     __syncthreads();
-    double c[4][4] = {};
-    for (int k = 0; k < 64; ++k) {
-        double y[4], x[4];
+    /* -Db G, column group `wave`; Db(r, k) is zero for k > r */
 #pragma unroll
-        for (int u = 0; u < 4; ++u) {
-            y[u] = Y[(i0 + u) + k * 65];
-            x[u] = X[k + (j0 + u) * 65];
-        }
+    for (int r = 0; r < 4; ++r) {
+        const v4d c = block_product(Z, 1, BLD, X, 1, BLD, r, wave, 0, r + 1, lane);
 #pragma unroll
-        for (int u = 0; u < 4; ++u)
-#pragma unroll
-            for (int v = 0; v < 4; ++v) c[u][v] = fma(y[u], x[v], c[u][v]);
-    }
-#pragma unroll
-    for (int u = 0; u < 4; ++u)
-#pragma unroll
-        for (int v = 0; v < 4; ++v) O[(64 + i0 + u) + (size_t)(j0 + v) * NSR] = -c[u][v];
-    for (int e = tid; e < 4096; e += 256) {
-        const int i = e & 63, j = e >> 6;
-        O[(64 + i) + (size_t)(64 + j) * NSR] = Y[i + j * 65];
+        for (int e = 0; e < 4; ++e) O[(64 + 16 * r + li) + (size_t)(16 * wave + lk + 4 * e) * NSR] = -c[e];
     }
 }
 
@@ -872,78 +884,50 @@ void dinv128(const double *A, const double *D, long long dts, long long doff, in
  *   backward Eb_s = (L(s+1, s) D_s)^T      for s <= S-2
  * with D_s the 64 x 64 inverse of the diagonal block (upper triangle taken
  * as zero), each 64 x 64 at E + s*4096, element (r, p) at r + p*64.  One
- * workgroup per strip, each thread a 4 x 4 block of the products. */
+ * workgroup per strip, its three blocks loaded at once and 2 x 40 FP64 MFMAs
+ * per wave, as dinv128_kernel (27 us with a 4 x 4 block of FMAs per thread,
+ * now 7; at N = 32768 46, now 23). */
 __global__ __launch_bounds__(256) void strip_products_kernel(const double *A, const double *D, long long dts,
                                                              long long doff, int ldd, int NT, int ldt, double *Ef,
                                                              double *Eb)
 {
-    __shared__ double Dl[64 * 65], Lb[64 * 65];
-    const int s = blockIdx.x, tid = threadIdx.x, S = NT * ldt / SR;
+    __shared__ double Dl[64 * BLD], Lp[64 * BLD], Ln[64 * BLD];
+    const int s = blockIdx.x, tid = threadIdx.x, lane = tid & 63, S = NT * ldt / SR;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int li = lane & 15, lk = lane >> 4;
     const int q = ldt / SR;
     const size_t ts = (size_t)ldt * ldt;
-    const double *Dg = D + (size_t)(s / q) * dts + (size_t)(s % q) * doff;
     auto block = [&](int row_strip, int col_strip) -> const double * {
         const int tr = row_strip / q, rr = (row_strip % q) * SR, tc = col_strip / q, rc = (col_strip % q) * SR;
         return A + ((size_t)tc * NT + tr) * ts + rr + (size_t)rc * ldt;   /* element (i, k) at i + k*ldt */
     };
-    for (int e = tid; e < 4096; e += 256) {
-        const int i = e & 63, k = e >> 6;
-        Dl[i + k * 65] = i >= k ? Dg[i + (size_t)k * ldd] : 0.0;
-    }
-    const int i0 = (tid & 15) * 4, j0 = (tid >> 4) * 4;
+    double vd[16], vp[16], vn[16];
+    block_load(D + (size_t)(s / q) * dts + (size_t)(s % q) * doff, ldd, tid, vd);
+    /* at the ends the missing neighbour's block is the diagonal one, not used */
+    block_load(block(s, s >= 1 ? s - 1 : s), ldt, tid, vp);
+    block_load(block(s <= S - 2 ? s + 1 : s, s), ldt, tid, vn);
+    block_store(Dl, tid, vd, true);
+    block_store(Lp, tid, vp, false);
+    block_store(Ln, tid, vn, false);
+    __syncthreads();
     if (s >= 1) {
-        const double *L = block(s, s - 1);
-        for (int e = tid; e < 4096; e += 256) {
-            const int i = e & 63, k = e >> 6;
-            Lb[i + k * 65] = L[i + (size_t)k * ldt];
-        }
-        __syncthreads();
-        double g[4][4] = {};
-        for (int k = 0; k < 64; ++k) {
-            double d[4], l[4];
-#pragma unroll
-            for (int u = 0; u < 4; ++u) {
-                d[u] = Dl[(i0 + u) + k * 65];
-                l[u] = Lb[k + (j0 + u) * 65];
-            }
-#pragma unroll
-            for (int u = 0; u < 4; ++u)
-#pragma unroll
-                for (int v = 0; v < 4; ++v) g[u][v] = fma(d[u], l[v], g[u][v]);
-        }
         double *O = Ef + (size_t)s * 4096;
 #pragma unroll
-        for (int u = 0; u < 4; ++u)
+        for (int r = 0; r < 4; ++r) {
+            const v4d c = block_product(Dl, 1, BLD, Lp, 1, BLD, r, wave, 0, r + 1, lane);
 #pragma unroll
-            for (int v = 0; v < 4; ++v) O[(i0 + u) + (j0 + v) * 64] = g[u][v];
+            for (int e = 0; e < 4; ++e) O[(16 * r + li) + (16 * wave + lk + 4 * e) * 64] = c[e];
+        }
     }
     if (s <= S - 2) {
-        const double *L = block(s + 1, s);
-        __syncthreads();                  /* Lb no longer read */
-        for (int e = tid; e < 4096; e += 256) {
-            const int i = e & 63, k = e >> 6;
-            Lb[i + k * 65] = L[i + (size_t)k * ldt];
-        }
-        __syncthreads();
-        /* G = L(s+1, s) D_s; Eb = G^T: Eb(r, p) = G(p, r) */
-        double g[4][4] = {};
-        for (int k = 0; k < 64; ++k) {
-            double l[4], d[4];
-#pragma unroll
-            for (int u = 0; u < 4; ++u) {
-                l[u] = Lb[(i0 + u) + k * 65];
-                d[u] = Dl[k + (j0 + u) * 65];
-            }
-#pragma unroll
-            for (int u = 0; u < 4; ++u)
-#pragma unroll
-                for (int v = 0; v < 4; ++v) g[u][v] = fma(l[u], d[v], g[u][v]);
-        }
+        /* Eb(r, p) = sum_k D(k, r) L(p, k), k >= r */
         double *O = Eb + (size_t)s * 4096;
 #pragma unroll
-        for (int u = 0; u < 4; ++u)
+        for (int r = 0; r < 4; ++r) {
+            const v4d c = block_product(Dl, BLD, 1, Ln, BLD, 1, r, wave, r, 4, lane);
 #pragma unroll
-            for (int v = 0; v < 4; ++v) O[(j0 + v) + (i0 + u) * 64] = g[u][v];
+            for (int e = 0; e < 4; ++e) O[(16 * r + li) + (16 * wave + lk + 4 * e) * 64] = c[e];
+        }
     }
 }
 
