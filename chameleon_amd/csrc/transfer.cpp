@@ -229,6 +229,7 @@ void download_pieces(Staging *st, CHAM_desc_t *A, Mirror *M, const std::vector<P
         const Piece &pc = ps[p];
         const int k = (int)(p % XFER_CHUNKS);
         CHX_HIP(hipEventSynchronize(st->ev[k]));
+        st->used[k] = false;      /* done, and `s` may be gone at the next use of the chunk */
         const double *h = (const double *)st->host[k];
         const int jb = pc.n * A->nb + pc.c0;
         st->workers->run([&](int w, int nw) {
