@@ -287,8 +287,8 @@ int CHAMELEON_dlacpy_Tile_Async(cham_uplo_t uplo, CHAM_desc_t *A, CHAM_desc_t *B
     if (uplo == ChamUpperLower) mirror_prepare_overwrite(B, MIRROR_NORMAL, false);
     else mirror_acquire(B, MIRROR_NORMAL, false, c->s_main);
     Mirror *MA = mirror_of(A), *MB = mirror_of(B);
-    k::lacpy_tiles((const double *)MA->d, (double *)MB->d, MA->mt, MA->nt, MA->ldt, MA->wdt, A->mb, A->nb, A->m, A->n,
-                   (int)uplo, c->s_main);
+    k::lacpy_tiles((const double *)MA->d, (double *)MB->d, MA->mt, MA->nt, MA->ldt, MA->wdt, MB->ldt, MB->wdt, A->mb,
+                   A->nb, A->m, A->n, (int)uplo, c->s_main);
     MB->diag_identity = MA->diag_identity;
     mirror_mark_written(B);
     return CHAMELEON_SUCCESS;

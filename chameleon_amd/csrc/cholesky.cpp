@@ -300,16 +300,16 @@ void solve_strips_lane(Lane *L, const double *A, const double *dinv, int NT, int
 
 /* B <- A^-1 B with the Lower factor in A: forward then backward solve on
  * the transposed right-hand sides. */
-static void solve_run(const SolvePlan &p, double *A, int NT, int ldt, double *B, int Bnt, int wdt, int *d_info,
-                      double flops)
+static void solve_run(const SolvePlan &p, double *A, int NT, int ldt, double *B, int ldb, int Bnt, int wdt,
+                      int *d_info, double flops)
 {
     Context *c = ctx();
     hipStream_t sm = c->s_main;
     const int nrp = Bnt * wdt;
     timed(CHAMAMD_KERNEL_SOLVE, flops, sm, [&] {
-        k::rhs_transpose(B, p.BT, NT, ldt, wdt, Bnt, 1, sm);
+        k::rhs_transpose(B, p.BT, NT, ldt, ldb, wdt, Bnt, 1, sm);
         solve_pair(p, A, NT, ldt, p.BT, nrp, d_info);
-        k::rhs_transpose(B, p.BT, NT, ldt, wdt, Bnt, 0, sm);
+        k::rhs_transpose(B, p.BT, NT, ldt, ldb, wdt, Bnt, 0, sm);
     });
 }
 
@@ -387,13 +387,13 @@ int potrs_async(cham_uplo_t uplo, CHAM_desc_t *A, CHAM_desc_t *B, RUNTIME_sequen
     mirror_acquire(B, MIRROR_NORMAL, false, c->s_main);
     Mirror *MA = mirror_of(A), *MB = mirror_of(B);
     SeqState *st = seq_state(sequence);
-    if (MB->ldt != MA->ldt) {
+    if (MB->ldt16 != MA->ldt16) {
         error("CHAMELEON_dpotrs", "B tiling does not match A");
         return CHAMELEON_ERR_ILLEGAL_VALUE;
     }
     const int nrp = MB->nt * MB->wdt;
     SolvePlan plan = solve_plan((double *)MA->d, MA->mt, MA->ldt, nrp, st->d_info, B->n);
-    solve_run(plan, (double *)MA->d, MA->mt, MA->ldt, (double *)MB->d, MB->nt, MB->wdt, st->d_info,
+    solve_run(plan, (double *)MA->d, MA->mt, MA->ldt, (double *)MB->d, MB->ldt, MB->nt, MB->wdt, st->d_info,
               2.0 * (double)A->m * (double)A->m * (double)B->n);
     /* a solve wait that ran out is reported through the info flag */
     st->pending_info = true;
@@ -518,7 +518,7 @@ int posv_async(cham_uplo_t uplo, CHAM_desc_t *A, CHAM_desc_t *B, RUNTIME_sequenc
     mirror_acquire(B, MIRROR_NORMAL, false, sm);
     Mirror *MA = mirror_of(A), *MB = mirror_of(B);
     if (c->stream_flush == A && uplo == ChamLower) xfer_stream_begin(A, MA);
-    if (!(potrf_solve_eligible(MA->ldt) && MB->ldt == MA->ldt)) {
+    if (!(potrf_solve_eligible(MA->ldt) && MB->ldt16 == MA->ldt16)) {
         potrf_async(uplo, A, sequence);
         /* the solve kernels return at once when the device info flag is
          * set, so a failed factorisation costs no host round trip here */
@@ -534,7 +534,7 @@ int posv_async(cham_uplo_t uplo, CHAM_desc_t *A, CHAM_desc_t *B, RUNTIME_sequenc
     const size_t npe = n128 ? 0 : 2 * (size_t)NT * ldt * 64;      /* predecessor products */
     double *ws = (double *)workspace(((size_t)NT * dper + (size_t)nrp * NT * ldt + n128 + npe) * sizeof(double));
     double *BT = ws + (size_t)NT * dper;
-    k::rhs_transpose((double *)MB->d, BT, NT, ldt, MB->wdt, MB->nt, 1, sm);
+    k::rhs_transpose((double *)MB->d, BT, NT, ldt, MB->ldt, MB->wdt, MB->nt, 1, sm);
 
     PotrfPlan p;
     p.A = (double *)MA->d;
@@ -550,7 +550,7 @@ int posv_async(cham_uplo_t uplo, CHAM_desc_t *A, CHAM_desc_t *B, RUNTIME_sequenc
     mirror_mark_written(A);
     A->sync = 1;
     /* a failed factorisation leaves B as it was */
-    k::rhs_transpose((double *)MB->d, BT, NT, ldt, MB->wdt, MB->nt, 0, sm, st->d_info);
+    k::rhs_transpose((double *)MB->d, BT, NT, ldt, MB->ldt, MB->wdt, MB->nt, 0, sm, st->d_info);
     mirror_mark_written(B);
     B->sync = 1;
     return CHAMELEON_SUCCESS;

@@ -5,7 +5,8 @@
  * (sub)matrix in HBM: mt x nt tiles stored tile after tile in column-major
  * tile order, each tile padded to ldt x wdt elements (ldt = mb rounded up to
  * a multiple of 16, wdt likewise unless the matrix is a single tile column,
- * where wdt = n rounded up to 16).  Padding is zero off the diagonal tiles
+ * where wdt = n rounded up to 16; square double matrices mostly round up to
+ * 64, see mirror_alloc in runtime.cpp).  Padding is zero off the diagonal tiles
  * and the identity on the padded diagonal of diagonal tiles, so the padded
  * matrix has the same Cholesky factor as the real one with identity blocks
  * in the holes; every kernel therefore works on full ldt x ldt tiles.
@@ -59,6 +60,7 @@ struct Mirror {
     void   *d = nullptr;       /* device tiles                              */
     int     mt = 0, nt = 0;    /* tiles of the submatrix                    */
     int     ldt = 0, wdt = 0;  /* padded tile rows / columns                */
+    int     ldt16 = 0;         /* tile rows rounded up to 16 only           */
     size_t  tile_elems = 0;    /* ldt * wdt                                 */
     size_t  bytes = 0;
     int     eltsize = 8;
@@ -294,8 +296,8 @@ void plrnt(double *d, int mt, int nt, int ldt, int wdt, int mb, int nb, int M, i
 void set_identity(double *d, int ntiles, int ldt, hipStream_t s);
 void norm_partials(const double *d, int mt, int nt, int ldt, int wdt, int mb, int nb, int M, int N, int uplo,
                    int trans, double *colsum, double *rowsum, double *w, hipStream_t s);
-void lacpy_tiles(const double *src, double *dst, int mt, int nt, int ldt, int wdt, int mb, int nb, int M, int N,
-                 int uplo, hipStream_t s);
+void lacpy_tiles(const double *src, double *dst, int mt, int nt, int ldt, int wdt, int dld, int dwd, int mb, int nb,
+                 int M, int N, int uplo, hipStream_t s);
 /* chol.hip */
 void potrf_diag(double *Akk, int ldt, double *dinv, int iinfo, int nvalid, int *info, int waves, hipStream_t s);
 /* scratch: panel_scratch doubles, flags: panel_flags of them, used by one
@@ -421,7 +423,8 @@ void dinv128(const double *A, const double *D, long long dts, long long doff, in
 void solve_coop(const double *A, const double *TN, const double *TT, double *BT, double *W, int NT, int ldt, int nrhs,
                 int trans, const int *info, hipStream_t s);
 /* with info != null, nothing is copied once *info is nonzero */
-void rhs_transpose(double *Bm, double *BT, int NT, int ldt, int wdt, int bnt, int to_bt, hipStream_t s,
+/* ldb: tile rows of B, at most ldt (the rows of BT past them are zero) */
+void rhs_transpose(double *Bm, double *BT, int NT, int ldt, int ldb, int wdt, int bnt, int to_bt, hipStream_t s,
                    const int *info = nullptr);
 /* forward substitution of one tile row right after its panel (dposv) */
 /* the forward tile solve addresses a tile row of the factor and of the

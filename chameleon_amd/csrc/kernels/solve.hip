@@ -1177,9 +1177,9 @@ void fwd_update(const double *A, double *BT, int k, int NT, int ldt, int nrp, co
 }
 
 /* ------------------------------------------------------------------ */
-/* B mirror (NT x bnt tiles of ldt x wdt) <-> BT (nrhs_p x NT*ldt), with
- * nrhs_p = bnt * wdt. */
-__global__ void rhs_transpose_kernel(double *Bm, double *BT, int NT, int ldt, int wdt, int bnt, int to_bt,
+/* B mirror (NT x bnt tiles of ldb x wdt) <-> BT (nrhs_p x NT*ldt), with
+ * nrhs_p = bnt * wdt; rows ldb .. ldt-1 of a tile row are zero in BT. */
+__global__ void rhs_transpose_kernel(double *Bm, double *BT, int NT, int ldt, int ldb, int wdt, int bnt, int to_bt,
                                      const int *info)
 {
     __shared__ double S[32][33];
@@ -1190,12 +1190,13 @@ __global__ void rhs_transpose_kernel(double *Bm, double *BT, int NT, int ldt, in
     const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;
     auto baddr = [&](int r, int c) -> size_t {
         const int m = r / ldt, i = r % ldt, n = c / wdt, j = c % wdt;
-        return ((size_t)n * NT + m) * ldt * wdt + i + (size_t)j * ldt;
+        return ((size_t)n * NT + m) * ldb * wdt + i + (size_t)j * ldb;
     };
+    const bool rpad = ldb < ldt;
     if (to_bt) {
         for (int jj = ty; jj < 32; jj += 8) {
             const int r = r0 + tx, c = c0 + jj;
-            S[tx][jj] = (r < rows && c < nrp) ? Bm[baddr(r, c)] : 0.0;
+            S[tx][jj] = (r < rows && c < nrp && !(rpad && r % ldt >= ldb)) ? Bm[baddr(r, c)] : 0.0;
         }
         __syncthreads();
         for (int jj = ty; jj < 32; jj += 8) {
@@ -1210,17 +1211,17 @@ __global__ void rhs_transpose_kernel(double *Bm, double *BT, int NT, int ldt, in
         __syncthreads();
         for (int jj = ty; jj < 32; jj += 8) {
             const int r = r0 + tx, c = c0 + jj;
-            if (r < rows && c < nrp) Bm[baddr(r, c)] = S[tx][jj];
+            if (r < rows && c < nrp && !(rpad && r % ldt >= ldb)) Bm[baddr(r, c)] = S[tx][jj];
         }
     }
 }
 
-void rhs_transpose(double *Bm, double *BT, int NT, int ldt, int wdt, int bnt, int to_bt, hipStream_t s,
+void rhs_transpose(double *Bm, double *BT, int NT, int ldt, int ldb, int wdt, int bnt, int to_bt, hipStream_t s,
                    const int *info)
 {
     const int rows = NT * ldt, nrp = bnt * wdt;
     dim3 grid((rows + 31) / 32, (nrp + 31) / 32);
-    hipLaunchKernelGGL(rhs_transpose_kernel, grid, dim3(256), 0, s, Bm, BT, NT, ldt, wdt, bnt, to_bt, info);
+    hipLaunchKernelGGL(rhs_transpose_kernel, grid, dim3(256), 0, s, Bm, BT, NT, ldt, ldb, wdt, bnt, to_bt, info);
 }
 
 /* Per-tile transpose of a batch of square tiles (TT -> TN). */

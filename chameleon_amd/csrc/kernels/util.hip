@@ -345,31 +345,33 @@ void norm_partials(const double *d, int mt, int nt, int ldt, int wdt, int mb, in
 }
 
 /* ------------------------------------------------------------------ */
-/* Tile-wise copy of the `uplo` part between two mirrors of equal geometry
- * (src in orientation src_trans, dst in normal orientation). */
-__global__ __launch_bounds__(256) void lacpy_kernel(const double *src, double *dst, Geo g, int uplo)
+/* Tile-wise copy of the `uplo` part between two mirrors of equal tiling (src
+ * in orientation src_trans, dst in normal orientation); dld/dwd are dst's
+ * padded tile sizes, which differ when only one of the two was rounded up. */
+__global__ __launch_bounds__(256) void lacpy_kernel(const double *src, double *dst, Geo g, int dld, int dwd, int uplo)
 {
     const int t = blockIdx.y;
     const int m = t % g.mt, n = t / g.mt;
-    const size_t ts = (size_t)g.ldt * g.wdt;
+    const size_t ts = (size_t)dld * dwd;
     const double *S = src + g.tile(m, n);
-    double *D = dst + g.tile(m, n);
+    double *D = dst + ((size_t)n * g.mt + m) * ts;
     for (size_t e = (size_t)blockIdx.x * blockDim.x + threadIdx.x; e < ts; e += (size_t)gridDim.x * blockDim.x) {
-        const int i = (int)(e % g.ldt), j = (int)(e / g.ldt);
+        const int i = (int)(e % dld), j = (int)(e / dld);
         const int r = m * g.mb + i, c = n * g.nb + j;
         if (uplo == 122 && r < c) continue;
         if (uplo == 121 && r > c) continue;
-        D[e] = S[e];
+        /* past src's tile: padding, zero (src carries no identity here) */
+        D[e] = (i < g.ldt && j < g.wdt) ? S[i + (size_t)j * g.ldt] : 0.0;
     }
 }
 
-void lacpy_tiles(const double *src, double *dst, int mt, int nt, int ldt, int wdt, int mb, int nb, int M, int N,
-                 int uplo, hipStream_t s)
+void lacpy_tiles(const double *src, double *dst, int mt, int nt, int ldt, int wdt, int dld, int dwd, int mb, int nb,
+                 int M, int N, int uplo, hipStream_t s)
 {
     if (mt * nt == 0) return;
     Geo g = geo(mt, nt, ldt, wdt, mb, nb, M, N);
     dim3 grid(16, mt * nt);
-    hipLaunchKernelGGL(lacpy_kernel, grid, dim3(256), 0, s, src, dst, g, uplo);
+    hipLaunchKernelGGL(lacpy_kernel, grid, dim3(256), 0, s, src, dst, g, dld, dwd, uplo);
 }
 
 } /* namespace k */

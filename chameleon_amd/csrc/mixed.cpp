@@ -164,8 +164,8 @@ int backward_error(cham_uplo_t uplo, CHAM_desc_t *A, CHAM_desc_t *X, CHAM_desc_t
     const size_t pv = k::residual_scratch(NT, ldt, nrp);
     double *w = (double *)workspace2((3 * vb + 2 * (size_t)nrp + pv) * sizeof(double));
     double *XT = w, *BT = w + vb, *RT = w + 2 * vb, *nw = w + 3 * vb, *part = nw + 2 * (size_t)nrp;
-    k::rhs_transpose((double *)MX->d, XT, NT, ldt, MX->wdt, MX->nt, 1, s);
-    k::rhs_transpose((double *)MB->d, BT, NT, ldt, MB->wdt, MB->nt, 1, s);
+    k::rhs_transpose((double *)MX->d, XT, NT, ldt, MX->ldt, MX->wdt, MX->nt, 1, s);
+    k::rhs_transpose((double *)MB->d, BT, NT, ldt, MB->ldt, MB->wdt, MB->nt, 1, s);
     k::residual((const double *)MA->d, NT, ldt, XT, BT, RT, nrp, part, s);
     std::vector<double> xn, rn;
     colmax_pair_host(XT, RT, nrp, rows, nw, xn, rn);
@@ -195,7 +195,8 @@ int mixed_posv(cham_uplo_t uplo, CHAM_desc_t *A, CHAM_desc_t *B, CHAM_desc_t *X,
     const double eps = std::ldexp(1.0, -53);
     int it_count = 0;
     double worst = 0.0;
-    bool converged = false, lp_ok = (ldt % 128 == 0);
+    /* the tile size the caller sees decides, not the mirror's padding */
+    bool converged = false, lp_ok = (MA->ldt16 % 128 == 0);
 
     RUNTIME_sequence_t *seq = nullptr;
     CHAMELEON_Sequence_Create(&seq);
@@ -245,7 +246,7 @@ int mixed_posv(cham_uplo_t uplo, CHAM_desc_t *A, CHAM_desc_t *B, CHAM_desc_t *X,
         const double cte = anrm * eps * std::sqrt((double)N);
         if (adaptive) tile_precision_map(Aw, NT, ldt, tss, dmap, s);
 
-        k::rhs_transpose((double *)MB->d, BT, NT, ldt, MB->wdt, MB->nt, 1, s);
+        k::rhs_transpose((double *)MB->d, BT, NT, ldt, MB->ldt, MB->wdt, MB->nt, 1, s);
         CHX_HIP(hipMemcpyAsync(XT, BT, vb * sizeof(double), hipMemcpyDeviceToDevice, s));
         PotrfPlan p;
         p.A = Aw;
@@ -315,7 +316,7 @@ int mixed_posv(cham_uplo_t uplo, CHAM_desc_t *A, CHAM_desc_t *B, CHAM_desc_t *X,
             st->pending_info = true;
             if (sequence_wait_internal(seq) != CHAMELEON_SUCCESS) converged = false;
             if (converged) {
-                k::rhs_transpose((double *)MX->d, XT, NT, ldt, MX->wdt, MX->nt, 0, s);
+                k::rhs_transpose((double *)MX->d, XT, NT, ldt, MX->ldt, MX->wdt, MX->nt, 0, s);
                 CHX_HIP(hipStreamSynchronize(s));
             } else {
                 it_count = -(ITERMAX + 1);

@@ -130,7 +130,7 @@ extern "C" int CHAMAMD_dpotrs_Tile_Async_NoAlloc(cham_uplo_t uplo, CHAM_desc_t *
         error(fn, "A's device copy holds its lower tiles only (an Upper solve would need an upload)");
         return request_fail(sequence, request, CHAMELEON_ERR_ILLEGAL_VALUE);
     }
-    if (MA->ldt % 64 != 0 || MB->ldt != MA->ldt) {
+    if (MA->ldt16 % 64 != 0 || MB->ldt16 != MA->ldt16) {
         error(fn, "the padded tile size must be a multiple of 64");
         return request_fail(sequence, request, CHAMELEON_ERR_ILLEGAL_VALUE);
     }
@@ -201,11 +201,11 @@ extern "C" int CHAMAMD_dpotrs_Tile_Async_NoAlloc(cham_uplo_t uplo, CHAM_desc_t *
         k::dinv128(Ad, dinv, (long long)dper, 64LL * 64, 64, NT, ldt, d128, s);
     else
         k::strip_products(Ad, dinv, (long long)dper, 64LL * 64, 64, NT, ldt, ef, eb, s);
-    k::rhs_transpose((double *)MB->d, BT, NT, ldt, MB->wdt, MB->nt, 1, s);
+    k::rhs_transpose((double *)MB->d, BT, NT, ldt, MB->ldt, MB->wdt, MB->nt, 1, s);
     for (int dir = 0; dir < 2; ++dir)
         k::solve_strips(Ad, dinv, (long long)dper, 64LL * 64, 64, BT, NT, ldt, nrp, dir, flags, epoch + dir * chunks,
                         ticket, st->d_info, s, 0, d128, B->n, dir ? eb : ef);
-    k::rhs_transpose((double *)MB->d, BT, NT, ldt, MB->wdt, MB->nt, 0, s);
+    k::rhs_transpose((double *)MB->d, BT, NT, ldt, MB->ldt, MB->wdt, MB->nt, 0, s);
     st->pending_info = true;
     mirror_mark_written(B);
     B->sync = 1;

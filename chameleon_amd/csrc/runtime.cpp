@@ -168,9 +168,35 @@ static void mirror_alloc(CHAM_desc_t *A, Mirror *M)
     if (M->ldt == 0) M->ldt = 16;
     if (M->wdt == 0) M->wdt = 16;
     M->eltsize = (int)CHAMELEON_Element_Size(A->dtyp);
-    M->tile_elems = (size_t)M->ldt * M->wdt;
-    M->bytes = M->tile_elems * M->mt * M->nt * M->eltsize;
-    if (M->bytes == 0) M->bytes = 256;
+    M->ldt16 = M->ldt;
+    auto size = [&](int ldt, int wdt) {
+        M->ldt = ldt;
+        M->wdt = wdt;
+        M->tile_elems = (size_t)ldt * wdt;
+        M->bytes = M->tile_elems * M->mt * M->nt * M->eltsize;
+        if (M->bytes == 0) M->bytes = 256;
+    };
+    size(M->ldt, M->wdt);
+    /* The fused panel, the strip solves and the 64-column updates want tiles
+     * of whole 64x64 blocks; other tiles take one workgroup per diagonal tile,
+     * one wavefront per 16 rows below it and cooperative solves, whose latency
+     * costs more than the added padding at every tile size: resident dposv, 16
+     * against 64, N = 96 in one tile 487 against 211 us, N = 611 nb = 40 4310
+     * and 751, N = 1000 nb = 80 3862 and 1169, nb = 100 3309 and 925, N = 2000
+     * nb = 17 29.7 and 7.6 ms, N = 4000 nb = 200 9.5 and 3.3 ms.  Matrices
+     * whose mirror would pass 16 GiB keep the small padding (16-column tiles
+     * grow 16 times), and so does one that finds no memory for the large. */
+    if (A->mb == A->nb && A->m == A->n && A->dtyp == ChamRealDouble && M->ldt % 64 != 0) {
+        const int t16 = M->ldt, t64 = (M->ldt + 63) & ~63;
+        size(t64, t64);
+        if (M->bytes <= (size_t)16 << 30 && hipMalloc(&M->d, M->bytes) == hipSuccess) {
+            M->state = MIRROR_NONE;
+            return;
+        }
+        (void)hipGetLastError();
+        M->d = nullptr;
+        size(t16, t16);
+    }
     CHX_HIP(hipMalloc(&M->d, M->bytes));
     M->state = MIRROR_NONE;
 }
