@@ -63,34 +63,42 @@ __device__ __forceinline__ void lstore_slice(double *lds, const v2d (&r)[L], int
  * of pzpotrf.c:112-117, the off-diagonal pairs are its GEMMs
  * (pzpotrf.c:123-129), all in one launch.
  *
- * Block tile BM x BN, K staged through LDS in BK-deep slices with the next
- * slice prefetched into registers while the current one is multiplied.
- * Each wavefront owns a WM x WN sub-tile of (WM/16)x(WN/16) MFMA blocks;
- * its operand fragments are read from LDS one 4-deep step ahead of the
- * MFMAs that use them (two register sets), and the first step of the next
- * slice right after the slice barrier, so LDS latency stays off the MFMA
- * pipe.  Operands are swapped (D = B A^T) so each lane's results are
+ * Block tile BM x BN, K staged through LDS in BK-deep slices with the next PF
+ * slices prefetched into registers while one is multiplied.  Each wavefront
+ * owns a WM x WN sub-tile of (WM/16)x(WN/16) MFMA blocks; its operand
+ * fragments are read from LDS one set (GQ 4-deep steps) ahead of the MFMAs
+ * that use them, and the first set of the next slice right after the slice
+ * barrier.  Operands are swapped (D = B A^T) so each lane's results are
  * consecutive rows of one column: stores of 16 lanes form one 128-byte
- * segment.                                                                */
-template <int BM, int BN, int WM, int WN>
+ * segment.
+ *
+ * The matrix cores bound it.  One wavefront on a SIMD issues an FP64 MFMA
+ * every 64 clocks with one LDS read after each product, every 76 with the
+ * reads before them and 83 after: the order is asked for where few
+ * wavefronts share a SIMD (PF > 1).  The 128 x 128 blocks run four wavefronts
+ * on a SIMD, which cover each other, and have no registers for two slices
+ * (measured 5 % slower with them).  The order of the sum over k is the same
+ * for all block sizes, and so are the results.                            */
+template <int BM, int BN, int WM, int WN, int BK, int PF>
 __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64, 2) void trailing_update_kernel(
     double *A, int lmt, int ldt, int k, int kp, int n0, int NT, int ncol, int total_blocks, const int *info,
     const unsigned char *pmap, int atomic_c)
 {
     constexpr int NW = (BM / WM) * (BN / WN);
     constexpr int NTH = NW * 64;
-    constexpr int BK = 16;
     constexpr int FM = WM / 16, FN = WN / 16;
     constexpr int LA = (BK * BM) / (2 * NTH);   /* v2d loads per thread for A */
     constexpr int LB = (BK * BN) / (2 * NTH);
     constexpr int KS = BK / 4;
     static_assert(LA >= 1 && LB >= 1, "tile too small for the thread count");
+    static_assert(PF == 1 || PF % 2 == 0, "the unrolled loop keeps the LDS stage static");
     /* two LDS stages: stage s+1 is stored while stage s is multiplied,
      * one barrier per K slice */
     __shared__ double As[2][BK * BM];
     __shared__ double Bs[2][BK * BN];
 
-    if (*info != 0) return;
+    const int bad = *info;
+    if (PF == 1 && bad != 0) return;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int bid = xcd_remap(blockIdx.x, total_blocks);
     const int tbm = ldt / BM, tbn = ldt / BN;
@@ -135,52 +143,98 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64, 2) void trailing_update
 #pragma unroll
         for (int fn = 0; fn < FN; ++fn) acc[fm][fn] = zero4d();
 
-    v2d ra[LA], rb[LB];
-    /* kp panels (tile columns k .. k+kp-1) of ldt / BK slices each */
+    v2d ra[PF][LA], rb[PF][LB];
+    /* kp panels (1 or 2, tile columns k ..) of ldt / BK slices each */
     const int SK = ldt / BK, S = kp * SK;
     const size_t pstride = (size_t)lmt * ts;
-    auto gload = [&](int st) {
-        const int pi = st / SK, kb = (st - pi * SK) * BK;
-        gload_slice<BM, LA, NTH>(ra, Am + pi * pstride, kb, ldt, tid);
-        gload_slice<BN, LB, NTH>(rb, An + pi * pstride, kb, ldt, tid);
+    auto gload = [&](int st, v2d (&xa)[LA], v2d (&xb)[LB]) {
+        const int pi = st >= SK, kb = (st - (pi ? SK : 0)) * BK;
+        gload_slice<BM, LA, NTH>(xa, Am + pi * pstride, kb, ldt, tid);
+        gload_slice<BN, LB, NTH>(xb, An + pi * pstride, kb, ldt, tid);
     };
-    /* operand fragments of one 4-deep step, two sets */
-    double fa[2][FM], fb[2][FN];
-    auto fload = [&](int buf, int kk, int set) {
+    auto lstore = [&](int buf, const v2d (&xa)[LA], const v2d (&xb)[LB]) {
+        lstore_slice<BM, LA, NTH>(As[buf], xa, tid);
+        lstore_slice<BN, LB, NTH>(Bs[buf], xb, tid);
+    };
+    /* operand fragments of GQ 4-deep steps, two sets */
+    constexpr int GQ = (PF > 1 && FM * FN < 4) ? 4 / (FM * FN) : 1, NG = KS / GQ;
+    static_assert(KS % GQ == 0 && NG % 2 == 0, "fragment sets alternate within a slice");
+    double fa[2][GQ][FM], fb[2][GQ][FN];
+    auto fload = [&](int buf, int g, int set) {
         const double *as = As[buf], *bs = Bs[buf];
 #pragma unroll
-        for (int fm = 0; fm < FM; ++fm) fa[set][fm] = as[(kk + (lane >> 4)) * BM + wm + fm * 16 + (lane & 15)];
+        for (int q = 0; q < GQ; ++q) {
+            const int kr = 4 * (g * GQ + q) + (lane >> 4);
 #pragma unroll
-        for (int fn = 0; fn < FN; ++fn) fb[set][fn] = bs[(kk + (lane >> 4)) * BN + wn + fn * 16 + (lane & 15)];
-    };
-    gload(0);
-    lstore_slice<BM, LA, NTH>(As[0], ra, tid);
-    lstore_slice<BN, LB, NTH>(Bs[0], rb, tid);
-    if (S > 1) gload(1);
-    __syncthreads();
-    fload(0, 0, 0);
-    for (int st = 0; st < S; ++st) {
-        const int cur = st & 1;
-        if (st + 1 < S) {
-            lstore_slice<BM, LA, NTH>(As[cur ^ 1], ra, tid);
-            lstore_slice<BN, LB, NTH>(Bs[cur ^ 1], rb, tid);
-            if (st + 2 < S) gload(st + 2);
+            for (int fm = 0; fm < FM; ++fm) fa[set][q][fm] = as[kr * BM + wm + fm * 16 + (lane & 15)];
+#pragma unroll
+            for (int fn = 0; fn < FN; ++fn) fb[set][q][fn] = bs[kr * BN + wn + fn * 16 + (lane & 15)];
         }
+    };
+    auto multiply = [&](int cur, bool more) {
 #pragma unroll
-        for (int q = 0; q < KS; ++q) {
-            const int set = q & 1;
-            if (q + 1 < KS) {
-                fload(cur, 4 * (q + 1), set ^ 1);
+        for (int g = 0; g < NG; ++g) {
+            const int set = g & 1;
+            if (g + 1 < NG) {
+                fload(cur, g + 1, set ^ 1);
             } else {
                 /* slice st+1 is in LDS and every wave is done reading
                  * slice st (its buffer is refilled next iteration) */
                 __syncthreads();
-                if (st + 1 < S) fload(cur ^ 1, 0, set ^ 1);
+                if (more) fload(cur ^ 1, 0, set ^ 1);
             }
 #pragma unroll
-            for (int fm = 0; fm < FM; ++fm)
+            for (int q = 0; q < GQ; ++q)
 #pragma unroll
-                for (int fn = 0; fn < FN; ++fn) acc[fm][fn] = mfma_f64(fb[set][fn], fa[set][fm], acc[fm][fn]);
+                for (int fm = 0; fm < FM; ++fm)
+#pragma unroll
+                    for (int fn = 0; fn < FN; ++fn)
+                        acc[fm][fn] = mfma_f64(fb[set][q][fn], fa[set][q][fm], acc[fm][fn]);
+            if constexpr (PF > 1) {
+#pragma unroll
+                for (int i = 0; i < GQ * FM * FN; ++i) {
+                    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);   /* one product, */
+                    __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);   /* one LDS read */
+                }
+            }
+        }
+    };
+    if constexpr (PF == 1) {
+        gload(0, ra[0], rb[0]);
+        lstore(0, ra[0], rb[0]);
+        if (S > 1) gload(1, ra[0], rb[0]);
+        __syncthreads();
+        fload(0, 0, 0);
+        for (int st = 0; st < S; ++st) {
+            const int cur = st & 1;
+            if (st + 1 < S) {
+                lstore(cur ^ 1, ra[0], rb[0]);
+                if (st + 2 < S) gload(st + 2, ra[0], rb[0]);
+            }
+            multiply(cur, st + 1 < S);
+        }
+    } else {
+        /* PF slices in flight: set st % PF holds slice st + 1.  Loads past the
+         * end repeat the last slice instead of being skipped, so that no wait
+         * for older loads follows a branch. */
+        {
+            v2d xa[LA], xb[LB];
+            gload(0, xa, xb);
+#pragma unroll
+            for (int j = 0; j < PF; ++j) gload(j + 1 < S ? j + 1 : S - 1, ra[j], rb[j]);
+            if (bad != 0) return;
+            lstore(0, xa, xb);
+        }
+        __syncthreads();
+        fload(0, 0, 0);
+        for (int st = 0; st < S; st += PF) {
+#pragma unroll
+            for (int j = 0; j < PF; ++j) {
+                if (st + j >= S) break;
+                lstore((j & 1) ^ 1, ra[j], rb[j]);
+                gload(st + j + 1 + PF < S ? st + j + 1 + PF : S - 1, ra[j], rb[j]);
+                multiply(j & 1, true);
+            }
         }
     }
 #pragma unroll
@@ -195,7 +249,7 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64, 2) void trailing_update
             }
 }
 
-template <int BM, int BN, int WM, int WN>
+template <int BM, int BN, int WM, int WN, int BK, int PF>
 static void launch_update(double *A, int lmt, int ldt, int k, int kp, int n0, int NT, int ncol, int npairs,
                           const int *info, hipStream_t s, const unsigned char *pmap)
 {
@@ -203,7 +257,7 @@ static void launch_update(double *A, int lmt, int ldt, int k, int kp, int n0, in
     const long long total = (long long)npairs * bpt;
     if (total <= 0) return;
     constexpr int NTH = (BM / WM) * (BN / WN) * 64;
-    hipLaunchKernelGGL((trailing_update_kernel<BM, BN, WM, WN>), dim3((unsigned)total), dim3(NTH), 0, s, A, lmt,
+    hipLaunchKernelGGL((trailing_update_kernel<BM, BN, WM, WN, BK, PF>), dim3((unsigned)total), dim3(NTH), 0, s, A, lmt,
                        ldt, k, kp, n0, NT, ncol, (int)total, info, pmap, atomic_tile_updates());
 }
 
@@ -235,29 +289,35 @@ void trailing_update(double *A, int lmt, int ldt, int k, int n0, int n1, int NT,
     if (n0 >= NT || n1 <= n0) return;
     int ncol = 0;
     const int npairs = update_pairs(n0, n1, NT, &ncol);
-    /* A column launch too small to give every compute unit two 128 x 128
-     * blocks is latency-bound (each block walks the whole K alone): it
-     * takes 64 x 64 blocks, four times as many with a quarter of the work
-     * each (the same k order per element, so the same sums). */
     static const int ncu = [] {
         int dev = 0, n = 0;
         CHX_HIP(hipGetDevice(&dev));
         CHX_HIP(hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev));
         return n;
     }();
-    static const bool use_small = [] {
-        const char *e = getenv("CHAMAMD_SMALL_COLS");
-        return !(e && atoi(e) == 0);
-    }();
-    const bool small_cols = use_small && ncol > 0 && (long long)npairs * (ldt / 128) * (ldt / 128) < 2LL * ncu;
-    if (ldt % 128 == 0 && !small_cols)
-        launch_update<128, 128, 32, 64>(A, lmt, ldt, k, kp, n0, NT, ncol, npairs, info, s, pmap);
-    else if (ldt % 64 == 0)
-        launch_update<64, 64, 32, 32>(A, lmt, ldt, k, kp, n0, NT, ncol, npairs, info, s, pmap);
+    /* By the launch's work in 64 x 64 blocks: small launches take small
+     * blocks, which spread over the compute units and end together, large ones
+     * large blocks, which read less.  Whole triangles of S tile columns on 256
+     * compute units, times in us with 32 / 64 / 128 blocks:
+     *   ldt 256, K 512:  S 8   (576 blocks)   46 /  55 /  80
+     *                    S 14  (1680)        128 / 121 / 143
+     *                    S 24  (4800)        368 / 313 / 370
+     *                    S 50  (20400)      1639 / 1337 / 1336
+     *   ldt 512, K 1024: S 8   (2304)        332 / 293 / 394
+     *                    S 18  (10944)      1659 / 1378 / 1418
+     *                    S 32  (33792)      5314 / 4343 / 4200
+     * and one tile column, ldt 320, K 320: 250 blocks 15 / 21 (the 64 x 64
+     * blocks as they were before took 22), 50 blocks 7 / 16 (18); ldt 320, S 10,
+     * K 640 (1375 blocks) 119 / 128 (133). */
+    const long long b64 = ((long long)npairs * ldt / 64) * ldt / 64;
+    if (ldt % 128 == 0 && b64 >= 80LL * ncu)
+        launch_update<128, 128, 32, 64, 16, 1>(A, lmt, ldt, k, kp, n0, NT, ncol, npairs, info, s, pmap);
+    else if (ldt % 64 == 0 && b64 >= 6LL * ncu)
+        launch_update<64, 64, 32, 32, 16, 2>(A, lmt, ldt, k, kp, n0, NT, ncol, npairs, info, s, pmap);
     else if (ldt % 32 == 0)
-        launch_update<32, 32, 16, 16>(A, lmt, ldt, k, kp, n0, NT, ncol, npairs, info, s, pmap);
+        launch_update<32, 32, 16, 16, 32, 2>(A, lmt, ldt, k, kp, n0, NT, ncol, npairs, info, s, pmap);
     else
-        launch_update<16, 16, 16, 16>(A, lmt, ldt, k, kp, n0, NT, ncol, npairs, info, s, pmap);
+        launch_update<16, 16, 16, 16, 16, 1>(A, lmt, ldt, k, kp, n0, NT, ncol, npairs, info, s, pmap);
 }
 
 /* ================================================================== */
