@@ -118,8 +118,8 @@ void run_gen(double *base, std::vector<BatchGenSys> &sys, int sym, hipStream_t s
 {
     std::vector<long long> unit0(sys.size() + 1, 0);
     for (size_t i = 0; i < sys.size(); ++i) {
-        const long long runs = (sys[i].rows + 31) / 32;
-        unit0[i + 1] = unit0[i] + runs * sys[i].cols;
+        const long long runs = (sys[i].cols + BATCH_GEN_RUN - 1) / BATCH_GEN_RUN;
+        unit0[i + 1] = unit0[i] + runs * sys[i].rows;
     }
     BatchGenSys *d_sys = upload(sys);
     long long *d_u = upload(unit0);

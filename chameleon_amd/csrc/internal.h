@@ -272,6 +272,8 @@ SolvePlan solve_plan(double *A, int NT, int ldt, int nrp, int *d_info, int ncols
 void solve_bt(const SolvePlan &p, double *A, int NT, int ldt, double *BT, int nrp, int *d_info);
 
 /* one system of a batched generation (kernels/batch.hip) */
+/* columns that one thread of batch_gen fills: a system takes rows * ceil(cols / BATCH_GEN_RUN) units */
+#define BATCH_GEN_RUN 32
 struct BatchGenSys {
     long long off;                 /* first element of the system                    */
     long long base;                /* origin of the element rule                     */

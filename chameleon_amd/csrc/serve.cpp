@@ -347,7 +347,7 @@ void launch_small_factor(Server *s, Slot &sl, Job *job)
     }
     std::vector<long long> unit0(gen.size() + 1, 0);
     for (size_t i = 0; i < gen.size(); ++i)
-        unit0[i + 1] = unit0[i] + (long long)((gen[i].rows + 31) / 32) * gen[i].cols;
+        unit0[i + 1] = unit0[i] + (long long)((gen[i].cols + BATCH_GEN_RUN - 1) / BATCH_GEN_RUN) * gen[i].rows;
     /* staging: [descriptors ... info] uploaded as one block, then each host
      * matrix packed with identity padding */
     Layout d;
