@@ -7,10 +7,9 @@
  *
  * Both work on 64-column blocks.  POTRF factors a 64-column block of the
  * diagonal tile with a 16-column inner loop (16 x 16 blocks factored in
- * registers by one wavefront), then builds the explicit inverse of the
- * 64 x 64 diagonal block from the 16 x 16 inverses; TRSM then needs one
- * 64-column MFMA product per block instead of a 16-column substitution
- * chain.  The inverses are stored as 64 x 64 column-major blocks, ldt/64
+ * registers by one wavefront) and keeps the inverses of the 16 x 16 blocks,
+ * with which the rows below are solved by MFMA products; the explicit inverse
+ * of the 64 x 64 block goes to the triangular solves.  The inverses are stored as 64 x 64 column-major blocks, ldt/64
  * (rounded up) per diagonal tile.
  */
 #include "../internal.h"
@@ -89,33 +88,6 @@ __device__ __forceinline__ double rsqrt_f64(double d)
     return r;
 }
 
-/* Cholesky of a 16 x 16 block by one wavefront: lane i (of each 16-lane
- * group; the four groups compute the same thing) holds row i in a[];
- * pivots and column entries are read from lanes 0-15 with readlane (a
- * scalar broadcast, no LDS round trip).  On return a[] holds row i of L
- * and rd = 1 / L(i,i).  `fail` is the 1-based index of the first
- * non-positive pivot (uniform), 0 if none. */
-__device__ __forceinline__ void block16_potrf(double (&a)[16], int lane, int &fail, double &rd)
-{
-    const int i = lane & 15;
-    fail = 0;
-    rd = 0.0;
-#pragma unroll
-    for (int j = 0; j < 16; ++j) {
-        const double d = readlane_f64(a[j], j);
-        if (fail == 0 && !(d > 0.0)) fail = j + 1;
-        const double r = rsqrt_f64(d);
-        const double lij = a[j] * r;                      /* l_ij for i > j, sqrt(d) for i == j */
-        if (i == j) rd = r;
-        if (i >= j) a[j] = lij;
-#pragma unroll
-        for (int k = j + 1; k < 16; ++k) {
-            const double lkj = readlane_f64(lij, k);
-            if (i > j && k <= i) a[k] -= lij * lkj;
-        }
-    }
-}
-
 /* Column (lane % 16) of the inverse of the lower triangular 16 x 16 block
  * L(r,p) = Ls[r * lds + p], by forward substitution, with the reciprocal
  * diagonal rdiag[r] = 1 / L(r,r). */
@@ -166,430 +138,6 @@ __device__ void assemble_inverse(const double (*Ld)[OBP], const double (*Lb)[16]
         }
         __syncthreads();
     }
-}
-
-/* ================================================================== */
-/* POTRF of one matrix held in HBM per job, one workgroup of 8 wavefronts
- * per job: the diagonal tile of the tiled factorisation (one job), or
- * every system of a batch (jobs taken from a queue).
- * For each 64-column block C (left-looking):
- *   (a) rows [C, np) of the block -= T[., 0:C] T[C:C+64, 0:C]^T   (MFMA)
- *   (b) factor the 64 x 64 diagonal block in LDS by 16-column steps
- *   (c) build its inverse, store it in dinv
- *   (d) rows below: X = P Linv^T                                  (MFMA)
- * The strictly upper triangle of the matrix is never written.  A failed
- * job reports the 1-based column of its first non-positive pivot, only
- * for pivots inside its valid part (nvalid columns).                    */
-
-struct PotrfJobs {
-    double *A;               /* job j: matrix at A + off[j] (off null: A)               */
-    const long long *off;
-    const int *np;           /* order (multiple of 16); null: np0                        */
-    const int *ld;           /* leading dimension; null: ld0, or np when ld0 = 0         */
-    const int *nvalid;       /* valid columns; null: nvalid0                             */
-    double *dinv;            /* 64 x 64 inverses: job j at dinv + doff[j] (null: dinv)   */
-    const long long *doff;
-    int np0, ld0, nvalid0;
-    int count;               /* number of jobs                                           */
-    int *queue;              /* job counter (batches); null: job = blockIdx.x            */
-    int *info;               /* single job: *info = iinfo + column on failure;
-                              * batches: info[j] = column or 0                           */
-    int iinfo, batch;
-};
-
-/* Phase (a) of potrf_jobs_kernel (below) for a full 64-column block C: the
- * same products in the same order as its general loop, without the
- * run-time tests of that loop (block width, last slice, rows past the
- * matrix) around the slice loads; the last slice is peeled off.  A wave
- * whose rows lie past the matrix reads row li instead and discards it. */
-template <int POTRF_WAVES, bool LP>
-__device__ __forceinline__ void potrf_update_full(double *T, int ldt, int C, int r0, bool active,
-                                                  double (*Ys)[16 * OB], int tid, int li, int lk)
-{
-    constexpr int POTRF_THREADS = POTRF_WAVES * 64, YH = 512 / POTRF_THREADS, YS = POTRF_THREADS / 32;
-    v4d acc[4] = {zero4d(), zero4d(), zero4d(), zero4d()};
-    v4f accf[4] = {zero4f(), zero4f(), zero4f(), zero4f()};
-    const double *px = T + (active ? r0 + li : li) + (size_t)lk * ldt;
-    const int yq = tid >> 5, yr = (tid & 31) * 2;
-    const double *py = T + (C + yr) + (size_t)yq * ldt;
-    auto products = [&](int cur, const double (&x)[4]) {
-        if (!active) return;
-#pragma unroll
-        for (int q = 0; q < 4; ++q)
-#pragma unroll
-            for (int f = 0; f < 4; ++f) {
-                if constexpr (LP)
-                    accf[f] = mfma_f32((float)Ys[cur][(4 * q + lk) * OB + 16 * f + li], (float)x[q], accf[f]);
-                else
-                    acc[f] = mfma_f64(Ys[cur][(4 * q + lk) * OB + 16 * f + li], x[q], acc[f]);
-            }
-    };
-    v2d yreg[YH];
-    double x[4];
-#pragma unroll
-    for (int h = 0; h < YH; ++h) yreg[h] = *reinterpret_cast<const v2d *>(py + (size_t)(h * YS) * ldt);
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-        const double v = px[(size_t)(4 * q) * ldt];
-        x[q] = active ? v : 0.0;
-    }
-#pragma unroll
-    for (int h = 0; h < YH; ++h) *reinterpret_cast<v2d *>(&Ys[0][(yq + h * YS) * OB + yr]) = yreg[h];
-    __syncthreads();
-    int p = 0;
-    for (; p + 16 < C; p += 16) {
-        const int cur = (p >> 4) & 1;
-        double xn[4];
-#pragma unroll
-        for (int h = 0; h < YH; ++h)
-            yreg[h] = *reinterpret_cast<const v2d *>(py + (size_t)(p + 16 + h * YS) * ldt);
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            const double v = px[(size_t)(p + 16 + 4 * q) * ldt];
-            xn[q] = active ? v : 0.0;
-        }
-        products(cur, x);
-#pragma unroll
-        for (int h = 0; h < YH; ++h) *reinterpret_cast<v2d *>(&Ys[cur ^ 1][(yq + h * YS) * OB + yr]) = yreg[h];
-#pragma unroll
-        for (int q = 0; q < 4; ++q) x[q] = xn[q];
-        __syncthreads();
-    }
-    products((p >> 4) & 1, x);
-    __syncthreads();
-    if (active) {
-        /* the 16 old values first, all in flight (a load-subtract-store per
-         * element waited for each load in turn); the block lies inside the
-         * matrix, so the upper-triangle ones are read and left as they are */
-        double old[4][4];
-#pragma unroll
-        for (int f = 0; f < 4; ++f)
-#pragma unroll
-            for (int s = 0; s < 4; ++s) {
-                const int c = C + 16 * f + (LP ? 4 * lk + s : lk + 4 * s);
-                old[f][s] = T[(r0 + li) + (size_t)c * ldt];
-            }
-#pragma unroll
-        for (int f = 0; f < 4; ++f)
-#pragma unroll
-            for (int s = 0; s < 4; ++s) {
-                const int r = r0 + li;
-                const int c = C + 16 * f + (LP ? 4 * lk + s : lk + 4 * s);
-                if (r >= c) T[r + (size_t)c * ldt] = old[f][s] - (LP ? (double)accf[f][s] : acc[f][s]);
-            }
-    }
-}
-
-template <int POTRF_WAVES, bool LP = false>
-__global__ __launch_bounds__(POTRF_WAVES * 64, 8 / POTRF_WAVES) void potrf_jobs_kernel(PotrfJobs J)
-{
-    constexpr int POTRF_THREADS = POTRF_WAVES * 64;
-    constexpr int YH = 512 / POTRF_THREADS;     /* Y-slice columns staged per thread */
-    __shared__ double Ld[OB][OBP];
-    /* Lv (the 64 x 64 inverse, phases (c)-(d)) and Ys (the staged Y slices
-     * of phase (a), 2 x 64 rows x 16 k) are never live at the same time */
-    __shared__ double LvYs[OB * OBP];
-    __shared__ double Lb[4][16][17];
-    __shared__ double Rd[16];
-    __shared__ int s_fail, s_job;
-    double (*Lv)[OBP] = reinterpret_cast<double (*)[OBP]>(LvYs);
-    double (*Ys)[16 * OB] = reinterpret_cast<double (*)[16 * OB]>(LvYs);
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int li = lane & 15, lk = lane >> 4;
-    if (!J.batch && *J.info != 0) return;
-    /* the single-job form is on the critical path of the factorisation:
-     * its waves win issue arbitration against co-resident update waves */
-    __builtin_amdgcn_s_setprio(2);
-  for (int pass = 0;; ++pass) {
-    if (tid == 0) s_job = J.queue ? atomicAdd(J.queue, 1) : (pass == 0 ? (int)blockIdx.x : J.count);
-    __syncthreads();
-    const int job = s_job;
-    if (job >= J.count) break;
-    double *T = J.A + (J.off ? J.off[job] : 0);
-    double *dinv = J.dinv + (J.doff ? J.doff[job] : 0);
-    const int np = J.np ? J.np[job] : J.np0;
-    const int ldt = J.ld ? J.ld[job] : (J.ld0 ? J.ld0 : np);
-    const int nvalid = J.nvalid ? J.nvalid[job] : J.nvalid0;
-    if (tid == 0) s_fail = 0;
-    __syncthreads();
-
-    for (int C = 0; C < np; C += OB) {
-        const int W = min(OB, np - C), nfb = W >> 4;
-        /* (a) rows [C, np) x cols [C, C+W) -= T[., 0:C] T[C:C+W, 0:C]^T.
-         * The 16-deep slices of the W shared rows (Y) are staged in LDS,
-         * double-buffered, so one CU's L2 bandwidth carries each slice
-         * once; every wavefront streams its own 16 rows (X). */
-        if (C > 0) {
-            const int nrb = (np - C) >> 4;
-            for (int rb0 = 0; rb0 < nrb; rb0 += POTRF_WAVES) {
-                const int rb = rb0 + wave;
-                const bool active = rb < nrb;
-                const int r0 = C + rb * 16;
-                if (W == OB) {
-                    potrf_update_full<POTRF_WAVES, LP>(T, ldt, C, r0, active, Ys, tid, li, lk);
-                    continue;
-                }
-                v4d acc[4] = {zero4d(), zero4d(), zero4d(), zero4d()};
-                /* LP: the same products with FP32 operands and accumulation
-                 * (v_mfma_f32_16x16x4_f32, result slot s at column 4 lk + s) */
-                v4f accf[4] = {zero4f(), zero4f(), zero4f(), zero4f()};
-                const double *px = T + (r0 + li) + (size_t)lk * ldt;
-                /* Y slice element (row r < 64, k q < 16) -> Ys[q * 64 + r];
-                 * thread tid moves rows 2*(tid%32)..+1 of columns
-                 * tid/32 + h * (threads/32), h < YH */
-                const int yq = tid >> 5, yr = (tid & 31) * 2;
-                const bool yv = yr < W;
-                v2d yreg[YH];
-#pragma unroll
-                for (int h = 0; h < YH; ++h) {
-                    yreg[h] = v2d{0.0, 0.0};
-                    if (yv) yreg[h] = *reinterpret_cast<const v2d *>(T + (C + yr) + (size_t)(yq + h * (POTRF_THREADS / 32)) * ldt);
-                }
-                double x[4];
-#pragma unroll
-                for (int q = 0; q < 4; ++q) x[q] = active ? px[(size_t)(4 * q) * ldt] : 0.0;
-#pragma unroll
-                for (int h = 0; h < YH; ++h)
-                    *reinterpret_cast<v2d *>(&Ys[0][(yq + h * (POTRF_THREADS / 32)) * OB + yr]) = yreg[h];
-                __syncthreads();
-                for (int p = 0; p < C; p += 16) {
-                    const int cur = (p >> 4) & 1;
-                    const bool more = p + 16 < C;
-                    double xn[4];
-                    if (more) {
-#pragma unroll
-                        for (int h = 0; h < YH; ++h)
-                            if (yv)
-                                yreg[h] = *reinterpret_cast<const v2d *>(
-                                    T + (C + yr) + (size_t)(p + 16 + yq + h * (POTRF_THREADS / 32)) * ldt);
-#pragma unroll
-                        for (int q = 0; q < 4; ++q) xn[q] = active ? px[(size_t)(p + 16 + 4 * q) * ldt] : 0.0;
-                    }
-                    if (active) {
-#pragma unroll
-                        for (int q = 0; q < 4; ++q)
-#pragma unroll
-                            for (int f = 0; f < 4; ++f)
-                                if (f < nfb) {
-                                    if constexpr (LP)
-                                        accf[f] = mfma_f32((float)Ys[cur][(4 * q + lk) * OB + 16 * f + li], (float)x[q],
-                                                           accf[f]);
-                                    else
-                                        acc[f] = mfma_f64(Ys[cur][(4 * q + lk) * OB + 16 * f + li], x[q], acc[f]);
-                                }
-                    }
-                    if (more) {
-#pragma unroll
-                        for (int h = 0; h < YH; ++h)
-                            *reinterpret_cast<v2d *>(&Ys[cur ^ 1][(yq + h * (POTRF_THREADS / 32)) * OB + yr]) = yreg[h];
-#pragma unroll
-                        for (int q = 0; q < 4; ++q) x[q] = xn[q];
-                    }
-                    __syncthreads();
-                }
-                if (active) {
-                    for (int f = 0; f < nfb; ++f)
-#pragma unroll
-                        for (int s = 0; s < 4; ++s) {
-                            const int r = r0 + li;
-                            const int c = C + 16 * f + (LP ? 4 * lk + s : lk + 4 * s);
-                            if (r >= c) T[r + (size_t)c * ldt] -= LP ? (double)accf[f][s] : acc[f][s];
-                        }
-                }
-            }
-            __syncthreads();
-        }
-        /* (b) diagonal block into LDS (lower part; zeros above) */
-        for (int e = tid; e < OB * OB; e += POTRF_THREADS) {
-            const int r = e % OB, c = e / OB;
-            Ld[r][c] = (r < W && c < W && r >= c) ? T[(C + r) + (size_t)(C + c) * ldt] : 0.0;
-        }
-        __syncthreads();
-        for (int cb = 0; cb < nfb; ++cb) {
-            const int c0 = 16 * cb;
-            /* (b1) columns [c0, c0+16) of rows [c0, W) -= Ld[., 0:c0] Ld[c0.., 0:c0]^T */
-            if (cb > 0) {
-                const int rb = wave;
-                if (rb < nfb - cb) {
-                    const int r0 = c0 + 16 * rb;
-                    v4d acc = zero4d();
-                    for (int p = 0; p < c0; p += 4)
-                        acc = mfma_f64(Ld[c0 + li][p + lk], Ld[r0 + li][p + lk], acc);
-#pragma unroll
-                    for (int s = 0; s < 4; ++s) {
-                        const int c = lk + 4 * s;
-                        if (rb > 0 || li >= c) Ld[r0 + li][c0 + c] -= acc[s];
-                    }
-                }
-                __syncthreads();
-            }
-            /* (b2) factor and invert the 16 x 16 block */
-            if (wave == 0) {
-                double a[16];
-#pragma unroll
-                for (int q = 0; q < 16; ++q) a[q] = (q <= li) ? Ld[c0 + li][c0 + q] : 0.0;
-                int fail;
-                double rd;
-                block16_potrf(a, lane, fail, rd);
-                if (lane < 16) {
-#pragma unroll
-                    for (int q = 0; q < 16; ++q) Ld[c0 + li][c0 + q] = (q <= li) ? a[q] : 0.0;
-                    Rd[li] = rd;
-                }
-                __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
-                __builtin_amdgcn_wave_barrier();
-                __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
-                double col[16];
-                block16_inverse_col(&Ld[c0][c0], OBP, Rd, lane, col);
-                if (lane < 16) {
-#pragma unroll
-                    for (int q = 0; q < 16; ++q) Lb[cb][q][li] = col[q];
-                }
-                if (lane == 0 && fail) s_fail = (C + c0 + fail - 1 < nvalid) ? C + c0 + fail : -1;
-            }
-            __syncthreads();
-            if (s_fail) break;
-            /* (b3) rows [c0+16, W): X = P Lb^T */
-            {
-                const int rb = wave;
-                if (rb < nfb - cb - 1) {
-                    const int r0 = c0 + 16 + 16 * rb;
-                    double pv[4];
-#pragma unroll
-                    for (int kk = 0; kk < 4; ++kk) pv[kk] = Ld[r0 + li][c0 + 4 * kk + lk];
-                    v4d acc = zero4d();
-#pragma unroll
-                    for (int kk = 0; kk < 4; ++kk) acc = mfma_f64(Lb[cb][li][4 * kk + lk], pv[kk], acc);
-#pragma unroll
-                    for (int s = 0; s < 4; ++s) Ld[r0 + li][c0 + lk + 4 * s] = acc[s];
-                }
-            }
-            __syncthreads();
-        }
-        if (s_fail) break;
-        /* (c) inverse of the 64 x 64 diagonal block */
-        assemble_inverse(Ld, Lb, Lv, nfb, wave, lane);
-        /* factor back into the tile, inverse into dinv (column-major 64 x 64) */
-        double *dv = dinv + (size_t)(C / OB) * OB * OB;
-        for (int e = tid; e < OB * OB; e += POTRF_THREADS) {
-            const int r = e % OB, c = e / OB;
-            if (r < W && c < W && r >= c) T[(C + r) + (size_t)(C + c) * ldt] = Ld[r][c];
-            dv[e] = Lv[r][c];
-        }
-        /* (d) rows [C+W, np): X = P Lv^T, D = Lv P^T */
-        {
-            const int nrb = (np - C - W) >> 4;
-            for (int rb = wave; rb < nrb; rb += POTRF_WAVES) {
-                const int r0 = C + W + rb * 16;
-                double pv[16];
-                if (W == OB) {
-                    /* full block: the 16 loads with no run-time test between
-                     * them (in flight together), the same products */
-#pragma unroll
-                    for (int kq = 0; kq < 16; ++kq) pv[kq] = T[(r0 + li) + (size_t)(C + 4 * kq + lk) * ldt];
-                    v4d acc[4] = {zero4d(), zero4d(), zero4d(), zero4d()};
-#pragma unroll
-                    for (int f = 0; f < 4; ++f)
-#pragma unroll
-                        for (int kq = 0; kq < 4 * (f + 1); ++kq)
-                            acc[f] = mfma_f64(Lv[16 * f + li][4 * kq + lk], pv[kq], acc[f]);
-#pragma unroll
-                    for (int f = 0; f < 4; ++f)
-#pragma unroll
-                        for (int s = 0; s < 4; ++s) T[(r0 + li) + (size_t)(C + 16 * f + lk + 4 * s) * ldt] = acc[f][s];
-                    continue;
-                }
-#pragma unroll
-                for (int kq = 0; kq < 16; ++kq)
-                    pv[kq] = (4 * kq < W) ? T[(r0 + li) + (size_t)(C + 4 * kq + lk) * ldt] : 0.0;
-                v4d acc[4] = {zero4d(), zero4d(), zero4d(), zero4d()};
-#pragma unroll
-                for (int f = 0; f < 4; ++f) {
-                    if (f < nfb) {
-#pragma unroll
-                        for (int kq = 0; kq < 16; ++kq)
-                            if (kq < 4 * (f + 1)) acc[f] = mfma_f64(Lv[16 * f + li][4 * kq + lk], pv[kq], acc[f]);
-                    }
-                }
-#pragma unroll
-                for (int f = 0; f < 4; ++f) {
-                    if (f < nfb) {
-#pragma unroll
-                        for (int s = 0; s < 4; ++s) T[(r0 + li) + (size_t)(C + 16 * f + lk + 4 * s) * ldt] = acc[f][s];
-                    }
-                }
-            }
-        }
-        __syncthreads();
-    }
-    if (tid == 0) {
-        if (J.batch) J.info[job] = s_fail > 0 ? s_fail : 0;
-        else if (s_fail > 0) *J.info = J.iinfo + s_fail;
-    }
-    __syncthreads();
-  }
-}
-
-void potrf_diag(double *Akk, int ldt, double *dinv, int iinfo, int nvalid, int *info, int waves, hipStream_t s)
-{
-    PotrfJobs J = {};
-    J.A = Akk; J.dinv = dinv;
-    J.np0 = ldt; J.ld0 = ldt; J.nvalid0 = nvalid;
-    J.count = 1; J.info = info; J.iinfo = iinfo; J.batch = 0;
-    if (waves == 8) hipLaunchKernelGGL(potrf_jobs_kernel<8>, dim3(1), dim3(512), 0, s, J);
-    else hipLaunchKernelGGL(potrf_jobs_kernel<4>, dim3(1), dim3(256), 0, s, J);
-}
-
-/* Batched form: `count` matrices, job j of order np[j] (multiple of 16)
- * at A + off[j] with leading dimension ld[j] (null: np[j]), inverses at
- * dinv + doff[j]; info[j] = first failing column or 0.  `queue` is a
- * zeroed device counter; jobs are taken in index order by `grid`
- * persistent workgroups (grid <= 0: as many as are resident at once; sort
- * the jobs largest first for balance). */
-template <int W, bool LP>
-static int potrf_jobs_resident()
-{
-    static int resident = 0;
-    if (!resident) {
-        int dev = 0, ncu = 0, per = 0;
-        CHX_HIP(hipGetDevice(&dev));
-        CHX_HIP(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev));
-        CHX_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, potrf_jobs_kernel<W, LP>, W * 64, 0));
-        resident = ncu * (per > 0 ? per : 1);
-    }
-    return resident;
-}
-
-template <int W, bool LP>
-static void potrf_jobs_launch(const PotrfJobs &J, int grid, hipStream_t s)
-{
-    if (grid <= 0) grid = potrf_jobs_resident<W, LP>();
-    if (grid > J.count) grid = J.count;
-    hipLaunchKernelGGL((potrf_jobs_kernel<W, LP>), dim3(grid), dim3(W * 64), 0, s, J);
-}
-
-void potrf_jobs(double *A, const long long *off, const int *np, const int *ld, const int *nvalid, double *dinv,
-                const long long *doff, int count, int *queue, int *info, int grid, hipStream_t s, int waves, bool lp)
-{
-    PotrfJobs J = {};
-    J.A = A; J.off = off; J.np = np; J.ld = ld; J.nvalid = nvalid; J.dinv = dinv; J.doff = doff;
-    J.count = count; J.queue = queue; J.info = info; J.batch = 1;
-    if (count <= 0) return;
-    if (waves == 8) {
-        if (lp) potrf_jobs_launch<8, true>(J, grid, s);
-        else potrf_jobs_launch<8, false>(J, grid, s);
-    } else {
-        if (lp) potrf_jobs_launch<4, true>(J, grid, s);
-        else potrf_jobs_launch<4, false>(J, grid, s);
-    }
-}
-
-void potrf_jobs_prepare()
-{
-    (void)potrf_jobs_resident<4, false>();
-    (void)potrf_jobs_resident<8, false>();
-    (void)potrf_jobs_resident<4, true>();
-    (void)potrf_jobs_resident<8, true>();
 }
 
 /* ================================================================== */
@@ -809,6 +357,10 @@ __device__ __forceinline__ double pf_ld(rsrc_t r, int vo, int so)
 {
     return __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(r, vo, so, DEV ? 16 : 0));
 }
+__device__ __forceinline__ v2d pf_ld2(rsrc_t r, int vo, int so)
+{
+    return __builtin_bit_cast(v2d, __builtin_amdgcn_raw_buffer_load_b128(r, vo, so, 0));
+}
 template <bool DEV = false>
 __device__ __forceinline__ void pf_st(double v, rsrc_t r, int vo, int so)
 {
@@ -964,8 +516,12 @@ __device__ __forceinline__ int pf_col16(double (&a)[16], int lane)
 
 /* The 64 x 64 inverse from M, into dinv (column-major, zeros above the
  * diagonal): Z(J, J) = Lb(J), Z(I, J) = -Lb(I) sum_{J<=P<I} L(I, P) Z(P, J);
- * wave J forms block column J in registers.  Xs: 32 KB of LDS. */
-__device__ __forceinline__ void pf_inverse(const double *Ms, double *Xs, double *dinv, int tid, int wave, int lane)
+ * wave J < 4 forms block column J in registers.  Xs: 32 KB of LDS, on return
+ * element (r, c) at (r ^ (c & 15)) + 64 c.  Of dinv, columns and rows from W on
+ * are zero. */
+template <int NT>
+__device__ __forceinline__ void pf_inverse(const double *Ms, double *Xs, double *dinv, int W, int tid, int wave,
+                                           int lane)
 {
     const int li = lane & 15, lk = lane >> 4;
     v4d z[4];
@@ -986,13 +542,15 @@ __device__ __forceinline__ void pf_inverse(const double *Ms, double *Xs, double 
         }
     }
     __syncthreads();
-    /* element (r, c) at r + 64 c, the row XORed with the column's low bits */
+    if (wave < 4) {
 #pragma unroll
-    for (int I = 0; I < 4; ++I)
+        for (int I = 0; I < 4; ++I)
 #pragma unroll
-        for (int s = 0; s < 4; ++s) Xs[((16 * I + lk + 4 * s) ^ li) + 64 * (16 * wave + li)] = z[I][s];
+            for (int s = 0; s < 4; ++s) Xs[((16 * I + lk + 4 * s) ^ li) + 64 * (16 * wave + li)] = z[I][s];
+    }
     __syncthreads();
-    for (int e = tid; e < 4096; e += 256) dinv[e] = Xs[e ^ ((e >> 6) & 15)];
+    for (int e = tid; e < 4096; e += NT)
+        dinv[e] = (W == 64 || max(e >> 6, e & 63) < W) ? Xs[e ^ ((e >> 6) & 15)] : 0.0;
 }
 
 /* M(C) from its scratch into LDS (whole workgroup; barriers by the caller) */
@@ -1236,7 +794,7 @@ __device__ __forceinline__ void panel_chain(const PanelArgs &a, PanelLds &L)
             }
         }
     }
-    pf_inverse(L.B[cur ^ 1], Xs, a.dinv + (size_t)(ND - 1) * 4096, tid, wave, lane);
+    pf_inverse<256>(L.B[cur ^ 1], Xs, a.dinv + (size_t)(ND - 1) * 4096, 64, tid, wave, lane);
 }
 
 /* Block (r, C) of the diagonal tile below its diagonal blocks; for C = r-1 it
@@ -1284,7 +842,7 @@ __device__ __forceinline__ void panel_block(const PanelArgs &a, PanelLds &L, int
     pf_load_m(a.W + (size_t)C * PF_W, L.B[0], tid);
     __syncthreads();
     if (is_r) {
-        pf_inverse(L.B[0], L.Xs, a.dinv + (size_t)C * 4096, tid, wave, lane);
+        pf_inverse<256>(L.B[0], L.Xs, a.dinv + (size_t)C * 4096, 64, tid, wave, lane);
         return;
     }
     pf_subst(L.B[0], lane, y);
@@ -1471,6 +1029,390 @@ void panel_factor(double *T, double *P, long long ts, int S, int ldt, double *di
     a.nw = nu < room ? nu : room;
     const int grid = 1 + a.nw + a.ND * S;
     hipLaunchKernelGGL(panel_factor_kernel, dim3(grid), dim3(256), 0, s, a);
+}
+
+/* ================================================================== */
+/* POTRF of one matrix held in HBM per job, one workgroup of 4 or 8 wavefronts
+ * per job: the diagonal tile of the tiled factorisation (one job), or
+ * every system of a batch (jobs taken from a queue).
+ * For each 64-column block C (left-looking):
+ *   (a) diagonal block -= T[C:C+64, 0:C] T[C:C+64, 0:C]^T, into LDS (MFMA)
+ *   (b) factor the 64 x 64 diagonal block in LDS by 16-column steps, the
+ *       inverses of its 16 x 16 diagonal blocks beside them
+ *   (c) build the 64 x 64 inverse, store it in dinv
+ *   (d) rows below: the products of (a) and X = P L^-T in one pass (MFMA)
+ * The strictly upper triangle of the matrix is never written.  A failed
+ * job reports the 1-based column of its first non-positive pivot, only
+ * for pivots inside its valid part (nvalid columns).
+ *
+ * A large batch is bound by (d): its operands come from beyond the L2 (512
+ * systems are in work at once), so what counts is how far ahead they are asked
+ * for and how often they are read.  A wavefront takes two 16-row blocks against
+ * the same 64 shared rows, keeps four slices of both in flight, and solves its
+ * rows while they are in registers.  With one block, one slice and a pass of
+ * its own for the solves, the 20 000 systems of orders 16 to 1023 took 24.0 ms,
+ * now 16.8; 1024 of order 1024 11.4 and 8.6 ms, 2048 of order 512 4.1 and 2.9.
+ * A small batch is bound by the serial (b), 18 us per block before and 9 now
+ * (the steps of the panel's chain): 4000 of order 64 366 and 191 us, one of
+ * order 256 198 and 124. */
+
+struct PotrfJobs {
+    double *A;               /* job j: matrix at A + off[j] (off null: A)               */
+    const long long *off;
+    const int *np;           /* order (multiple of 16); null: np0                        */
+    const int *ld;           /* leading dimension; null: ld0, or np when ld0 = 0         */
+    const int *nvalid;       /* valid columns; null: nvalid0                             */
+    double *dinv;            /* 64 x 64 inverses: job j at dinv + doff[j] (null: dinv)   */
+    const long long *doff;
+    int np0, ld0, nvalid0;
+    int count;               /* number of jobs                                           */
+    int *queue;              /* job counter (batches); null: job = blockIdx.x            */
+    int *info;               /* single job: *info = iinfo + column on failure;
+                              * batches: info[j] = column or 0                           */
+    int iinfo, batch;
+};
+
+/* Products of the 16-row blocks rb0 + wave + NW u, u < NB, of the nrb from row
+ * C on, and what follows them: DIAG, the diagonal block's (NB = 1, four
+ * wavefronts), goes to Db; rows below are solved with M in Db and stored.  The
+ * 16-deep slices of the 64 shared rows (Y) are staged in LDS, double-buffered;
+ * every wavefront streams its own rows (X; DIAG reads them from Y).  C is a
+ * multiple of 64, so the ring of four slices needs no test; loads past the
+ * last slice repeat it.  A block past the matrix reads rows li instead, and
+ * shared rows past the matrix (last block column) whatever follows in it:
+ * neither is used.  FP32 products leave other columns in a slot than FP64
+ * ones; their shared rows are read in an order (pi) that undoes it. */
+template <int NW, int NB, bool LP, bool DIAG>
+__device__ __forceinline__ void jobs_update(double *T, int ldt, int C, int rb0, int nrb, double *Ys, double *Db,
+                                            int tid)
+{
+    constexpr int NT = NW * 64, YH = 512 / NT;
+    const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), li = lane & 15, lk = lane >> 4;
+    const int pi = LP ? (li >> 2) + 4 * (li & 3) : li;
+    const int S = C >> 4;
+    /* offsets from the first column of a slice, whose address is a scalar */
+    int vx[NB];
+#pragma unroll
+    for (int u = 0; u < NB; ++u) {
+        const int rb = rb0 + wave + NW * u;
+        vx[u] = ((rb < nrb ? C + 16 * rb + li : li) + lk * ldt) * 8;
+    }
+    const int vy = (C + (tid & 31) * 2 + (tid >> 5) * ldt) * 8;
+    double *const ys = Ys + (tid >> 5) * OB + (tid & 31) * 2;
+    v4d acc[NB][4];
+    v4f accf[NB][4];
+#pragma unroll
+    for (int u = 0; u < NB; ++u)
+#pragma unroll
+        for (int f = 0; f < 4; ++f) {
+            acc[u][f] = zero4d();
+            accf[u][f] = zero4f();
+        }
+    v2d y[4][YH];
+    double x[4][NB][4];
+    auto yload = [&](int st, v2d (&r)[YH]) {
+        const rsrc_t b = pf_rsrc(T + (size_t)(16 * min(st, S - 1)) * ldt);
+#pragma unroll
+        for (int h = 0; h < YH; ++h) r[h] = pf_ld2(b, vy, h * (NT / 4) * ldt);
+    };
+    auto ystore = [&](int buf, const v2d (&r)[YH]) {
+#pragma unroll
+        for (int h = 0; h < YH; ++h) *reinterpret_cast<v2d *>(ys + buf * 16 * OB + h * (NT / 32) * OB) = r[h];
+    };
+    auto xload = [&](int st, double (&r)[NB][4]) {
+        const rsrc_t b = pf_rsrc(T + (size_t)(16 * min(st, S - 1)) * ldt);
+#pragma unroll
+        for (int u = 0; u < NB; ++u)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) r[u][q] = pf_ld(b, vx[u], 32 * q * ldt);
+    };
+    auto products = [&](int buf, const double (&r)[NB][4]) {
+        const double *yb = Ys + buf * 16 * OB + lk * OB + pi;
+        const double *xb = Ys + buf * 16 * OB + lk * OB + 16 * (wave & 3) + li;
+        double v[2][4];
+#pragma unroll
+        for (int f = 0; f < 4; ++f) v[0][f] = yb[16 * f];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            if (q < 3) {
+#pragma unroll
+                for (int f = 0; f < 4; ++f) v[(q + 1) & 1][f] = yb[(q + 1) * 4 * OB + 16 * f];
+            }
+#pragma unroll
+            for (int u = 0; u < NB; ++u)
+#pragma unroll
+                for (int f = 0; f < 4; ++f) {
+                    const double x = DIAG ? xb[q * 4 * OB] : r[u][q];
+                    if constexpr (LP) accf[u][f] = mfma_f32((float)v[q & 1][f], (float)x, accf[u][f]);
+                    else acc[u][f] = mfma_f64(v[q & 1][f], x, acc[u][f]);
+                }
+            if constexpr (!LP && !DIAG) {
+                /* one LDS read behind each of the first products */
+                if (q < 3) {
+                    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+                    __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+                    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+                    __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+                    __builtin_amdgcn_sched_group_barrier(0x008, 4 * NB - 2, 0);
+                }
+            }
+        }
+    };
+    if (S > 0) {
+        yload(0, y[0]);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            if (!DIAG) xload(j, x[j]);
+            if (j > 0) yload(j, y[j]);
+        }
+        ystore(0, y[0]);
+        yload(4, y[0]);
+        __syncthreads();
+        for (int st = 0; st < S; st += 4) {
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                ystore((j & 1) ^ 1, y[(j + 1) & 3]);
+                yload(st + j + 5, y[(j + 1) & 3]);
+                products(j & 1, x[j]);
+                if (!DIAG) xload(st + j + 4, x[j]);
+                __syncthreads();
+            }
+        }
+    }
+    /* the old values of all blocks first, all in flight; of the diagonal block
+     * the lower 16 x 16 blocks only */
+    const int vt = (li + lk * ldt) * 8;
+    v4d old[NB][4];
+#pragma unroll
+    for (int u = 0; u < NB; ++u) {
+        const int rb = min(rb0 + wave + NW * u, nrb - 1);
+        const rsrc_t t = pf_rsrc(T + C + 16 * rb + (size_t)C * ldt);
+#pragma unroll
+        for (int f = 0; f < 4; ++f)
+#pragma unroll
+            for (int s = 0; s < 4; ++s) old[u][f][s] = pf_ld(t, vt, (16 * (DIAG ? min(f, rb) : f) + 4 * s) * ldt * 8);
+    }
+#pragma unroll
+    for (int u = 0; u < NB; ++u) {
+        const int rb = rb0 + wave + NW * u;
+        if (rb >= nrb) continue;
+#pragma unroll
+        for (int f = 0; f < 4; ++f)
+#pragma unroll
+            for (int s = 0; s < 4; ++s) old[u][f][s] -= LP ? (double)accf[u][f][s] : acc[u][f][s];
+        if constexpr (DIAG) {
+#pragma unroll
+            for (int f = 0; f < 4; ++f)
+                if (f <= rb) {
+#pragma unroll
+                    for (int s = 0; s < 4; ++s) Db[pf_low(rb, f) + 64 * s + lane] = old[u][f][s];
+                }
+        } else {
+            pf_subst(Db, lane, old[u]);
+            const rsrc_t t = pf_rsrc(T + C + 16 * rb + (size_t)C * ldt);
+#pragma unroll
+            for (int f = 0; f < 4; ++f)
+#pragma unroll
+                for (int s = 0; s < 4; ++s) pf_st(old[u][f][s], t, vt, (16 * f + 4 * s) * ldt * 8);
+        }
+    }
+}
+
+template <int POTRF_WAVES, bool LP = false>
+__global__ __launch_bounds__(POTRF_WAVES * 64, 2) void potrf_jobs_kernel(PotrfJobs J)
+{
+    constexpr int NW = POTRF_WAVES, NT = NW * 64;
+    /* Ys holds the staged shared rows, Xs the 64 x 64 inverse on its way out,
+     * Db the diagonal block's lower 16 x 16 blocks, which turn into L with the
+     * inverses on the diagonal, and Ld the diagonal ones of L */
+    __shared__ double Xs[OB * OB], Ys[2 * 16 * OB], Db[PF_LOW], Ld[4 * PF_BLK];
+    __shared__ int s_fail, s_job;
+    if (!J.batch && *J.info != 0) return;
+    /* the single-job form is on the critical path of the factorisation:
+     * its waves win issue arbitration against co-resident update waves */
+    __builtin_amdgcn_s_setprio(2);
+  for (int pass = 0;; ++pass) {
+    if (threadIdx.x == 0) {
+        s_job = J.queue ? atomicAdd(J.queue, 1) : (pass == 0 ? (int)blockIdx.x : J.count);
+        s_fail = 0;
+    }
+    __syncthreads();
+    const int job = __builtin_amdgcn_readfirstlane(s_job);
+    if (job >= J.count) break;
+    double *T = J.A + (J.off ? J.off[job] : 0);
+    double *dinv = J.dinv + (J.doff ? J.doff[job] : 0);
+    const int np = J.np ? J.np[job] : J.np0;
+    const int ldt = J.ld ? J.ld[job] : (J.ld0 ? J.ld0 : np);
+    const int nvalid = J.nvalid ? J.nvalid[job] : J.nvalid0;
+
+    for (int C = 0; C < np; C += OB) {
+        /* (kept from being taken out of the loop: the addresses formed from it
+         * need more registers than there are) */
+        int tid = threadIdx.x;
+        asm volatile("" : "+v"(tid));
+        const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), li = lane & 15, lk = lane >> 4;
+        const int W = min(OB, np - C), nfb = W >> 4;
+        /* a last block column narrower than 64 goes on as if identity */
+        if (nfb < 4) {
+            for (int e = tid; e < PF_LOW; e += NT) {
+                const int b = e >> 8, i = b < 1 ? 0 : b < 3 ? 1 : b < 6 ? 2 : 3;
+                if (i >= nfb) Db[e] = (b == i * (i + 3) / 2 && (e & 15) == ((e >> 4) & 15)) ? 1.0 : 0.0;
+            }
+        }
+        /* (a) for the diagonal block: of a first one, its values */
+        jobs_update<NW, 1, LP, true>(T, ldt, C, 0, nfb, Ys, Db, tid);
+        __syncthreads();
+        /* (b), as in the panel's chain: wave 0 the columns, the others what
+         * comes after them; wave 3 repeats the first block for its inverse
+         * when the first step has no lane left for the identity */
+#pragma unroll 1
+        for (int cb = 0; cb < nfb; ++cb) {
+            if (wave == 0 || (wave == 3 && cb == 1 && nfb == 4)) {
+                /* row group lk: block (c + lk, c), lk < nr, then identity rows */
+                const int c = wave == 0 ? cb : 0, nr = wave == 0 ? nfb - cb : 1;
+                const bool row = lk < nr;
+                double *const blk = Db + pf_low(row ? c + lk : c, c);
+                double v[16];
+#pragma unroll
+                for (int q = 0; q < 16; ++q) {
+                    const double e = blk[li + 16 * q];
+                    v[q] = row ? e : (q == li ? 1.0 : 0.0);
+                }
+                const int fail = pf_col16(v, lane);
+                if (lk == 0) {
+#pragma unroll
+                    for (int q = 0; q < 16; ++q)
+                        if (nr < 4) Ld[c * PF_BLK + li + 16 * q] = v[q];
+                } else if (row) {
+#pragma unroll
+                    for (int q = 0; q < 16; ++q) blk[li + 16 * q] = v[q];
+                } else if (lk == nr) {
+#pragma unroll
+                    for (int q = 0; q < 16; ++q) blk[pf_inv(q, li)] = q >= li ? v[q] : 0.0;
+                }
+                if (lane == 0 && fail) s_fail = C + 16 * c + fail - 1 < nvalid ? C + 16 * c + fail : -1;
+            } else if (cb > 0 && cb < 3 && wave < 3) {
+                /* what step cb-1 takes off the columns after cb: (2,2), (3,2),
+                 * (3,3), then (3,3) */
+                for (int u = wave - 1; u < (cb == 1 ? 3 : 1); u += 2) {
+                    const int i = u == 0 && cb == 1 ? 2 : 3, j = u == 2 || cb == 2 ? 3 : 2;
+                    v4d x;
+#pragma unroll
+                    for (int s = 0; s < 4; ++s) x[s] = Db[pf_low(i, j) + 64 * s + lane];
+#pragma unroll
+                    for (int s = 0; s < 4; ++s)
+                        x = mfma_f64(-Db[pf_low(j, cb - 1) + 64 * s + lane], Db[pf_low(i, cb - 1) + 64 * s + lane], x);
+#pragma unroll
+                    for (int s = 0; s < 4; ++s) Db[pf_low(i, j) + 64 * s + lane] = x[s];
+                }
+            }
+            __syncthreads();
+            if (s_fail) break;
+            if (cb + 1 < nfb) {
+                /* column cb+1 takes off step cb: block (cb + 1 + wave, cb + 1) */
+                const int i = cb + 1 + wave;
+                if (i < nfb) {
+                    v4d x;
+#pragma unroll
+                    for (int s = 0; s < 4; ++s) x[s] = Db[pf_low(i, cb + 1) + 64 * s + lane];
+#pragma unroll
+                    for (int s = 0; s < 4; ++s)
+                        x = mfma_f64(-Db[pf_low(cb + 1, cb) + 64 * s + lane], Db[pf_low(i, cb) + 64 * s + lane], x);
+#pragma unroll
+                    for (int s = 0; s < 4; ++s) Db[pf_low(i, cb + 1) + 64 * s + lane] = x[s];
+                }
+                __syncthreads();
+            }
+        }
+        if (s_fail) break;
+        /* (c) inverse into dinv (zero past the matrix) and Xs, L into the matrix */
+        pf_inverse<NT>(Db, Xs, dinv + (size_t)(C / OB) * OB * OB, W, tid, wave, lane);
+        if (tid < 256) {
+#pragma unroll
+            for (int b = 0; b < 10; ++b) {
+                const int i = b < 1 ? 0 : b < 3 ? 1 : b < 6 ? 2 : 3, j = b - i * (i + 1) / 2;
+                const double v = i == j ? Ld[j * PF_BLK + tid] : Db[b * PF_BLK + tid];
+                if (i < nfb && (i > j || (tid & 15) >= (tid >> 4)))
+                    T[(C + 16 * i + (tid & 15)) + (size_t)(C + 16 * j + (tid >> 4)) * ldt] = v;
+            }
+        }
+        /* (a) and (d) for the rows below */
+        {
+            const int nrb = (np - C) >> 4;
+            int rb0 = 4;
+            for (; nrb - rb0 > NW; rb0 += 2 * NW) jobs_update<NW, 2, LP, false>(T, ldt, C, rb0, nrb, Ys, Db, tid);
+            if (rb0 < nrb) jobs_update<NW, 1, LP, false>(T, ldt, C, rb0, nrb, Ys, Db, tid);
+        }
+        __syncthreads();
+    }
+    if (threadIdx.x == 0) {
+        if (J.batch) J.info[job] = s_fail > 0 ? s_fail : 0;
+        else if (s_fail > 0) *J.info = J.iinfo + s_fail;
+    }
+    __syncthreads();
+  }
+}
+
+void potrf_diag(double *Akk, int ldt, double *dinv, int iinfo, int nvalid, int *info, int waves, hipStream_t s)
+{
+    PotrfJobs J = {};
+    J.A = Akk; J.dinv = dinv;
+    J.np0 = ldt; J.ld0 = ldt; J.nvalid0 = nvalid;
+    J.count = 1; J.info = info; J.iinfo = iinfo; J.batch = 0;
+    if (waves == 8) hipLaunchKernelGGL(potrf_jobs_kernel<8>, dim3(1), dim3(512), 0, s, J);
+    else hipLaunchKernelGGL(potrf_jobs_kernel<4>, dim3(1), dim3(256), 0, s, J);
+}
+
+/* Batched form: `count` matrices, job j of order np[j] (multiple of 16)
+ * at A + off[j] with leading dimension ld[j] (null: np[j]), inverses at
+ * dinv + doff[j]; info[j] = first failing column or 0.  `queue` is a
+ * zeroed device counter; jobs are taken in index order by `grid`
+ * persistent workgroups (grid <= 0: as many as are resident at once; sort
+ * the jobs largest first for balance). */
+template <int W, bool LP>
+static int potrf_jobs_resident()
+{
+    static int resident = 0;
+    if (!resident) {
+        int dev = 0, ncu = 0, per = 0;
+        CHX_HIP(hipGetDevice(&dev));
+        CHX_HIP(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev));
+        CHX_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, potrf_jobs_kernel<W, LP>, W * 64, 0));
+        resident = ncu * (per > 0 ? per : 1);
+    }
+    return resident;
+}
+
+template <int W, bool LP>
+static void potrf_jobs_launch(const PotrfJobs &J, int grid, hipStream_t s)
+{
+    if (grid <= 0) grid = potrf_jobs_resident<W, LP>();
+    if (grid > J.count) grid = J.count;
+    hipLaunchKernelGGL((potrf_jobs_kernel<W, LP>), dim3(grid), dim3(W * 64), 0, s, J);
+}
+
+void potrf_jobs(double *A, const long long *off, const int *np, const int *ld, const int *nvalid, double *dinv,
+                const long long *doff, int count, int *queue, int *info, int grid, hipStream_t s, int waves, bool lp)
+{
+    PotrfJobs J = {};
+    J.A = A; J.off = off; J.np = np; J.ld = ld; J.nvalid = nvalid; J.dinv = dinv; J.doff = doff;
+    J.count = count; J.queue = queue; J.info = info; J.batch = 1;
+    if (count <= 0) return;
+    if (waves == 8) {
+        if (lp) potrf_jobs_launch<8, true>(J, grid, s);
+        else potrf_jobs_launch<8, false>(J, grid, s);
+    } else {
+        if (lp) potrf_jobs_launch<4, true>(J, grid, s);
+        else potrf_jobs_launch<4, false>(J, grid, s);
+    }
+}
+
+void potrf_jobs_prepare()
+{
+    (void)potrf_jobs_resident<4, false>();
+    (void)potrf_jobs_resident<8, false>();
+    (void)potrf_jobs_resident<4, true>();
+    (void)potrf_jobs_resident<8, true>();
 }
 
 } /* namespace k */
