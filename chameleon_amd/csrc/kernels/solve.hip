@@ -172,7 +172,8 @@ void solve_coop(const double *A, const double *TN, const double *TT, double *BT,
  * rows of block j+1 are loaded into registers (before waiting for its
  * publication: the factor does not depend on it) and its solution block
  * into staging registers, which go to LDS (one copy for the 4 waves)
- * after the block is done.  D_s goes to LDS before any wait.
+ * after the block is done.  This wave's rows of D_s are in registers before
+ * any wait.
  *
  * Publication is a per-strip flag set to this launch's epoch after a
  * device-scope release (the strip's stores written back from L2).  Readers
@@ -198,7 +199,7 @@ struct StripArgs {
     int ldd;
     double *BT;           /* right-hand sides, element (c, r) at c + r * nrp         */
     int *flags;           /* one per strip and column chunk: chunk c at flags + c*S   */
-    unsigned *ticket;     /* task counter of the launch (cleared before it)           */
+    unsigned *ticket;     /* task counter, zero between launches                      */
     int NT, ldt, nrp, c0; /* c0: first column of this launch's chunks                 */
     int nchunk;           /* column chunks of 16*NC columns solved side by side       */
     int S;                /* number of strips                                         */
@@ -228,6 +229,66 @@ __device__ __forceinline__ void load_op4(const double *M, int ld, bool vec, int 
     }
 }
 
+/* loads from a wave-uniform base: 32-bit byte offsets per lane (vo) and for the
+ * wave (so); DEV: device-scope (coherent) */
+typedef __amdgpu_buffer_rsrc_t rsrc_t;
+__device__ __forceinline__ rsrc_t sv_rsrc(const double *p)
+{
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<double *>(p), 0, 0x7fffffff, 0x00020000);
+}
+__device__ __forceinline__ double sv_ld(rsrc_t r, int vo, int so)
+{
+    return __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(r, vo, so, 0));
+}
+template <bool DEV = false>
+__device__ __forceinline__ v2d sv_ld2(rsrc_t r, int vo, int so)
+{
+    return __builtin_bit_cast(v2d, __builtin_amdgcn_raw_buffer_load_b128(r, vo, so, DEV ? 16 : 0));
+}
+
+/* acc[c] -= m X(., 16c ..) for a 64-row block X in LDS (element (r, c) at
+ * r * 16 NC + c): m[pc][q] is the operand at column 16 pc + 4 lk + q.  The LDS
+ * reads of a step go behind the products of the one before: left to itself the
+ * compiler reads each operand where it is used, an LDS latency per step. */
+template <int NC>
+__device__ __forceinline__ void strip_mma(const double (&m)[4][4], const double *X, int lane, v4d (&acc)[NC])
+{
+    const double *x0 = X + 4 * (lane >> 4) * 16 * NC + (lane & 15);
+    double x[2][NC];
+#pragma unroll
+    for (int c = 0; c < NC; ++c) x[0][c] = x0[c * 16];
+#pragma unroll
+    for (int k = 0; k < 16; ++k) {
+        if (k < 15) {
+#pragma unroll
+            for (int c = 0; c < NC; ++c) x[(k + 1) & 1][c] = x0[((k + 1) / 4 * 16 + (k + 1) % 4) * 16 * NC + c * 16];
+        }
+#pragma unroll
+        for (int c = 0; c < NC; ++c) acc[c] = mfma_f64(-m[k / 4][k % 4], x[k & 1][c], acc[c]);
+#pragma unroll
+        for (int c = 0; c < NC; ++c) {
+            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+            __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+        }
+    }
+}
+
+/* The next task of a strip launch, drawn by thread 0 into *s_task, for the
+ * whole workgroup between two barriers.  Every workgroup draws until a ticket
+ * past the last task comes, so the last draw of all is ntask + gridDim.x - 1;
+ * it clears the counter for the next launch (a clearing launch before each
+ * solve cost 5 us).  Past that the counter was not clear at the start, which
+ * is recorded as a stall; `skip` is set when the factorisation had failed at
+ * the first draw: the tasks are then drawn and left. */
+__device__ __forceinline__ void strip_draw(unsigned *ticket, int ntask, const int *info, int *s_task, int *s_skip)
+{
+    const unsigned t = atomicAdd(ticket, 1u), last = (unsigned)ntask + gridDim.x - 1;
+    if (t == last) __hip_atomic_store(ticket, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    else if (t > last) atomicCAS((int *)info, 0, PANEL_STALLED);
+    *s_task = t < (unsigned)ntask ? (int)t : ntask;
+    if (*s_skip < 0) *s_skip = __hip_atomic_load(info, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0;
+}
+
 #define SR 64            /* strip rows */
 /* polls of one flag wait before it gives up: about a second at ~0.3 us per
  * poll, far beyond any chain (a full direction at N = 32768 is ~3 ms) */
@@ -240,14 +301,15 @@ __global__ __launch_bounds__(256, 2) void strip_solve_kernel(StripArgs a)
     /* the solution block being consumed; after the block loop, the acc of
      * the strip (input of the diagonal product) */
     __shared__ double Xb[SR * NCOL];
-    __shared__ double Ds[SR * (SR + 1)];          /* D_s, element (r, p) at r + p*65 */
     double *Xs = Xb;
-    if (*a.info != 0) return;     /* uniform over the grid: nobody is left waiting */
-    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+    const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
     const int li = lane & 15, lk = lane >> 4;
     const int q = a.ldt / SR, nrp = a.nrp, ldt = a.ldt;
     const size_t ts = (size_t)ldt * ldt;
     const int wr = wave * 16;
+    /* this lane's place in a factor block and in a solution block, in bytes */
+    const int vl = FWD ? (wr + li + 4 * lk * ldt) * 8 : (4 * lk + (wr + li) * ldt) * 8;
+    const int vx = ((2 * tid) % NCOL + (2 * tid) / NCOL * nrp) * 8;
     /* the direction is a template parameter: with a run-time choice
      * between the two operand loads the compiler put a wait for all
      * outstanding loads before each 16-column piece of a factor block */
@@ -256,18 +318,19 @@ __global__ __launch_bounds__(256, 2) void strip_solve_kernel(StripArgs a)
     /* task t = (strip in chain order) * nchunk + chunk: the chunks are
      * independent chains, interleaved so that the tasks a task waits for
      * always have smaller indices.  Tasks are taken from a ticket counter
-     * (cleared before the launch), so every task a workgroup waits for
+     * (strip_draw), so every task a workgroup waits for
      * belongs to a workgroup that has started: the chain moves whatever
      * else occupies the device, no co-residency of the grid is needed. */
-    __shared__ int s_task;
-    unsigned *const ticket = a.ticket;
+    __shared__ int s_task, s_skip;
     const int ntask = (a.S - a.s0) * a.nchunk;
+    if (tid == 0) s_skip = -1;
     for (;;) {
         __syncthreads();
-        if (tid == 0) s_task = (int)atomicAdd(ticket, 1u);
+        if (tid == 0) strip_draw(a.ticket, ntask, a.info, &s_task, &s_skip);
         __syncthreads();
-        const int t = s_task;
+        const int t = __builtin_amdgcn_readfirstlane(s_task);
         if (t >= ntask) break;
+        if (s_skip) continue;
         const int si = t / a.nchunk, cc = t - si * a.nchunk;
         const int s = fwd ? a.s0 + si : a.S - 1 - si;
         const int c0 = a.c0 + cc * NCOL;
@@ -286,21 +349,15 @@ __global__ __launch_bounds__(256, 2) void strip_solve_kernel(StripArgs a)
         for (int c = 0; c < NC; ++c)
 #pragma unroll
             for (int e = 0; e < 4; ++e) acc[c][e] = Bs[(c * 16 + li) + (size_t)(wr + lk + 4 * e) * nrp];
-        /* D_s into LDS before any wait (read by the diagonal product) */
+        /* this wave's rows of D_s, and of E_s, before any wait */
         const double *Dg = a.D + (size_t)tm * a.dts + (size_t)(s % q) * a.doff;
-        {
-            /* all 16 loads in flight before the first LDS store */
-            double dv[SR * SR / 256];
+        double dv[NPC][4], ev[NPC][4];
 #pragma unroll
-            for (int h = 0; h < SR * SR / 256; ++h) {
-                const int e = tid + 256 * h;
-                dv[h] = Dg[(e % SR) + (size_t)(e / SR) * a.ldd];
-            }
+        for (int pc = 0; pc < NPC; ++pc) load_op4(Dg, a.ldd, lvec, wr, pc * 16, li, lk, dv[pc]);
+        if constexpr (PE) {
+            const double *Eg = a.E + (size_t)s * SR * SR;
 #pragma unroll
-            for (int h = 0; h < SR * SR / 256; ++h) {
-                const int e = tid + 256 * h;
-                Ds[(e % SR) + (e / SR) * (SR + 1)] = dv[h];
-            }
+            for (int pc = 0; pc < NPC; ++pc) load_op4(Eg, SR, false, wr, pc * 16, li, lk, ev[pc]);
         }
         const int pc0 = fwd ? 0 : wave, pc1 = fwd ? wave + 1 : NPC;   /* nonzero chunks of row group `wave` */
 
@@ -345,15 +402,9 @@ __global__ __launch_bounds__(256, 2) void strip_solve_kernel(StripArgs a)
             __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
         };
         auto stage_load = [&](int j, v2d (&xv)[XV]) {
-            const double *Xj = xblock(j);
+            const rsrc_t x = sv_rsrc(xblock(j));
 #pragma unroll
-            for (int h = 0; h < XV; ++h) {
-                const int e = 2 * (tid + 256 * h), r = e / NCOL, c = e % NCOL;
-                const unsigned long long *src = (const unsigned long long *)&Xj[c + (size_t)r * nrp];
-                const unsigned long long u0 = __hip_atomic_load(src, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                const unsigned long long u1 = __hip_atomic_load(src + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                xv[h] = v2d{__longlong_as_double((long long)u0), __longlong_as_double((long long)u1)};
-            }
+            for (int h = 0; h < XV; ++h) xv[h] = sv_ld2<true>(x, vx, h * (512 / NCOL) * 8 * nrp);
         };
         auto stage_store = [&](const v2d (&xv)[XV]) {
 #pragma unroll
@@ -374,56 +425,48 @@ __global__ __launch_bounds__(256, 2) void strip_solve_kernel(StripArgs a)
         if (nblk > 0) {
             double lcur[NPC][4], lnext[NPC][4];
             v2d xv[XV];
-            int j = fwd ? a.s0 : a.S - 1;
-            {
-                const double *L = block_of(j);
+            auto at = [&](int b) { return fwd ? a.s0 + b : a.S - 1 - b; };
+            auto load_l = [&](int b, double (&l)[NPC][4]) {
+                const rsrc_t L = sv_rsrc(block_of(at(b < nblk ? b : nblk - 1)));
 #pragma unroll
-                for (int pc = 0; pc < NPC; ++pc) load_op4(L, ldt, lvec, wr, pc * 16, li, lk, lcur[pc]);
-                wait_for(j);
-                stage_load(j, xv);
-                stage_store(xv);
-                __syncthreads();
-            }
-            for (int b = 0; b < nblk; ++b) {
-                const bool more = b + 1 < nblk;
-                const int jn = fwd ? j + 1 : j - 1;
-                if (more) {
-                    const double *L = block_of(jn);
+                for (int pc = 0; pc < NPC; ++pc) {
+                    if (lvec) {
+                        const v2d u = sv_ld2(L, vl, pc * 128), v = sv_ld2(L, vl, pc * 128 + 16);
+                        l[pc][0] = u[0]; l[pc][1] = u[1]; l[pc][2] = v[0]; l[pc][3] = v[1];
+                    } else {
 #pragma unroll
-                    for (int pc = 0; pc < NPC; ++pc) load_op4(L, ldt, lvec, wr, pc * 16, li, lk, lnext[pc]);
+                        for (int qq = 0; qq < 4; ++qq) l[pc][qq] = sv_ld(L, vl, (pc * 16 + qq) * 8 * ldt);
+                    }
                 }
+            };
+            auto products = [&]() { strip_mma<NC>(lcur, Xb, lane, acc); };
+            auto take_l = [&](int b) {
 #pragma unroll
                 for (int pc = 0; pc < NPC; ++pc)
 #pragma unroll
-                    for (int qq = 0; qq < 4; ++qq)
-#pragma unroll
-                        for (int c = 0; c < NC; ++c)
-                            acc[c] = mfma_f64(-lcur[pc][qq], Xb[(pc * 16 + 4 * lk + qq) * NCOL + c * 16 + li], acc[c]);
-                if (more) {
-                    wait_for(jn);
-                    stage_load(jn, xv);
-                }
+                    for (int qq = 0; qq < 4; ++qq) lcur[pc][qq] = lnext[pc][qq];
+                load_l(b, lnext);
+            };
+            load_l(0, lcur);
+            load_l(1, lnext);
+            wait_for(at(0));
+            stage_load(at(0), xv);
+            stage_store(xv);
+            __syncthreads();
+            /* block b is in Xb and lcur, the factor's block b+1 on its way */
+            for (int b = 0;; ++b) {
+                products();
+                if (b == nblk - 1) break;
+                wait_for(at(b + 1));
+                stage_load(at(b + 1), xv);
                 __syncthreads();                 /* every wave is done with Xb */
-                if (more) {
-                    stage_store(xv);
-#pragma unroll
-                    for (int pc = 0; pc < NPC; ++pc)
-#pragma unroll
-                        for (int qq = 0; qq < 4; ++qq) lcur[pc][qq] = lnext[pc][qq];
-                }
+                stage_store(xv);
+                take_l(b + 2);
                 __syncthreads();                 /* the next block is in Xb */
-                j = jn;
             }
+            __syncthreads();
         }
 
-        /* the predecessor product's operand, requested before the
-         * diagonal step (its latency hides behind it) */
-        double ev[NPC][4];
-        if constexpr (PE) {
-            const double *Eg = a.E + (size_t)s * SR * SR;
-#pragma unroll
-            for (int pc = 0; pc < NPC; ++pc) load_op4(Eg, SR, false, wr, pc * 16, li, lk, ev[pc]);
-        }
         /* diagonal block: X_s = D_s acc (forward) or D_s^T acc (backward) */
 #pragma unroll
         for (int c = 0; c < NC; ++c)
@@ -433,14 +476,18 @@ __global__ __launch_bounds__(256, 2) void strip_solve_kernel(StripArgs a)
         v4d x[NC];
 #pragma unroll
         for (int c = 0; c < NC; ++c) x[c] = zero4d();
-        for (int pc = pc0; pc < pc1; ++pc) {
 #pragma unroll
-            for (int qq = 0; qq < 4; ++qq) {
-                const int p = pc * 16 + 4 * lk + qq, r = wr + li;
-                const double dv = fwd ? Ds[r + p * (SR + 1)] : Ds[p + r * (SR + 1)];
+        for (int pc = 0; pc < NPC; ++pc) {
+            if (pc < pc0 || pc >= pc1) continue;
+            double xd[4][NC];
 #pragma unroll
-                for (int c = 0; c < NC; ++c) x[c] = mfma_f64(dv, Xs[p * NCOL + c * 16 + li], x[c]);
-            }
+            for (int qq = 0; qq < 4; ++qq)
+#pragma unroll
+                for (int c = 0; c < NC; ++c) xd[qq][c] = Xs[(pc * 16 + 4 * lk + qq) * NCOL + c * 16 + li];
+#pragma unroll
+            for (int qq = 0; qq < 4; ++qq)
+#pragma unroll
+                for (int c = 0; c < NC; ++c) x[c] = mfma_f64(dv[pc][qq], xd[qq][c], x[c]);
         }
         if (PE && use_e) {
             /* X_s -= E_s X_pred once the predecessor is published */
@@ -451,13 +498,7 @@ __global__ __launch_bounds__(256, 2) void strip_solve_kernel(StripArgs a)
             __syncthreads();                     /* every wave is done with Xs */
             stage_store(xv);
             __syncthreads();
-#pragma unroll
-            for (int pc = 0; pc < NPC; ++pc)
-#pragma unroll
-                for (int qq = 0; qq < 4; ++qq)
-#pragma unroll
-                    for (int c = 0; c < NC; ++c)
-                        x[c] = mfma_f64(-ev[pc][qq], Xb[(pc * 16 + 4 * lk + qq) * NCOL + c * 16 + li], x[c]);
+            strip_mma<NC>(ev, Xb, lane, x);
         }
         {
             /* publication by completion: X_s is written with device-scope
@@ -493,7 +534,6 @@ static void strip_launch_dir(const StripArgs &a, hipStream_t s)
     }
     int grid = ncu * per_cu;
     if (grid > (a.S - a.s0) * a.nchunk) grid = (a.S - a.s0) * a.nchunk;
-    zero_ints(reinterpret_cast<int *>(a.ticket), 1, s);
     hipLaunchKernelGGL((strip_solve_kernel<NC, PE, FWD>), dim3(grid), dim3(256), 0, s, a);
 }
 
@@ -536,7 +576,7 @@ struct NarrowArgs {
                            * D128 + s * 16384, element (r, p) at r + p * 128            */
     double *BT;           /* right-hand sides, element (c, r) at c + r * nrp            */
     int *flags;           /* one per strip                                              */
-    unsigned *ticket;     /* task counter of the launch (cleared before it)              */
+    unsigned *ticket;     /* task counter, zero between launches                         */
     int NT, ldt, nrp;
     int S, s0;            /* strips of 128 rows; forward: first strip solved            */
     int trans, epoch;
@@ -557,8 +597,7 @@ __global__ __launch_bounds__(512, 1) void strip_narrow_kernel(NarrowArgs a)
     double *const T = smem;               /* backward: op(r, p) at T[r*TLD + p]               */
     double (*const P)[NSR * NCV] = reinterpret_cast<double (*)[NSR * NCV]>(smem);   /* partial sums */
     double *const Acc = smem + 4 * NSR * NCV;                                        /* diagonal input */
-    __shared__ int s_task;
-    if (*a.info != 0) return;     /* uniform over the grid at launch */
+    __shared__ int s_task, s_skip;
     /* wave and k range are uniform over a wavefront: scalar registers, so
      * the uniform part of every load address is scalar too */
     const int tid = threadIdx.x, lane = tid & 63;
@@ -568,12 +607,14 @@ __global__ __launch_bounds__(512, 1) void strip_narrow_kernel(NarrowArgs a)
     const size_t ts = (size_t)ldt * ldt;
     constexpr bool fwd = FWD;
     const int ntask = a.S - a.s0;
+    if (tid == 0) s_skip = -1;
     for (;;) {
         __syncthreads();
-        if (tid == 0) s_task = (int)atomicAdd(a.ticket, 1u);
+        if (tid == 0) strip_draw(a.ticket, ntask, a.info, &s_task, &s_skip);
         __syncthreads();
         const int t = s_task;
         if (t >= ntask) break;
+        if (s_skip) continue;
         const int s = fwd ? a.s0 + t : a.S - 1 - t;
         const int tm = s / q, rs = (s % q) * NSR;
         double *Bs = a.BT + (size_t)s * NSR * nrp;
@@ -773,7 +814,6 @@ static void narrow_launch(const NarrowArgs &a, hipStream_t s)
     }
     int grid = ncu * per_cu;
     if (grid > a.S - a.s0) grid = a.S - a.s0;
-    zero_ints(reinterpret_cast<int *>(a.ticket), 1, s);
     if (a.trans)
         hipLaunchKernelGGL((strip_narrow_kernel<NCV, false>), dim3(grid), dim3(512), 0, s, a);
     else
@@ -969,39 +1009,33 @@ int solve_strips(const double *A, const double *D, long long dts, long long doff
     a.trans = trans;
     a.info = info;
     a.E = E;
-    /* groups of up to 64 columns per launch; a full group is split into
-     * two chunks of 32 columns that run as separate chains side by side
-     * (shorter work per chain link).  Each chunk fetches the factor rows
-     * past the L2 itself: at N = 32768, NRHS 64 two chunks fetch ~10.5 GB
-     * per direction for a 4.4 GB factor, and still beat one 64-column
-     * chain (3.2 against 4.0 ms) or four 16-column ones (3.9 ms). */
-    const int snc = 2;
+    /* Groups of up to 64 columns per launch, in chunks of 16 or 32 columns that
+     * run as separate chains side by side.  A chain link costs 2.4 us with 16
+     * columns and 3.3 with 32 (0.45 us of matrix instructions per 16 columns,
+     * twice, and the transfers), but every chunk fetches the factor for itself,
+     * which counts once there are more tasks than places (two workgroups on a
+     * compute unit).  dpotrs in us, chunks of 16 / 32: N = 4096, 64 columns (256
+     * tasks of 16) 493 / 576, 8192 (512) 886 / 1017, 16384 (1024) 2085 / 1978,
+     * 32768 (2048) 6100 / 5310; 32 columns, 24576 (768) 2608 / 2789, 32768 (1024)
+     * 4025 / 3751.  48 columns do not divide into chunks of 32: three of 16, 4990
+     * at N = 32768 (one of 48 took 6150). */
+    static const int ncu = [] {
+        int dev = 0, n = 0;
+        CHX_HIP(hipGetDevice(&dev));
+        CHX_HIP(hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev));
+        return n;
+    }();
     int used = 0;
     for (int c0 = 0; c0 < nrp; c0 += 64) {
         const int cols = (nrp - c0 >= 64) ? 64 : nrp - c0;
         a.c0 = c0;
         a.epoch = epoch + used++;
-        int nc = cols / 16;
-        a.nchunk = 1;
-        if (cols == 64 && snc < 4) {
-            nc = snc;
-            a.nchunk = 4 / snc;
-        }
-        /* the predecessor products for chunks of 16 and 32 columns (wider
-         * chunks would not fit their registers) */
-        if (nc <= 2 && E) {
-            if (nc == 1) strip_launch<1, true>(a, s);
-            else strip_launch<2, true>(a, s);
-        } else {
-            a.E = nullptr;
-            switch (nc) {
-            case 1: strip_launch<1, false>(a, s); break;
-            case 2: strip_launch<2, false>(a, s); break;
-            case 3: strip_launch<3, false>(a, s); break;
-            default: strip_launch<4, false>(a, s); break;
-            }
-            a.E = E;
-        }
+        const int nc = (cols % 32 != 0 || (a.S - a.s0) * (cols / 16) <= 3 * ncu) ? 1 : 2;
+        a.nchunk = cols / 16 / nc;
+        if (nc == 1 && E) strip_launch<1, true>(a, s);
+        else if (nc == 1) strip_launch<1, false>(a, s);
+        else if (E) strip_launch<2, true>(a, s);
+        else strip_launch<2, false>(a, s);
     }
     return used;
 }
