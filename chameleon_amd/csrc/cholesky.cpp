@@ -166,8 +166,16 @@ void potrf_run(const PotrfPlan &p)
          *           [wait bulk(k-2,k-1)] columns k+2, k+3 by panels k, k+1
          *           (one two-column launch);
          *           POTRF+TRSM(k+2)
-         *   update: bulk(k, k+1) on the columns from k+4 (after panel k+1)
-         * Events: 2k = panel k+1 done, 2k+1 = bulk(k, k+1) done. */
+         *   update: [after the two-column launch] bulk(k, k+1) on the
+         *           columns from k+4
+         * Started together, the two updates share the compute units, the
+         * columns the next panel waits for end as late as the bulk, and the
+         * panels then have the device to themselves; one after the other, the
+         * bulk runs beside the panels.  dposv, together and in turn: N = 4096
+         * (nb 320) 1.97 and 1.86 ms, N = 7003 (256) 5.38 and 5.11, N = 10000
+         * (192) 9.93 and 9.54, N = 16384 (512) 29.9 and 29.7, N = 32768 (512)
+         * 198.6 and 196.3.
+         * Events: 2k = columns k+2, k+3 done, 2k+1 = bulk(k, k+1) done. */
         CHX_HIP(hipEventRecord(event(0), sm));
         CHX_HIP(hipStreamWaitEvent(su, event(0), 0));
         panel(0);
@@ -176,15 +184,15 @@ void potrf_run(const PotrfPlan &p)
             update(k, k + 1, k + 2, sm);
             panel(k + 1);
             if (k + 2 >= NT) break;
-            CHX_HIP(hipEventRecord(event(2 * k), sm));
-            CHX_HIP(hipStreamWaitEvent(su, event(2 * k), 0));
-            update(k, k + 4, NT, su, 2);
-            CHX_HIP(hipEventRecord(event(2 * k + 1), su));
             if (p.after_panels) p.after_panels(p.after_arg, k + 1);
             xfer_stream_columns(p.A, k + 2, sm);        /* tile columns 0..k+1 are final */
             if (last_bulk >= 0) CHX_HIP(hipStreamWaitEvent(sm, event(2 * last_bulk + 1), 0));
             last_bulk = k;
             update(k, k + 2, k + 4, sm, 2);
+            CHX_HIP(hipEventRecord(event(2 * k), sm));
+            CHX_HIP(hipStreamWaitEvent(su, event(2 * k), 0));
+            update(k, k + 4, NT, su, 2);
+            CHX_HIP(hipEventRecord(event(2 * k + 1), su));
             panel(k + 2);
         }
         if (last_bulk >= 0) CHX_HIP(hipStreamWaitEvent(sm, event(2 * last_bulk + 1), 0));
