@@ -113,8 +113,10 @@ __device__ __forceinline__ void decode_pair(int pair, int n0, int ncol, int NT, 
 }
 
 /* ------------------------------------------------------------------ */
-/* FP32-operand trailing update: A(m,n) -= P(m) P(n)^T, 128 x 128 block, 8
- * wavefronts of 64 x 32, K in 32-deep LDS slices (double-buffered). */
+/* FP32-operand trailing update: A(m,n) -= P(m) P(n)^T, BM x BN block (128: 8
+ * wavefronts of 64 x 32; 64 and 32: 4), K in 32-deep LDS slices
+ * (double-buffered).  A block alone on its compute unit waits for each slice
+ * (41 us for K 512 whatever the launch); see trailing_update_lp. */
 template <int BM, int BN, int WM, int WN>
 __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64, 2) void update_f32_kernel(
     double *A, const float *P, const float *P2, int lmt, int ldt, int n0, int ncol, int total_blocks,
@@ -221,14 +223,14 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64, 2) void update_f32_kern
  * different 4-bank groups.  The next slice is loaded into registers while
  * the current one is multiplied.  Both measured together: 246 -> 274
  * TFLOP/s FP64-equivalent on one paired launch (neither alone helps). */
-template <int SPLIT>
-__global__ __launch_bounds__(512, 4) void update_bf16_kernel(double *A, const unsigned short *P,
+template <int SPLIT, int BM, int BN, int WM, int WN>
+__global__ __launch_bounds__((BM / WM) * (BN / WN) * 64, 4) void update_bf16_kernel(double *A, const unsigned short *P,
                                                              const unsigned short *P2, int NT, int lmt, int ldt,
                                                              int n0, int ncol, int total_blocks, const int *info,
                                                              const unsigned char *pmap, int atomic_c)
 {
-    constexpr int BM = 128, BN = 128, WM = 64, WN = 32, BK = 64, LDK = BK;
-    constexpr int FM = WM / 16, FN = WN / 16, NTH = 512;
+    constexpr int BK = 64, LDK = BK;
+    constexpr int FM = WM / 16, FN = WN / 16, NTH = (BM / WM) * (BN / WN) * 64;
     constexpr int NP = (SPLIT == 3) ? 2 : 1;          /* planes per operand */
     constexpr int LA = (BM * BK) / (8 * NTH), LB = (BN * BK) / (8 * NTH);
     __shared__ unsigned short As[NP][BM * LDK];
@@ -639,19 +641,40 @@ void trailing_update_lp(double *A, const void *P, const void *P2, int mode, int 
     if (n0 >= NT || n1 <= n0) return;
     int ncol = 0;
     const int npairs = update_pairs(n0, n1, NT, &ncol);
-    const int bpt = (ldt / 128) * (ldt / 128);
-    const long long total = (long long)npairs * bpt;
-    if (total <= 0) return;
+    if (npairs <= 0) return;
+    static const int ncu = [] {
+        int dev = 0, n = 0;
+        CHX_HIP(hipGetDevice(&dev));
+        CHX_HIP(hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev));
+        return n;
+    }();
+    /* Block size by the launch's work in 64 x 64 blocks, as for the FP64 update.
+     * One launch on 256 compute units, us with 32 / 64 / 128 blocks:
+     *   FP32, one tile column, ldt 256, K 256: 128 blocks 8.0 / 11.8 / 23.7,
+     *     800 26 / 33 / 39; triangle, ldt 256, K 512: 1680 83 / 80 / 87; ldt 512,
+     *     K 1024: 6720 576 / 493 / 499, 10944 947 / 797 / 771
+     *   BF16 (3 products), ldt 256, K 256: 128 6.4 / 7.7 / 10.6; ldt 512, K 1024:
+     *     512 29 / 26 / 35, 2304 110 / 78 / 95, 6720 313 / 209 / 216, 19200
+     *     927 / 626 / 576.
+     * The order of the sum over k is the same in all. */
+    const long long b64 = (long long)npairs * (ldt / 64) * (ldt / 64);
+    const int bs = mode == 3 || b64 > 32LL * ncu ? 128 : b64 > (mode == 0 ? 4LL : 2LL) * ncu ? 64 : 32;
+    const unsigned total = (unsigned)((long long)npairs * (ldt / bs) * (ldt / bs)), nt = bs == 128 ? 512 : 256;
     const int ac = atomic_tile_updates();
-    if (mode == 0)
-        hipLaunchKernelGGL((update_f32_kernel<128, 128, 64, 32>), dim3((unsigned)total), dim3(512), 0, s, A,
-                           (const float *)P, (const float *)P2, lmt, ldt, n0, ncol, (int)total, info, pmap, ac);
-    else if (mode == 3)
-        hipLaunchKernelGGL(update_fp8_kernel, dim3((unsigned)total), dim3(512), 0, s, A, (const unsigned char *)P,
+    if (mode == 0) {
+        auto *kern = bs == 128 ? update_f32_kernel<128, 128, 64, 32>
+                   : bs == 64  ? update_f32_kernel<64, 64, 32, 32> : update_f32_kernel<32, 32, 16, 16>;
+        hipLaunchKernelGGL(kern, dim3(total), dim3(nt), 0, s, A, (const float *)P, (const float *)P2, lmt, ldt, n0, ncol,
+                           (int)total, info, pmap, ac);
+    } else if (mode == 3) {
+        hipLaunchKernelGGL(update_fp8_kernel, dim3(total), dim3(nt), 0, s, A, (const unsigned char *)P,
                            (const unsigned char *)P2, NT, lmt, ldt, n0, ncol, (int)total, info, ac);
-    else {
-        auto *kern = mode == 1 ? update_bf16_kernel<1> : update_bf16_kernel<3>;
-        hipLaunchKernelGGL(kern, dim3((unsigned)total), dim3(512), 0, s, A, (const unsigned short *)P,
+    } else {
+        auto *one = bs == 128 ? update_bf16_kernel<1, 128, 128, 64, 32>
+                  : bs == 64  ? update_bf16_kernel<1, 64, 64, 32, 32> : update_bf16_kernel<1, 32, 32, 16, 16>;
+        auto *three = bs == 128 ? update_bf16_kernel<3, 128, 128, 64, 32>
+                    : bs == 64  ? update_bf16_kernel<3, 64, 64, 32, 32> : update_bf16_kernel<3, 32, 32, 16, 16>;
+        hipLaunchKernelGGL((mode == 1 ? one : three), dim3(total), dim3(nt), 0, s, A, (const unsigned short *)P,
                            (const unsigned short *)P2, NT, lmt, ldt, n0, ncol, (int)total, info, pmap, ac);
     }
 }
