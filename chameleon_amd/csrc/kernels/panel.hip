@@ -292,15 +292,19 @@ void trsm_right_lower_trans(double *panel, int ntiles, size_t tile_stride, int l
  *
  * Measured on MI355X, the launch alone, against one owner per 64 rows with two
  * exchanges per link and the 64 x 64 inverse on the chain (us; tile size, tiles
- * below): 128, 0: 50 -> 37; 256, 27: 109 -> 70; 320, 12: 132 -> 86; 512, 0: 207 ->
- * 125; 512, 30: 227 -> 166; 512, 63: 301 -> 256.  One link is 14 us (was 25): 1.3
- * the substitution, 1.0 the first products, 4 x 1.2 the columns, the rest LDS
- * round trips and barriers between the steps.  With many tiles below, the
- * FP64 MFMAs are the bound (36 products of 64^3 per row unit, 1.9 us each).
+ * below): 128, 0: 50 -> 36; 256, 27: 109 -> 64; 320, 12: 132 -> 78; 512, 0: 207 ->
+ * 103; 512, 30: 227 -> 164; 512, 63: 301 -> 255.  One link is 11.4 us (was 25): 1.2
+ * the substitution, 0.9 the first products, 4 x 1.6 the steps (1.2 of it the
+ * columns), 3 x 0.5 and 2 x 0.4 the updates and barriers between them.  The other
+ * waves' share of each step is cut so that wave 0 never waits for them: it did
+ * for 0.8 us in the first and 0.5 in the second step, for the stores behind
+ * M(C)'s flag and for R(C+1).  With many tiles below, the FP64 MFMAs are the
+ * bound (36 products of 64^3 per row unit, 1.9 us each).
  *
  * Publication: a flag set to this launch's epoch after the data was written
- * with device-scope (coherent) stores, every wave has waited for its stores
- * to complete and the workgroup has met at a barrier; readers poll the flag
+ * with device-scope (coherent) stores and every wave has waited for its own
+ * to complete (the waves then meet at a barrier, or count themselves in LDS and
+ * the last one sets the flag); readers poll the flag
  * and read with device-scope loads, past the non-coherent L2 of other XCDs
  * (a release fence would write back the whole L2 at each link).  Everything
  * published goes through scratch, packed so that 64 units reading one block
@@ -368,21 +372,30 @@ __device__ __forceinline__ void pf_st(double v, rsrc_t r, int vo, int so)
     __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u2, v), r, vo, so, DEV ? 16 : 0);
 }
 
+template <bool DEV = false>
+__device__ __forceinline__ void pf_st2(v2d v, rsrc_t r, int vo, int so)
+{
+    typedef unsigned int u4 __attribute__((ext_vector_type(4)));
+    __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u4, v), r, vo, so, DEV ? 16 : 0);
+}
+
 /* Packed lower blocks.  A block below the diagonal: lane (li, lk) slot s of an
  * MFMA operand, element (li, lk + 4s), is at block + 64 s + lane.  The inverse
- * of a diagonal block has element (r, c) at (r ^ c) + 16 c, so that lanes on
- * consecutive columns (as pf_col16 leaves it) meet different banks too. */
+ * of a diagonal block has element (r, c) at (r ^ c) + 16 r: lanes on consecutive
+ * columns (as pf_col16 leaves it) or on consecutive rows meet different banks. */
 __device__ __forceinline__ constexpr int pf_low(int i, int j) { return (i * (i + 1) / 2 + j) * PF_BLK; }
-__device__ __forceinline__ int pf_inv(int r, int c) { return (r ^ c) + 16 * c; }
+__device__ __forceinline__ int pf_inv(int r, int c) { return (r ^ c) + 16 * r; }
 
 /* One wave's wait for flag idx of this launch; false if the factorisation
  * failed meanwhile (or the poll limit was reached).  The rows below, hundreds
  * of units on one flag, poll more rarely (SLEEP x 64 cycles between polls). */
 template <int SLEEP = 1>
-__device__ __forceinline__ bool pf_wave_wait(const PanelArgs &a, int idx)
+__device__ __forceinline__ bool pf_wave_wait(const PanelArgs &a, int idx, int idx2 = -1)
 {
+    const int at = idx2 >= 0 && (threadIdx.x & 1) ? idx2 : idx;      /* both flags in one load */
     for (int n = 0;; ++n) {
-        if (__hip_atomic_load(&a.flags[idx], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == a.epoch) return true;
+        const bool set = __hip_atomic_load(&a.flags[at], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == a.epoch;
+        if (__ballot(!set) == 0) return true;
         if ((n & 7) == 7 && __hip_atomic_load(a.info, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0) return false;
         if (n > PF_SPIN_LIMIT) {
             atomicCAS(a.info, 0, PANEL_STALLED);
@@ -397,7 +410,7 @@ template <int SLEEP = 1>
 __device__ __forceinline__ bool pf_wait(const PanelArgs &a, int idx, int tid, int *s_bad, int idx2 = -1)
 {
     if (tid < 64) {
-        const bool ok = pf_wave_wait<SLEEP>(a, idx) && (idx2 < 0 || pf_wave_wait<SLEEP>(a, idx2));
+        const bool ok = pf_wave_wait<SLEEP>(a, idx, idx2);
         if (tid == 0) *s_bad = !ok;
     }
     __syncthreads();
@@ -475,8 +488,30 @@ __device__ __forceinline__ void pf_subst(const double *Ms, int lane, v4d (&y)[4]
 __device__ __forceinline__ v4d pf_syrk(const double *Xs, int i, int j, int lane, v4d d)
 {
     const double *row = Xs + (lane >> 4) * 64 + (lane & 15);
+    double xi[2][4], xj[2][4];
 #pragma unroll
-    for (int q = 0; q < 16; ++q) d = mfma_f64(-row[256 * q + 16 * j], row[256 * q + 16 * i], d);
+    for (int q = 0; q < 4; ++q) {
+        xi[0][q] = row[256 * q + 16 * i];
+        xj[0][q] = row[256 * q + 16 * j];
+    }
+#pragma unroll
+    for (int b = 0; b < 4; ++b) {
+        if (b < 3) {
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                xi[(b + 1) & 1][q] = row[256 * (4 * b + 4 + q) + 16 * i];
+                xj[(b + 1) & 1][q] = row[256 * (4 * b + 4 + q) + 16 * j];
+            }
+        }
+#pragma unroll
+        for (int q = 0; q < 4; ++q) d = mfma_f64(-xj[b & 1][q], xi[b & 1][q], d);
+    }
+    __builtin_amdgcn_sched_group_barrier(0x100, 4, 0);
+#pragma unroll
+    for (int q = 0; q < 16; ++q) {
+        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+        __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+    }
     return d;
 }
 
@@ -512,6 +547,31 @@ __device__ __forceinline__ int pf_col16(double (&a)[16], int lane)
 #pragma unroll
     for (int j = 0; j < 16; ++j) a[j] *= readlane_f64(rs, j);
     return __builtin_ffsll((long long)bad);
+}
+
+/* One 16-column step of a 64 x 64 block whose lower 16 x 16 blocks are in Db,
+ * by one wavefront: lane group lk < nr takes block (c + lk, c), group nr rows of
+ * the identity (Id, in LDS).  L(c, c) goes to Ld, the blocks below it back to
+ * their place, the inverse of L(c, c) to the diagonal one's.  Every lane has one
+ * place to read from and one to write to: as three kinds of lanes each with
+ * loads, selects and stores of their own, a step was 2.1 us, with 1.2 for the
+ * columns; now 1.6.  Returns the failing column or 0. */
+__device__ __forceinline__ int pf_step16(double *Db, double *Ld, const double *Id, int c, int nr, int lane)
+{
+    const int li = lane & 15, lk = lane >> 4;
+    const int low = pf_low(lk < nr ? c + lk : c, c);
+    const double *const src = lk < nr ? Db + low : Id;
+    double *const dst = (lk == 0 ? Ld + c * PF_BLK : Db + low) + li;
+    const int flip = lk == nr ? 15 : 0;      /* the inverse's element (q, li) is at 16 q + (li ^ q) */
+    double v[16];
+#pragma unroll
+    for (int q = 0; q < 16; ++q) v[q] = src[li + 16 * q];
+    const int fail = pf_col16(v, lane);
+    if (lk <= nr) {
+#pragma unroll
+        for (int q = 0; q < 16; ++q) dst[16 * q + ((li ^ (q & flip)) - li)] = v[q];
+    }
+    return fail;
 }
 
 /* The 64 x 64 inverse from M, into dinv (column-major, zeros above the
@@ -572,7 +632,8 @@ __device__ __forceinline__ double *pf_xw(const PanelArgs &a, int r, int C)
 struct PanelLds {
     double Xs[4096];
     double B[2][PF_LOW];
-    int s_int, s_fail;
+    double Id[PF_BLK];       /* identity */
+    int s_int, s_fail, s_parts;
 };
 
 /* the chain (see above) */
@@ -582,7 +643,8 @@ __device__ __forceinline__ void panel_chain(const PanelArgs &a, PanelLds &L)
     const int li = lane & 15, lk = lane >> 4;
     const int ldt = a.ldt, ND = a.ND;
     double *const Xs = L.Xs;
-    if (tid == 0) L.s_fail = L.s_int = 0;
+    if (tid == 0) L.s_fail = L.s_int = L.s_parts = 0;
+    L.Id[tid] = (tid & 15) == (tid >> 4) ? 1.0 : 0.0;
     /* R(C) and D(C): rv this wave's rows of R, dcol block (wave, 0) of D, drest
      * blocks (wave, 1) and the wave-th of (2,2), (3,2), (3,3); block rows 0 and
      * 1 come from the tile, the others from their units */
@@ -597,6 +659,25 @@ __device__ __forceinline__ void panel_chain(const PanelArgs &a, PanelLds &L)
         double *const Db = L.B[cur], *const Ms = L.B[cur ^ 1], *const Ld = Ms + PF_LOW - 4 * PF_BLK;
         const rsrc_t rM = pf_rsrc(a.W + (size_t)C * PF_W);
         const rsrc_t rD = pf_rsrc(a.T + 64 * C + (size_t)64 * C * ldt);     /* the diagonal block in the tile */
+        /* a finished block of M to its scratch, and of L to the tile */
+        auto publish = [&](int i, int j) {
+            v2d m[2];
+#pragma unroll
+            for (int h = 0; h < 2; ++h) m[h] = *reinterpret_cast<const v2d *>(Db + pf_low(i, j) + 128 * h + 2 * lane);
+#pragma unroll
+            for (int h = 0; h < 2; ++h) pf_st2<true>(m[h], rM, lane * 16, (pf_low(i, j) + 128 * h) * 8);
+            if (i > j) {
+                const int v2 = (2 * (lane & 7) + (lane >> 3) * ldt) * 8;
+#pragma unroll
+                for (int h = 0; h < 2; ++h) pf_st2(m[h], rD, v2, tile_at(i, j) + 64 * h * ldt);
+            } else {
+#pragma unroll
+                for (int s = 0; s < 4; ++s) {
+                    const double y = Ld[j * PF_BLK + 64 * s + lane];
+                    if (li >= lk + 4 * s) pf_st(y, rD, vt, tile_at(j, j) + 32 * s * ldt);
+                }
+            }
+        };
         if (C == 0) {
             double d[10];
             const int vo = ((tid & 15) + (tid >> 4) * ldt) * 8;
@@ -617,6 +698,10 @@ __device__ __forceinline__ void panel_chain(const PanelArgs &a, PanelLds &L)
                 for (int s = 0; s < 4; ++s) dcol[s] = Db[(16 + s) * 64 + lane];
             }
             pf_subst(Ms, lane, rv);
+            if (wave == 1) {
+                pf_stores_done();
+                if (lane == 0) pf_set(a, (C - 1) * (ND + 1));
+            }
 #pragma unroll
             for (int f = 0; f < 4; ++f)
 #pragma unroll
@@ -636,28 +721,8 @@ __device__ __forceinline__ void panel_chain(const PanelArgs &a, PanelLds &L)
             /* wave 3 repeats the first block during the second step, for its
              * inverse: in the first there is no lane left for the identity */
             if (wave == 0 || (wave == 3 && cb == 1)) {
-                /* row group lk: block (c + lk, c), lk < nr, then identity rows */
-                const int c = wave == 0 ? cb : 0, nr = wave == 0 ? 4 - cb : 1;
-                const bool row = lk < nr;
-                double *const blk = Db + pf_low(row ? c + lk : c, c);
-                double v[16];
-#pragma unroll
-                for (int q = 0; q < 16; ++q) {
-                    const double x = blk[li + 16 * q];
-                    v[q] = row ? x : (q == li ? 1.0 : 0.0);
-                }
-                const int fail = pf_col16(v, lane);
-                if (lk == 0) {
-#pragma unroll
-                    for (int q = 0; q < 16; ++q)
-                        if (cb > 0) Ld[c * PF_BLK + li + 16 * q] = v[q];       /* L(c, c), for the tile */
-                } else if (row) {
-#pragma unroll
-                    for (int q = 0; q < 16; ++q) blk[li + 16 * q] = v[q];
-                } else if (lk == nr) {
-#pragma unroll
-                    for (int q = 0; q < 16; ++q) blk[pf_inv(q, li)] = q >= li ? v[q] : 0.0;
-                }
+                const int c = wave == 0 ? cb : 0;
+                const int fail = pf_step16(Db, Ld, L.Id, c, wave == 0 ? 4 - cb : 1, lane);
                 /* (the padding's own pivots do not count) */
                 const int col = 64 * C + 16 * c + fail;
                 if (lane == 0 && fail && col - 1 < a.nvalid) L.s_fail = col;
@@ -665,27 +730,44 @@ __device__ __forceinline__ void panel_chain(const PanelArgs &a, PanelLds &L)
                 if (C > 0) {
                     /* publish X(C, C-1) (R(C+1) waits for it), element (row lane, column k) */
                     const rsrc_t rP = pf_rsrc(pf_xw(a, C, C - 1));
+                    v2d xp[11];
 #pragma unroll
-                    for (int u = 0; u < 22; ++u) {
-                        const int k = min(3 * u + wave - 1, 63);
-                        pf_st<true>(Xs[64 * k + lane], rP, lane * 8, k * 512);
-                    }
-                    /* the products of the columns factored later */
+                    for (int u = 0; u < 11; ++u) xp[u] = *reinterpret_cast<const v2d *>(Xs + 128 * min(3 * u + wave - 1, 31) + 2 * lane);
 #pragma unroll
-                    for (int u = 0; u < 2; ++u) {
-                        const int i = u ? r2i : wave, j = u ? r2j : 1;
-                        const v4d x = pf_syrk(Xs, i, j, lane, drest[u]);
+                    for (int u = 0; u < 11; ++u) pf_st2<true>(xp[u], rP, lane * 16, min(3 * u + wave - 1, 31) * 1024);
+                    /* the products of column 1, and of (3, 3); in between, the
+                     * last wave whose part of X is out sets its flag */
+                    const v4d x = pf_syrk(Xs, wave, 1, lane, drest[0]);
 #pragma unroll
-                        for (int s = 0; s < 4; ++s) Db[pf_low(i, j) + 64 * s + lane] = x[s];
+                    for (int s = 0; s < 4; ++s) Db[pf_low(wave, 1) + 64 * s + lane] = x[s];
+                    pf_stores_done();
+                    if (lane == 0 && __hip_atomic_fetch_add(&L.s_parts, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) == 3 * C - 1)
+                        pf_set(a, C * ND + C - 1);
+                    if (wave == 3) {
+                        const v4d y = pf_syrk(Xs, 3, 3, lane, drest[1]);
+#pragma unroll
+                        for (int s = 0; s < 4; ++s) Db[pf_low(3, 3) + 64 * s + lane] = y[s];
                     }
                 }
             } else {
                 if (cb == 1 && C > 0) {
-                    if (wave == 1 && lane == 0) pf_set(a, C * ND + C - 1);
-                    /* X(C, C-1) to the tile */
+                    /* X(C, C-1) to the tile, two columns a store */
                     const rsrc_t rX = pf_rsrc(a.T + 64 * C + (size_t)64 * (C - 1) * ldt);
-#pragma unroll 8
-                    for (int k = 32 * (wave - 1); k < 32 * wave; ++k) pf_st(Xs[64 * k + lane], rX, lane * 8, k * ldt * 8);
+                    const int vx = (lane & 31) * 16 + (lane >> 5) * ldt * 8;
+#pragma unroll
+                    for (int h = 0; h < 2; ++h) {
+                        v2d xp[8];
+#pragma unroll
+                        for (int u = 0; u < 8; ++u)
+                            xp[u] = *reinterpret_cast<const v2d *>(Xs + 128 * (16 * (wave - 1) + 8 * h + u) + 2 * lane);
+#pragma unroll
+                        for (int u = 0; u < 8; ++u)
+                            pf_st2(xp[u], rX, vx, (16 * (wave - 1) + 8 * h + u) * 16 * ldt);
+                    }
+                    /* the products of (2, 2) and (3, 2) */
+                    const v4d x = pf_syrk(Xs, r2i, 2, lane, drest[1]);
+#pragma unroll
+                    for (int s = 0; s < 4; ++s) Db[pf_low(r2i, 2) + 64 * s + lane] = x[s];
                 }
                 if (cb < 3) {
                     /* what step cb-1 takes off the columns after cb: (2,2),
@@ -704,18 +786,9 @@ __device__ __forceinline__ void panel_chain(const PanelArgs &a, PanelLds &L)
                 }
                 /* publish the finished columns of M and store them to the
                  * tile: 0 and 1 beside step 2 (waves 2 and 3), 2 beside step 3 */
-                const int j = cb == 2 ? wave - 2 : cb == 3 && wave == 1 ? 2 : -1;
-                if (j >= 0) {
-                    for (int i = j; i < 4; ++i) {
-#pragma unroll
-                        for (int s = 0; s < 4; ++s) {
-                            const double x = Db[pf_low(i, j) + 64 * s + lane];
-                            pf_st<true>(x, rM, lane * 8, (pf_low(i, j) + 64 * s) * 8);
-                            const double y = i == j ? Ld[j * PF_BLK + 64 * s + lane] : x;
-                            if (i > j || li >= lk + 4 * s) pf_st(y, rD, vt, tile_at(i, j) + 32 * s * ldt);
-                        }
-                    }
-                }
+                const int j = cb == 2 ? wave - 2 : cb == 3 && wave == 3 ? 2 : -1;
+                if (j >= 0)
+                    for (int i = j; i < 4; ++i) publish(i, j);
                 if (cb == 3 && C + 1 < ND) {
                     /* R(C+1) and D(C+1), wave 0's share among them */
                     bool ok = true;
@@ -726,7 +799,7 @@ __device__ __forceinline__ void panel_chain(const PanelArgs &a, PanelLds &L)
                         rd = pf_rsrc(a.T + 64 + (size_t)64 * ldt);
                         vo = vt; sr = sd = 32 * ldt;
                     } else {
-                        ok = pf_wave_wait(a, C + 1) && pf_wave_wait(a, ND + C + 1);
+                        ok = pf_wave_wait(a, C + 1, ND + C + 1);
                         rr = pf_rsrc(a.W + (size_t)(C + 1) * PF_W + 2 * PF_LOW);
                         rd = pf_rsrc(a.W + (size_t)(C + 1) * PF_W + PF_LOW);
                         vo = lane * 8; sr = sd = 512;
@@ -756,7 +829,7 @@ __device__ __forceinline__ void panel_chain(const PanelArgs &a, PanelLds &L)
                     }
                 }
             }
-            if (cb == 0 || cb == 3) pf_stores_done();       /* X(C, C-1); M's columns */
+            if (cb == 3) pf_stores_done();                  /* M's columns */
             __syncthreads();
             if (L.s_fail) break;
             if (cb < 3) {
@@ -780,19 +853,12 @@ __device__ __forceinline__ void panel_chain(const PanelArgs &a, PanelLds &L)
             return;
         }
         if (L.s_int) return;
-        if (wave == 1) {
-#pragma unroll
-            for (int s = 0; s < 4; ++s)
-                pf_st<true>(Db[pf_low(3, 3) + 64 * s + lane], rM, lane * 8, (pf_low(3, 3) + 64 * s) * 8);
-            pf_stores_done();
-            if (lane == 0) pf_set(a, C * (ND + 1));
-        } else if (wave == 2) {
-#pragma unroll
-            for (int s = 0; s < 4; ++s) {
-                const double y = Ld[3 * PF_BLK + 64 * s + lane];
-                if (li >= lk + 4 * s) pf_st(y, rD, vt, tile_at(3, 3) + 32 * s * ldt);
-            }
-        }
+        /* the flag of M(C) follows when the stores are done, in the next link */
+        if (wave == 1) publish(3, 3);
+    }
+    if (wave == 1) {
+        pf_stores_done();
+        if (lane == 0) pf_set(a, (ND - 1) * (ND + 1));
     }
     pf_inverse<256>(L.B[cur ^ 1], Xs, a.dinv + (size_t)(ND - 1) * 4096, 64, tid, wave, lane);
 }
@@ -1225,8 +1291,9 @@ __global__ __launch_bounds__(POTRF_WAVES * 64, 2) void potrf_jobs_kernel(PotrfJo
     /* Ys holds the staged shared rows, Xs the 64 x 64 inverse on its way out,
      * Db the diagonal block's lower 16 x 16 blocks, which turn into L with the
      * inverses on the diagonal, and Ld the diagonal ones of L */
-    __shared__ double Xs[OB * OB], Ys[2 * 16 * OB], Db[PF_LOW], Ld[4 * PF_BLK];
+    __shared__ double Xs[OB * OB], Ys[2 * 16 * OB], Db[PF_LOW], Ld[4 * PF_BLK], Id[PF_BLK];
     __shared__ int s_fail, s_job;
+    for (int e = threadIdx.x; e < PF_BLK; e += NT) Id[e] = (e & 15) == (e >> 4) ? 1.0 : 0.0;
     if (!J.batch && *J.info != 0) return;
     /* the single-job form is on the critical path of the factorisation:
      * its waves win issue arbitration against co-resident update waves */
@@ -1268,28 +1335,8 @@ __global__ __launch_bounds__(POTRF_WAVES * 64, 2) void potrf_jobs_kernel(PotrfJo
 #pragma unroll 1
         for (int cb = 0; cb < nfb; ++cb) {
             if (wave == 0 || (wave == 3 && cb == 1 && nfb == 4)) {
-                /* row group lk: block (c + lk, c), lk < nr, then identity rows */
-                const int c = wave == 0 ? cb : 0, nr = wave == 0 ? nfb - cb : 1;
-                const bool row = lk < nr;
-                double *const blk = Db + pf_low(row ? c + lk : c, c);
-                double v[16];
-#pragma unroll
-                for (int q = 0; q < 16; ++q) {
-                    const double e = blk[li + 16 * q];
-                    v[q] = row ? e : (q == li ? 1.0 : 0.0);
-                }
-                const int fail = pf_col16(v, lane);
-                if (lk == 0) {
-#pragma unroll
-                    for (int q = 0; q < 16; ++q)
-                        if (nr < 4) Ld[c * PF_BLK + li + 16 * q] = v[q];
-                } else if (row) {
-#pragma unroll
-                    for (int q = 0; q < 16; ++q) blk[li + 16 * q] = v[q];
-                } else if (lk == nr) {
-#pragma unroll
-                    for (int q = 0; q < 16; ++q) blk[pf_inv(q, li)] = q >= li ? v[q] : 0.0;
-                }
+                const int c = wave == 0 ? cb : 0;
+                const int fail = pf_step16(Db, Ld, Id, c, wave == 0 ? nfb - cb : 1, lane);
                 if (lane == 0 && fail) s_fail = C + 16 * c + fail - 1 < nvalid ? C + 16 * c + fail : -1;
             } else if (cb > 0 && cb < 3 && wave < 3) {
                 /* what step cb-1 takes off the columns after cb: (2,2), (3,2),
