@@ -238,12 +238,12 @@ SolvePlan solve_plan(double *A, int NT, int ldt, int nrp, int *d_info, int ncols
     SolvePlan p;
     p.R = (ldt % 64 == 0) ? 64 : 0;
     p.ncols = ncols;
-    const bool narrow = k::narrow_eligible(ldt, ncols);
+    const bool narrow = k::narrow_eligible(ldt, NT, ncols);
     const size_t ntile_inv = p.R == 64 ? 0 : 2;
-    /* the narrow solve's 128 x 128 strip inverses, or the MFMA strip
-     * solve's predecessor products (both directions) */
+    /* the narrow solve's 128 x 128 strip inverses, and the predecessor
+     * products of either strip solve (both directions) */
     const size_t n128 = narrow ? (size_t)NT * ldt * 128 : 0;
-    const size_t npe = (!narrow && p.R == 64) ? 2 * (size_t)NT * ldt * 64 : 0;
+    const size_t npe = narrow ? (k::narrow_products(ldt, NT) ? 2 * n128 : 0) : p.R == 64 ? 2 * (size_t)NT * ldt * 64 : 0;
     const size_t need = (ntile_inv * NT * ts + (size_t)nrp * NT * ldt + (size_t)nrp * ldt + (size_t)NT * dper + n128 +
                          npe) * sizeof(double);
     double *ws = (double *)workspace(need);
@@ -252,12 +252,14 @@ SolvePlan solve_plan(double *A, int NT, int ldt, int nrp, int *d_info, int ncols
     p.dinv = p.W + (size_t)nrp * ldt;
     p.d128 = narrow ? p.dinv + (size_t)NT * dper : nullptr;
     p.ef = npe ? p.dinv + (size_t)NT * dper + n128 : nullptr;
-    p.eb = npe ? p.ef + (size_t)NT * ldt * 64 : nullptr;
+    p.eb = npe ? p.ef + npe / 2 : nullptr;
     p.TT = ntile_inv ? p.dinv + (size_t)NT * dper + n128 + npe : nullptr;
     p.TN = ntile_inv ? p.TT + (size_t)NT * ts : nullptr;
     k::dinv_all(A, NT, (size_t)(NT + 1) * ts, ldt, p.dinv, sm);
-    if (narrow) k::dinv128(A, p.dinv, (long long)dper, 64LL * 64, 64, NT, ldt, p.d128, sm);
-    if (npe) k::strip_products(A, p.dinv, (long long)dper, 64LL * 64, 64, NT, ldt, p.ef, p.eb, sm);
+    if (narrow) {
+        k::dinv128(A, p.dinv, (long long)dper, 64LL * 64, 64, NT, ldt, p.d128, sm);
+        if (npe) k::strip_products128(A, p.d128, NT, ldt, p.ef, p.eb, sm);
+    } else if (npe) k::strip_products(A, p.dinv, (long long)dper, 64LL * 64, 64, NT, ldt, p.ef, p.eb, sm);
     if (p.R == 64) return p;
     k::set_identity(p.TT, NT, ldt, sm);
     k::trsm_right_lower_trans_batched(p.TT, NT, (long long)ts, ldt, A, (long long)(NT + 1) * ts, p.dinv,
@@ -502,12 +504,15 @@ void potrf_solve_run(PotrfPlan p, double *BT, int nrp, int nrhs, double rate)
     const double n = (double)(NT - 1) * p.nb + p.nvalid_last, rows_left = n - (double)f.next * p.nb;
     /* with few right-hand sides: the 128 x 128 strip inverses, from the
      * panels' 64 x 64 ones (all final once potrf_run has issued) */
-    const bool narrow = p.d128 && k::narrow_eligible(ldt, nrhs);
-    if (narrow) k::dinv128(f.A, f.dinv, (long long)f.dper, 64LL * 64, 64, NT, ldt, p.d128, sm);
+    const bool narrow = p.d128 && k::narrow_eligible(ldt, NT, nrhs);
     const double *d128 = narrow ? p.d128 : nullptr;
-    /* otherwise the predecessor products of the MFMA strip solve */
-    double *ef = (!narrow && p.epred) ? p.epred : nullptr, *eb = ef ? ef + (size_t)NT * ldt * 64 : nullptr;
-    if (ef) k::strip_products(f.A, f.dinv, (long long)f.dper, 64LL * 64, 64, NT, ldt, ef, eb, sm);
+    /* and the predecessor products of either strip solve */
+    const size_t per = (size_t)NT * ldt * (narrow ? 128 : 64);
+    double *ef = !narrow ? p.epred : k::narrow_products(ldt, NT) ? p.d128 + per : nullptr, *eb = ef ? ef + per : nullptr;
+    if (narrow) {
+        k::dinv128(f.A, f.dinv, (long long)f.dper, 64LL * 64, 64, NT, ldt, p.d128, sm);
+        if (ef) k::strip_products128(f.A, p.d128, NT, ldt, ef, eb, sm);
+    } else if (ef) k::strip_products(f.A, f.dinv, (long long)f.dper, 64LL * 64, 64, NT, ldt, ef, eb, sm);
     timed(CHAMAMD_KERNEL_SOLVE, (rows_left * rows_left + n * n) * nrhs, sm, [&] {
         k::solve_strips(f.A, f.dinv, (long long)f.dper, 64LL * 64, 64, f.BT, NT, ldt, nrp, 0, flags, epoch,
                         lane_counters(L) + 2, p.d_info, sm, s0, d128, nrhs, ef);
@@ -537,8 +542,9 @@ int posv_async(cham_uplo_t uplo, CHAM_desc_t *A, CHAM_desc_t *B, RUNTIME_sequenc
     const size_t dper = (size_t)(ldt / 64) * 64 * 64;
     /* one workspace: the block inverses of the factorisation (where
      * potrf_run puts them), the transposed right-hand sides, and with few
-     * right-hand sides the 128 x 128 strip inverses of the solves */
-    const size_t n128 = k::narrow_eligible(ldt, B->n) ? (size_t)NT * ldt * 128 : 0;
+     * right-hand sides the 128 x 128 strip inverses of the solves and their
+     * predecessor products */
+    const size_t n128 = k::narrow_eligible(ldt, NT, B->n) ? 3 * (size_t)NT * ldt * 128 : 0;
     const size_t npe = n128 ? 0 : 2 * (size_t)NT * ldt * 64;      /* predecessor products */
     double *ws = (double *)workspace(((size_t)NT * dper + (size_t)nrp * NT * ldt + n128 + npe) * sizeof(double));
     double *BT = ws + (size_t)NT * dper;

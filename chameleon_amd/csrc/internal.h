@@ -237,8 +237,9 @@ struct PotrfPlan {
      * of the same factor read them there) */
     Lane *lane = nullptr;
     double *dinv = nullptr;
-    /* potrf_solve_run with at most 8 right-hand sides: room for the 128 x 128
-     * strip inverses (NT*ldt*128 doubles), or null for the MFMA strip solve */
+    /* potrf_solve_run with few right-hand sides: room for the 128 x 128
+     * strip inverses and their predecessor products (3 x NT*ldt*128 doubles),
+     * or null for the MFMA strip solve */
     double *d128 = nullptr;
     /* potrf_solve_run, MFMA strip solve: room for the predecessor products
      * (2 x NT*ldt*64 doubles), or null to solve without them */
@@ -262,7 +263,7 @@ void potrf_solve_run(PotrfPlan p, double *BT, int nrp, int nrhs, double rate);
 struct SolvePlan {
     double *TT, *TN, *BT, *W, *dinv;   /* diagonal-tile inverses, transposed RHS, one block, 64x64 inverses */
     double *d128 = nullptr;            /* 128 x 128 strip inverses (narrow solves), or null */
-    double *ef = nullptr, *eb = nullptr;   /* predecessor products (MFMA strip solve), or null */
+    double *ef = nullptr, *eb = nullptr;   /* predecessor products, or null */
     int ncols = 0;                     /* right-hand-side columns in use */
     int R = 0;                         /* 64: strip solve; 0: tile-step solve */
 };
@@ -406,22 +407,26 @@ void sumsq_tiles(const double *A, int ntiles, int ldt, double *part, hipStream_t
 void tile_gemm_nt(const double *A, int amt, const double *B, int bmt, double *C, int cmt, int ldt, int k0, int k1,
                   int r0, int nr, int c0, int nc, int lower, double alpha, double beta, hipStream_t s);
 /* solve.hip */
-/* ticket: one device counter, cleared by the call before each launch and
- * used by that launch only (launches on one stream may share it) */
-/* With D128 (dinv128 of the same factor) and 1 <= ncols <= 8 columns in
- * use with ldt a multiple of 128, the narrow kernel solves the first ncols
- * columns only (128-row strips, vector FMAs); otherwise the MFMA strip
- * kernel solves all nrp columns. */
-/* E (optional, MFMA kernel only): the predecessor products of this
- * direction from strip_products (Ef forward, Eb backward). */
+/* ticket: one device counter, zero between launches (each clears it at its
+ * end; launches on one stream may share it) */
+/* With D128 (dinv128 of the same factor) and narrow_eligible (ncols columns in
+ * use), the narrow kernel solves the first ncols columns only (128-row strips,
+ * vector FMAs); otherwise the MFMA strip kernel solves all nrp columns. */
+/* E (optional): the predecessor products of this direction (Ef forward, Eb
+ * backward), from strip_products128 for the narrow kernel, else from
+ * strip_products. */
 int solve_strips(const double *A, const double *D, long long dts, long long doff, int ldd, double *BT, int NT,
                  int ldt, int nrp, int trans, int *flags, int epoch, unsigned *ticket, const int *info, hipStream_t s,
                  int s0 = 0, const double *D128 = nullptr, int ncols = 0, const double *E = nullptr);
+/* predecessor products of the 128-row strips with inverses D128 (NT*ldt*128
+ * doubles each at Ef and Eb) */
+void strip_products128(const double *A, const double *D128, int NT, int ldt, double *Ef, double *Eb, hipStream_t s);
 /* predecessor products of the 64-row strips (NT*ldt*64 doubles each at Ef
  * and Eb): Ef_s = D_s L(s, s-1), Eb_s = (L(s+1, s) D_s)^T */
 void strip_products(const double *A, const double *D, long long dts, long long doff, int ldd, int NT, int ldt,
                     double *Ef, double *Eb, hipStream_t s);
-bool narrow_eligible(int ldt, int ncols);
+bool narrow_eligible(int ldt, int NT, int ncols);
+bool narrow_products(int ldt, int NT);
 /* 128 x 128 inverses of the diagonal blocks of the 128-row strips (NT*ldt*128
  * doubles at D128) from the 64 x 64 inverses D (addressed as in solve_strips) */
 void dinv128(const double *A, const double *D, long long dts, long long doff, int ldd, int NT, int ldt,

@@ -344,11 +344,16 @@ __global__ __launch_bounds__(256, 2) void strip_solve_kernel(StripArgs a)
         };
         auto xblock = [&](int j) -> const double * { return a.BT + c0 + (size_t)j * SR * nrp; };
 
-        v4d acc[NC];
+        /* 16 columns: the products are summed by themselves and taken from B at
+         * the end, which rounds less (they are small beside B in a dominant
+         * system); there are no registers for it with 32 */
+        v4d acc[NC], bv[NC];
 #pragma unroll
-        for (int c = 0; c < NC; ++c)
+        for (int c = 0; c < NC; ++c) {
 #pragma unroll
-            for (int e = 0; e < 4; ++e) acc[c][e] = Bs[(c * 16 + li) + (size_t)(wr + lk + 4 * e) * nrp];
+            for (int e = 0; e < 4; ++e) bv[c][e] = Bs[(c * 16 + li) + (size_t)(wr + lk + 4 * e) * nrp];
+            acc[c] = NC == 1 ? zero4d() : bv[c];
+        }
         /* this wave's rows of D_s, and of E_s, before any wait */
         const double *Dg = a.D + (size_t)tm * a.dts + (size_t)(s % q) * a.doff;
         double dv[NPC][4], ev[NPC][4];
@@ -471,7 +476,8 @@ __global__ __launch_bounds__(256, 2) void strip_solve_kernel(StripArgs a)
 #pragma unroll
         for (int c = 0; c < NC; ++c)
 #pragma unroll
-            for (int e = 0; e < 4; ++e) Xs[(wr + lk + 4 * e) * NCOL + c * 16 + li] = acc[c][e];
+            for (int e = 0; e < 4; ++e)
+                Xs[(wr + lk + 4 * e) * NCOL + c * 16 + li] = NC == 1 ? bv[c][e] + acc[c][e] : acc[c][e];
         __syncthreads();
         v4d x[NC];
 #pragma unroll
@@ -545,17 +551,19 @@ static void strip_launch(const StripArgs &a, hipStream_t s)
 }
 
 /* ------------------------------------------------------------------ */
-/* Narrow right-hand sides (at most 8 columns): strips of 128 rows solved
+/* Narrow right-hand sides (one or two columns): strips of 128 rows solved
  * with FP64 FMAs on the vector ALUs.
  *
  * An FP64 MFMA computes 16 columns whether or not they are in use, and on
  * this device the FP64 matrix and vector peaks are the same, so for one
- * to eight columns the vector ALUs do the chain's arithmetic 2-16x sooner
+ * or two columns the vector ALUs do the chain's arithmetic 8-16x sooner
  * and strips twice as tall halve the number of chain links (each link is
  * a few memory round trips: flag seen, solution block read, solution
  * stored and flag set).  The strip's diagonal step uses the 128 x 128
  * inverse of its diagonal block (D128, built by dinv128 from the 64 x 64
- * inverses): X_s = D128_s acc (forward) or D128_s^T acc (backward).
+ * inverses): X_s = D128_s acc (forward) or D128_s^T acc (backward), and with
+ * the predecessor products E (strip_products128, held in registers from before
+ * the first wait) as in strip_solve_kernel X_s = D128_s acc' - E_s X_pred.
  *
  * Workgroup of 512 threads per strip: thread (r, kq) = (tid % 128,
  * tid / 128) owns row r of the strip and the k range [32 kq, 32 kq + 32)
@@ -581,9 +589,12 @@ struct NarrowArgs {
     int S, s0;            /* strips of 128 rows; forward: first strip solved            */
     int trans, epoch;
     const int *info;
+    const double *E;      /* null, or the predecessor products of this direction        *
+                           * (strip_products128), element (r, p) of strip s at          *
+                           * E + s * 16384 + r + p * 128                                 */
 };
 
-template <int NCV, bool FWD>
+template <int NCV, bool FWD, bool PE>
 __global__ __launch_bounds__(512, 1) void strip_narrow_kernel(NarrowArgs a)
 {
     /* backward: one factor block at a time goes through LDS (rows of TLD
@@ -658,6 +669,12 @@ __global__ __launch_bounds__(512, 1) void strip_narrow_kernel(NarrowArgs a)
                 }
             }
         }
+        double ereg[32];
+        if constexpr (PE) {
+            const double *Eg = a.E + (size_t)s * NSR * NSR;
+#pragma unroll
+            for (int i = 0; i < 32; ++i) ereg[i] = Eg[r + (size_t)(32 * kq + i) * NSR];
+        }
         double part[NCV];
 #pragma unroll
         for (int c = 0; c < NCV; ++c) part[c] = 0.0;
@@ -711,7 +728,10 @@ __global__ __launch_bounds__(512, 1) void strip_narrow_kernel(NarrowArgs a)
         /* block j's factor rows are requested before the wait for its
          * solution, so their latency hides behind the wait; one block in
          * flight per workgroup (128 KB) is enough to keep HBM busy */
-        const int nblk = fwd ? s - a.s0 : a.S - 1 - s;
+        /* with E the predecessor is left out here, as in strip_solve_kernel */
+        const int nall = fwd ? s - a.s0 : a.S - 1 - s;
+        const bool use_e = PE && nall > 0;
+        const int nblk = use_e ? nall - 1 : nall;
         int j = fwd ? a.s0 : a.S - 1;
         if constexpr (FWD) {
             for (int b = 0; b < nblk; ++b) {
@@ -784,13 +804,42 @@ __global__ __launch_bounds__(512, 1) void strip_narrow_kernel(NarrowArgs a)
 #pragma unroll
         for (int c = 0; c < NCV; ++c) P[kq][r * NCV + c] = xp[c];
         __syncthreads();
+        double x[NCV];
         if (kq == 0) {
 #pragma unroll
             for (int c = 0; c < NCV; ++c) {
                 const int e = r * NCV + c;
-                const double x = ((P[0][e] + P[1][e]) + P[2][e]) + P[3][e];
-                __hip_atomic_store(&Bs[c + (size_t)r * nrp], x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                x[c] = ((P[0][e] + P[1][e]) + P[2][e]) + P[3][e];
             }
+        }
+        if (use_e) {
+            /* x -= E_s X_pred once the predecessor is published */
+            const double *xb = Xs[nblk & 1];
+            if (wave == 0) fetch(fwd ? s - 1 : s + 1, nblk & 1);
+            __syncthreads();
+#pragma unroll
+            for (int c = 0; c < NCV; ++c) xp[c] = 0.0;
+#pragma unroll
+            for (int i = 0; i < 32; ++i) {
+                const int p = 32 * kq + i;
+#pragma unroll
+                for (int c = 0; c < NCV; ++c) xp[c] = fma(ereg[i], xb[p * NCV + c], xp[c]);
+            }
+#pragma unroll
+            for (int c = 0; c < NCV; ++c) P[kq][r * NCV + c] = xp[c];
+            __syncthreads();
+            if (kq == 0) {
+#pragma unroll
+                for (int c = 0; c < NCV; ++c) {
+                    const int e = r * NCV + c;
+                    x[c] -= ((P[0][e] + P[1][e]) + P[2][e]) + P[3][e];
+                }
+            }
+        }
+        if (kq == 0) {
+#pragma unroll
+            for (int c = 0; c < NCV; ++c)
+                __hip_atomic_store(&Bs[c + (size_t)r * nrp], x[c], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
         /* publication by completion, as in strip_solve_kernel */
         __builtin_amdgcn_s_waitcnt(0x0F70);
@@ -799,7 +848,7 @@ __global__ __launch_bounds__(512, 1) void strip_narrow_kernel(NarrowArgs a)
     }
 }
 
-template <int NCV>
+template <int NCV, bool PE>
 static void narrow_launch(const NarrowArgs &a, hipStream_t s)
 {
     static int per_cu = -1, ncu = 0;
@@ -807,17 +856,24 @@ static void narrow_launch(const NarrowArgs &a, hipStream_t s)
         int dev = 0, pf = 0, pb = 0;
         CHX_HIP(hipGetDevice(&dev));
         CHX_HIP(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev));
-        CHX_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&pf, strip_narrow_kernel<NCV, true>, 512, 0));
-        CHX_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&pb, strip_narrow_kernel<NCV, false>, 512, 0));
+        CHX_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&pf, strip_narrow_kernel<NCV, true, PE>, 512, 0));
+        CHX_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&pb, strip_narrow_kernel<NCV, false, PE>, 512, 0));
         per_cu = pf < pb ? pf : pb;
         if (per_cu < 1) per_cu = 1;
     }
     int grid = ncu * per_cu;
     if (grid > a.S - a.s0) grid = a.S - a.s0;
     if (a.trans)
-        hipLaunchKernelGGL((strip_narrow_kernel<NCV, false>), dim3(grid), dim3(512), 0, s, a);
+        hipLaunchKernelGGL((strip_narrow_kernel<NCV, false, PE>), dim3(grid), dim3(512), 0, s, a);
     else
-        hipLaunchKernelGGL((strip_narrow_kernel<NCV, true>), dim3(grid), dim3(512), 0, s, a);
+        hipLaunchKernelGGL((strip_narrow_kernel<NCV, true, PE>), dim3(grid), dim3(512), 0, s, a);
+}
+
+template <int NCV>
+static void narrow_launch(const NarrowArgs &a, hipStream_t s)
+{
+    if (a.E) narrow_launch<NCV, true>(a, s);
+    else narrow_launch<NCV, false>(a, s);
 }
 
 /* 64 x 64 products of the two kernels below, P = X Y with X(i, k) at X[i*xi + k*xk]
@@ -909,7 +965,24 @@ __global__ __launch_bounds__(256) void dinv128_kernel(const double *A, const dou
     }
 }
 
-bool narrow_eligible(int ldt, int ncols) { return ldt % NSR == 0 && ncols >= 1 && ncols <= 8; }
+/* One or two right-hand sides take the narrow kernel, unless there are so few
+ * strips that forming the 128 x 128 inverses and products costs more than the
+ * shorter chain saves.  dpotrs in us, narrow / 16-column chunks: N = 640, 1
+ * column 219 / 192, 2 columns 215 / 183; N = 2000 265 / 287 and 297 / 299; N =
+ * 4096 359 / 422 and 384 / 425; N = 32768 2288 / 2945 and 2498 / 2997.  With more
+ * columns its products on the vector ALUs and their LDS reads outgrow what an
+ * MFMA spends on unused columns: 3 columns N = 4096 456 / 420, 7 N = 7003 1340 /
+ * 629, 8 N = 32768 6740 / 3025. */
+bool narrow_eligible(int ldt, int NT, int ncols)
+{
+    return ldt % NSR == 0 && ncols >= 1 && ncols <= 2 && NT * ldt >= 1536;
+}
+
+/* The narrow solve takes predecessor products as long as the no-allocation
+ * call's fixed array holds them too (480 doubles a row; it solves with the same
+ * sums); they are
+ * worth less the longer the chain, 2535 and 2288 us at N = 32768, 1 column. */
+bool narrow_products(int ldt, int NT) { return NT * ldt <= 34816; }
 
 void dinv128(const double *A, const double *D, long long dts, long long doff, int ldd, int NT, int ldt,
              double *D128, hipStream_t s)
@@ -971,6 +1044,67 @@ __global__ __launch_bounds__(256) void strip_products_kernel(const double *A, co
     }
 }
 
+/* The same for the 128-row strips, from their inverses D128:
+ *   Ef_s = D_s L(s, s-1),   Eb_s = (L(s+1, s) D_s)^T,
+ * each 128 x 128 at E + s * 16384, element (r, p) at r + p * 128.  One workgroup
+ * per strip and direction, 16 rows per wavefront against all columns, operands
+ * straight from memory (k = 16 kc + 4 lk + q in product q, so that the ones that
+ * run along k are 32-byte loads).  About 10 us at N = 4096 and 60 at 32768. */
+__global__ __launch_bounds__(512) void strip_products128_kernel(const double *A, const double *D128, int NT, int ldt,
+                                                                double *Ef, double *Eb)
+{
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int li = lane & 15, lk = lane >> 4, q = ldt / NSR, S = NT * q;
+    const bool fwd = blockIdx.y == 0;
+    const int s = blockIdx.x, o = fwd ? s - 1 : s + 1;
+    if (o < 0 || o >= S) return;
+    const int m = fwd ? s : o, n = fwd ? o : s;             /* the factor block L(m, n) */
+    const double *L = A + ((size_t)(n / q) * NT + m / q) * ldt * ldt + (m % q) * NSR + (size_t)(n % q) * NSR * ldt;
+    const double *D = D128 + (size_t)s * NSR * NSR;
+    double *O = (fwd ? Ef : Eb) + (size_t)s * NSR * NSR + 16 * wave + li;
+    v4d acc[8];
+#pragma unroll
+    for (int f = 0; f < 8; ++f) acc[f] = zero4d();
+    /* D(r, k) with k <= r forward, D(k, r) with k >= r backward */
+    for (int kc = fwd ? 0 : wave; kc < (fwd ? wave + 1 : 8); ++kc) {
+        const int k = 16 * kc + 4 * lk;
+        double x[4], y[8][4];
+        if (fwd) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) x[e] = D[16 * wave + li + (k + e) * NSR];
+#pragma unroll
+            for (int f = 0; f < 8; ++f) {
+                const v4d v = *(const v4d *)(L + k + (size_t)(16 * f + li) * ldt);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) y[f][e] = v[e];
+            }
+        } else {
+            const v4d v = *(const v4d *)(D + k + (16 * wave + li) * NSR);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) x[e] = v[e];
+#pragma unroll
+            for (int f = 0; f < 8; ++f)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) y[f][e] = L[16 * f + li + (size_t)(k + e) * ldt];
+        }
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+#pragma unroll
+            for (int f = 0; f < 8; ++f) acc[f] = mfma_f64(y[f][e], x[e], acc[f]);
+    }
+#pragma unroll
+    for (int f = 0; f < 8; ++f)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) O[(16 * f + lk + 4 * e) * NSR] = acc[f][e];
+}
+
+void strip_products128(const double *A, const double *D128, int NT, int ldt, double *Ef, double *Eb, hipStream_t s)
+{
+    const int S = NT * ldt / NSR;
+    if (S <= 1) return;
+    hipLaunchKernelGGL(strip_products128_kernel, dim3(S, 2), dim3(512), 0, s, A, D128, NT, ldt, Ef, Eb);
+}
+
 void strip_products(const double *A, const double *D, long long dts, long long doff, int ldd, int NT, int ldt,
                     double *Ef, double *Eb, hipStream_t s)
 {
@@ -983,7 +1117,7 @@ int solve_strips(const double *A, const double *D, long long dts, long long doff
                  int ldt, int nrp, int trans, int *flags, int epoch, unsigned *ticket, const int *info, hipStream_t s,
                  int s0, const double *D128, int ncols, const double *E)
 {
-    if (D128 && narrow_eligible(ldt, ncols)) {
+    if (D128 && narrow_eligible(ldt, NT, ncols)) {
         NarrowArgs na;
         na.A = A; na.D128 = D128; na.BT = BT; na.flags = flags; na.ticket = ticket;
         na.NT = NT; na.ldt = ldt; na.nrp = nrp;
@@ -993,10 +1127,9 @@ int solve_strips(const double *A, const double *D, long long dts, long long doff
         na.trans = trans;
         na.epoch = epoch;
         na.info = info;
+        na.E = E;
         if (ncols == 1) narrow_launch<1>(na, s);
-        else if (ncols == 2) narrow_launch<2>(na, s);
-        else if (ncols <= 4) narrow_launch<4>(na, s);
-        else narrow_launch<8>(na, s);
+        else narrow_launch<2>(na, s);
         return 1;
     }
     StripArgs a;

@@ -214,9 +214,9 @@ int mixed_posv(cham_uplo_t uplo, CHAM_desc_t *A, CHAM_desc_t *B, CHAM_desc_t *X,
         const int npanel = adaptive ? 8 : 4;
         const size_t mapbytes = adaptive ? (((size_t)NT * NT + 255) & ~(size_t)255) : 0;
         /* at the end, for the first solve (beside the factorisation): with
-         * few right-hand sides the 128 x 128 strip inverses, else the
-         * predecessor products of the MFMA strip solve */
-        const size_t n128 = k::narrow_eligible(ldt, X->n) ? (size_t)NT * ldt * 128 : 2 * (size_t)NT * ldt * 64;
+         * few right-hand sides the 128 x 128 strip inverses and their
+         * predecessor products, else those of the MFMA strip solve */
+        const size_t n128 = k::narrow_eligible(ldt, NT, X->n) ? 3 * (size_t)NT * ldt * 128 : 2 * (size_t)NT * ldt * 64;
         char *w = (char *)workspace2(abytes + npanel * pbytes + mapbytes +
                                      (3 * vb + 2 * (size_t)nrp + pv + rows + (size_t)NT * NT + n128) * sizeof(double));
         double *Aw = (double *)w;
@@ -256,7 +256,7 @@ int mixed_posv(cham_uplo_t uplo, CHAM_desc_t *A, CHAM_desc_t *B, CHAM_desc_t *X,
         p.nvalid_last = N - (NT - 1) * A->mb;
         p.d_info = st->d_info;
         p.lp_mode = prec;
-        if (k::narrow_eligible(ldt, X->n))
+        if (k::narrow_eligible(ldt, NT, X->n))
             p.d128 = tss + (size_t)NT * NT;
         else
             p.epred = tss + (size_t)NT * NT;     /* predecessor products of the first solve */

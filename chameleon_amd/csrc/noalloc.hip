@@ -3,10 +3,10 @@
  *
  * CHAMAMD_dpotrs_Tile_Async_NoAlloc runs the same kernels, in the same
  * order, as CHAMELEON_dpotrs_Tile_Async with tiles a multiple of 64 (the
- * 64 x 64 diagonal-block inverses, then with at most 8 right-hand sides and
- * tiles a multiple of 128 the 128 x 128 strip inverses, else the strip
- * solve's predecessor products, the transposition of B, one strip-solve
- * launch per direction, the transposition back), but takes every buffer
+ * 64 x 64 diagonal-block inverses, then with one or two right-hand sides and
+ * tiles a multiple of 128 the 128 x 128 strip inverses, the strip solve's
+ * predecessor products, the transposition of B, one strip-solve launch per
+ * direction, the transposition back), but takes every buffer
  * beyond A and B from `scratch`, a device array of fixed size that the
  * code object carries, instead of the library's growable workspaces.  It
  * is for callers that cannot call hipMalloc: code under stream capture,
@@ -17,14 +17,15 @@
  *                                 tagged by launch epoch (never cleared
  *                                 between calls; cleared once at set-up,
  *                                 CHAMELEON_Init), and in its last int the
- *                                 launches' task ticket (cleared before
- *                                 each launch)
+ *                                 launches' task ticket (zero between
+ *                                 launches)
  *   [NOALLOC_FLAG_BYTES, ...)     doubles: the 64 x 64 inverses
  *                                 (Npad * 64), the 128 x 128 strip
- *                                 inverses of a narrow solve or the two
- *                                 directions' predecessor products
- *                                 (Npad * 128), then the transposed
- *                                 right-hand sides (nrp * Npad)
+ *                                 inverses of a narrow solve (Npad * 128)
+ *                                 and its two directions' predecessor
+ *                                 products (Npad * 256) or those of the
+ *                                 MFMA solve (Npad * 128), then the
+ *                                 transposed right-hand sides (nrp * Npad)
  * with Npad = NT * ldt (padded rows) and nrp = B's padded column count.
  * Calls are rejected (CHAMELEON_ERR_OUT_OF_RESOURCES) when that exceeds
  * NOALLOC_MAX_DOUBLES (128 MiB of doubles), e.g. N = 32768 is served with
@@ -137,10 +138,11 @@ extern "C" int CHAMAMD_dpotrs_Tile_Async_NoAlloc(cham_uplo_t uplo, CHAM_desc_t *
     const int NT = MA->mt, ldt = MA->ldt;
     const size_t npad = (size_t)NT * ldt;
     const int nrp = MB->nt * MB->wdt;
-    const bool narrow = k::narrow_eligible(ldt, B->n);
-    /* the narrow solve's strip inverses or the MFMA solve's predecessor
-     * products: Npad * 128 doubles either way */
-    const size_t ndinv = npad * 64, naux = npad * 128, nbt = (size_t)nrp * npad;
+    const bool narrow = k::narrow_eligible(ldt, NT, B->n), products = narrow && k::narrow_products(ldt, NT);
+    /* the narrow solve's strip inverses (Npad * 128 doubles, and twice that for
+     * their predecessor products, which narrow_products limits to what fits) or
+     * the MFMA solve's predecessor products (Npad * 128) */
+    const size_t ndinv = npad * 64, naux = npad * (products ? 384 : 128), nbt = (size_t)nrp * npad;
     const int S = (int)(npad / 64);
     if (ndinv + naux + nbt > NOALLOC_MAX_DOUBLES || (size_t)(4 * S + 1) * sizeof(int) > NOALLOC_FLAG_BYTES) {
         error(fn, "problem larger than the fixed scratch array (N_padded * (192 + NRHS_padded) <= 16777216)");
@@ -172,7 +174,7 @@ extern "C" int CHAMAMD_dpotrs_Tile_Async_NoAlloc(cham_uplo_t uplo, CHAM_desc_t *
     double *dinv = (double *)(d->ptr + NOALLOC_FLAG_BYTES);
     double *aux = dinv + ndinv;
     double *d128 = narrow ? aux : nullptr;
-    double *ef = narrow ? nullptr : aux, *eb = narrow ? nullptr : aux + npad * 64;
+    double *ef = !narrow ? aux : products ? aux + npad * 128 : nullptr, *eb = ef ? ef + npad * (narrow ? 128 : 64) : nullptr;
     double *BT = dinv + ndinv + naux;
     SeqState *st = seq_state(sequence);
 
@@ -197,9 +199,10 @@ extern "C" int CHAMAMD_dpotrs_Tile_Async_NoAlloc(cham_uplo_t uplo, CHAM_desc_t *
     const double *Ad = (const double *)MA->d;
     const size_t ts = (size_t)ldt * ldt, dper = (size_t)(ldt / 64) * 64 * 64;
     k::dinv_all(Ad, NT, (size_t)(NT + 1) * ts, ldt, dinv, s);
-    if (narrow)
+    if (narrow) {
         k::dinv128(Ad, dinv, (long long)dper, 64LL * 64, 64, NT, ldt, d128, s);
-    else
+        if (ef) k::strip_products128(Ad, d128, NT, ldt, ef, eb, s);
+    } else
         k::strip_products(Ad, dinv, (long long)dper, 64LL * 64, 64, NT, ldt, ef, eb, s);
     k::rhs_transpose((double *)MB->d, BT, NT, ldt, MB->ldt, MB->wdt, MB->nt, 1, s);
     for (int dir = 0; dir < 2; ++dir)

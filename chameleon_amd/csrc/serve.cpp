@@ -544,7 +544,7 @@ void launch_large_solve(Server *s, Slot &sl, Job *job)
     /* few right-hand sides: the narrow strip solve, with the 128 x 128
      * strip inverses formed here from the factor's 64 x 64 ones; else the
      * MFMA strip solve with its predecessor products, formed here too */
-    const bool narrow = k::narrow_eligible(f->ldt, q->r.nrhs);
+    const bool narrow = k::narrow_eligible(f->ldt, f->NT, q->r.nrhs);
     Layout d;
     const size_t o_bt = d.add(vb * 8), o_aux = d.add((size_t)rows * 128 * 8);
     char *dv = slot_dev(sl, d.used);
@@ -614,7 +614,7 @@ void launch_mixed_solve(Server *s, Slot &sl, Job *job)
     job->rows = f->NT * f->ldt;
     const size_t vb = (size_t)job->nrp * job->rows;
     Layout d;
-    const bool narrow = k::narrow_eligible(f->ldt, q->r.nrhs);
+    const bool narrow = k::narrow_eligible(f->ldt, f->NT, q->r.nrhs);
     const size_t o_bt = d.add(vb * 8), o_xt = d.add(vb * 8), o_rt = d.add(vb * 8),
                  o_part = d.add(k::residual_scratch(f->NT, f->ldt, job->nrp) * 8), o_nw = d.add(2 * job->nrp * 8),
                  o_aux = d.add((size_t)job->rows * 128 * 8);

@@ -78,3 +78,23 @@ def test_solve_after_a_failed_factorisation(ch, k):
                 if info == 0:
                     check(A, dB.to_array(n, k), B)
             seq.destroy()
+
+
+@pytest.mark.parametrize("n,nb,k", [(1408, 128, 1), (1500, 128, 2), (1537, 128, 1), (2000, 384, 2), (4100, 256, 1),
+                                    (4100, 256, 2), (4100, 256, 3), (9000, 512, 1)])
+@pytest.mark.parametrize("uplo", [LOWER, UPPER])
+def test_few_columns(ch, n, nb, k, uplo):
+    """One to three columns about the lines between the narrow solve with its
+    predecessor products and the 16-column chunks."""
+    print("[case] few columns", n, nb, k, uplo, flush=True)
+    A = matrix(n, n)
+    B = np.asfortranarray(np.random.default_rng(k).standard_normal((n, k)))
+    seq = ch.Sequence()
+    with ch.Desc.from_array(A.copy(order="F"), nb) as dA, ch.Desc.from_array(B.copy(order="F"), nb) as dB, \
+            ch.Desc.from_array(B.copy(order="F"), nb) as dX:
+        ch.check(ch.lib.CHAMELEON_dposv_Tile_Async(uplo, dA.ptr, dB.ptr, seq.ptr, seq.req))
+        ch.check(ch.lib.CHAMELEON_dpotrs_Tile_Async(uplo, dA.ptr, dX.ptr, seq.ptr, seq.req))
+        assert seq.wait() == 0
+        check(A, dB.to_array(n, k), B)
+        check(A, dX.to_array(n, k), B)
+    seq.destroy()
