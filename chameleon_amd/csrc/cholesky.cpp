@@ -474,7 +474,7 @@ bool potrf_solve_eligible(int ldt)
     return c->panel && c->lookahead > 0 && ldt % 64 == 0;
 }
 
-void potrf_solve_run(PotrfPlan p, double *BT, int nrp, int nrhs, double rate)
+SolvePlan potrf_solve_run(PotrfPlan p, double *BT, int nrp, int nrhs, double rate)
 {
     Context *c = ctx();
     Lane *L = p.lane ? p.lane : main_lane();
@@ -519,6 +519,14 @@ void potrf_solve_run(PotrfPlan p, double *BT, int nrp, int nrhs, double rate)
         k::solve_strips(f.A, f.dinv, (long long)f.dper, 64LL * 64, 64, f.BT, NT, ldt, nrp, 1, flags,
                         epoch + chunks, lane_counters(L) + 2, p.d_info, sm, 0, d128, nrhs, eb);
     });
+    SolvePlan sp = {};
+    sp.dinv = f.dinv;
+    sp.d128 = narrow ? p.d128 : nullptr;
+    sp.ef = ef;
+    sp.eb = eb;
+    sp.ncols = nrhs;
+    sp.R = 64;
+    return sp;
 }
 
 int posv_async(cham_uplo_t uplo, CHAM_desc_t *A, CHAM_desc_t *B, RUNTIME_sequence_t *sequence)

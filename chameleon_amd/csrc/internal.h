@@ -252,14 +252,7 @@ void potrf_run(const PotrfPlan &p);
 void solve_strips_lane(Lane *L, const double *A, const double *dinv, int NT, int ldt, double *BT, int nrp,
                        const int *d_info, const double *d128 = nullptr, int ncols = 0, const double *ef = nullptr,
                        const double *eb = nullptr);
-/* potrf_run with the forward solve of BT (transposed right-hand sides,
- * nrp x NT*ldt, nrhs of them in use) issued beside the factorisation, then
- * the forward strips it left and the backward solve: BT <- A^-1 BT.  The
- * solve kernels return at once when the device info flag is set.  `rate`:
- * the bulk update rate (flop/s) the overlap is sized for.  Requires
- * potrf_solve_eligible(ldt). */
-bool potrf_solve_eligible(int ldt);
-void potrf_solve_run(PotrfPlan p, double *BT, int nrp, int nrhs, double rate);
+/* strip (or tile-step) solves with a factor: what they read beside it */
 struct SolvePlan {
     double *TT, *TN, *BT, *W, *dinv;   /* diagonal-tile inverses, transposed RHS, one block, 64x64 inverses */
     double *d128 = nullptr;            /* 128 x 128 strip inverses (narrow solves), or null */
@@ -267,6 +260,15 @@ struct SolvePlan {
     int ncols = 0;                     /* right-hand-side columns in use */
     int R = 0;                         /* 64: strip solve; 0: tile-step solve */
 };
+/* potrf_run with the forward solve of BT (transposed right-hand sides,
+ * nrp x NT*ldt, nrhs of them in use) issued beside the factorisation, then
+ * the forward strips it left and the backward solve: BT <- A^-1 BT.  The
+ * solve kernels return at once when the device info flag is set.  `rate`:
+ * the bulk update rate (flop/s) the overlap is sized for.  Requires
+ * potrf_solve_eligible(ldt).  Returns the plan of further solves with the
+ * factor (dinv, d128 and the products stay in the caller's room). */
+bool potrf_solve_eligible(int ldt);
+SolvePlan potrf_solve_run(PotrfPlan p, double *BT, int nrp, int nrhs, double rate);
 /* ncols: columns of the right-hand sides in use (at most nrp); with few of
  * them the plan also holds the 128 x 128 strip inverses */
 SolvePlan solve_plan(double *A, int NT, int ldt, int nrp, int *d_info, int ncols = 0);
@@ -371,21 +373,21 @@ void panel_demote(const double *A, int NT, int ldt, int k, int m0, int m1, void 
  * per tile; a tile with a non-finite entry sets *info = LP_RANGE */
 void panel_demote_fp8(const double *A, int NT, int ldt, int k, int m0, int m1, void *P, int *info, hipStream_t s);
 /* symmetric diagonal scaling: sc[i] = a_ii^-1/2 over the NT*ldt padded rows,
- * lower tiles of A scaled by sc_i sc_j; scale_bt: rows of transposed
- * right-hand sides (element (c, r) at c + r*nrp) times sc[r] */
+ * lower tiles of A scaled by sc_i sc_j; scale_bt: BT = rows of the transposed
+ * right-hand sides src (element (c, r) at c + r*nrp) times sc[r] */
 void diag_scaling(double *A, int NT, int ldt, double *sc, hipStream_t s);
 void diag_rsqrt(const double *A, int NT, int ldt, double *sc, hipStream_t s);   /* sc only */
-void scale_bt(double *BT, int nrp, int rows, const double *sc, hipStream_t s);
+void scale_bt(double *BT, const double *src, int nrp, int rows, const double *sc, hipStream_t s);
 void trailing_update_lp(double *A, const void *P, const void *P2, int mode, int lmt, int ldt, int n0, int n1, int NT,
                         const int *info, hipStream_t s, const unsigned char *pmap = nullptr);
 void tile_sumsq_lower(const double *A, int NT, int ldt, double *ss, hipStream_t s);
+/* R = B - A X in RT (with sc: row r times sc[r]), and the column maxima of |X|
+ * in out[0..nrp) and of |R| (unscaled) in out[nrp..2 nrp) */
 void residual(const double *A, int NT, int ldt, const double *XT, const double *BT, double *RT, int nrp, double *part,
-              hipStream_t s);
+              double *out, const double *sc, hipStream_t s);
 size_t residual_scratch(int NT, int ldt, int nrp);   /* doubles of `part` */
-/* column maxima of X into out[0..ncols) and of R into out[nrp..nrp+ncols)
- * (max-combined into out: clear it first) */
-void colmax2(const double *X, const double *R, int nrp, int ncols, int nrows, double *out, hipStream_t s);
-void axpy(double *Y, const double *X, size_t n, hipStream_t s);
+/* X += D, with sc row r of D times sc[r] */
+void correct(double *XT, const double *DT, int nrp, int rows, const double *sc, hipStream_t s);
 /* lower tiles of S copied to W (with sc: scaled by sc_i sc_j as
  * diag_scaling does, in the same pass) and the symmetric inf-norm's row
  * sums of S into rowsum[N]; returns -1 (nothing launched) unless ldt is a

@@ -570,11 +570,11 @@ __global__ void scale_lower_kernel(double *A, int NT, int ldt, const double *sc)
     }
 }
 
-__global__ void scale_bt_kernel(double *BT, int nrp, int rows, const double *sc)
+__global__ void scale_bt_kernel(double *BT, const double *src, int nrp, int rows, const double *sc)
 {
     const size_t total = (size_t)nrp * rows;
     for (size_t e = (size_t)blockIdx.x * blockDim.x + threadIdx.x; e < total; e += (size_t)gridDim.x * blockDim.x)
-        BT[e] *= sc[e / nrp];
+        BT[e] = src[e] * sc[e / nrp];
 }
 
 void diag_rsqrt(const double *A, int NT, int ldt, double *sc, hipStream_t s)
@@ -589,12 +589,12 @@ void diag_scaling(double *A, int NT, int ldt, double *sc, hipStream_t s)
                        0, s, A, NT, ldt, sc);
 }
 
-void scale_bt(double *BT, int nrp, int rows, const double *sc, hipStream_t s)
+void scale_bt(double *BT, const double *src, int nrp, int rows, const double *sc, hipStream_t s)
 {
     const size_t total = (size_t)nrp * rows;
     if (!total) return;
     hipLaunchKernelGGL(scale_bt_kernel, dim3((unsigned)std::min<size_t>((total + 255) / 256, 8192)), dim3(256), 0, s,
-                       BT, nrp, rows, sc);
+                       BT, src, nrp, rows, sc);
 }
 
 /* ------------------------------------------------------------------ */
@@ -684,7 +684,7 @@ void trailing_update_lp(double *A, const void *P, const void *P2, int mode, int 
  * tile mirror A (NT x NT tiles of ldt x ldt), right-hand sides transposed
  * (element (j, p) at j + p*nrp).
  *
- * The row range of A is cut in RES_KS pieces: wavefront (rb, jc, ks)
+ * The row range of A is cut in KS pieces: wavefront (rb, jc, ks)
  * forms the (16 RG) x 64 block (rows 16 RG rb.., columns 64 jc..) of
  * A(:, piece ks) X(piece ks, :) into its own partial buffer, and a second
  * kernel adds the pieces in a fixed order (deterministic).  With RG = 2 a
@@ -698,11 +698,14 @@ void trailing_update_lp(double *A, const void *P, const void *P2, int mode, int 
  * column count is a constant, so the loop body has no branches: with
  * run-time tests around each load and product the compiler split it into
  * dozens of basic blocks. */
-#define RES_KS 8
-template <int RG, bool FULL>
-__global__ __launch_bounds__(256, 2) void residual_kernel(const double *A, int NT, int ldt, const double *XT, int nrp,
-                                                        double *part)
+template <int RG, int NF, bool FULL>
+__global__ __launch_bounds__(256, NF == 1 ? 4 : 2) void residual_kernel(const double *A, int NT, int ldt,
+                                                                        const double *XT, int nrp, int KS, double *part,
+                                                                        double *out)
 {
+    /* the maxima that residual_finish_kernel combines start from 0 */
+    if (blockIdx.x == 0)
+        for (int j = threadIdx.x; j < 2 * nrp; j += 256) out[j] = 0.0;
     const int lane = threadIdx.x & 63, li = lane & 15, lk = lane >> 4;
     const int rows = NT * ldt;
     const int jchunks = (nrp + 63) / 64;
@@ -710,26 +713,26 @@ __global__ __launch_bounds__(256, 2) void residual_kernel(const double *A, int N
     /* the four waves of a workgroup take four consecutive row blocks of
      * one k range, so they read the same X chunks at the same time */
     const int groups = (nrb + 3) / 4;
-    const int ks = blockIdx.x % RES_KS, rest = blockIdx.x / RES_KS;
+    const int ks = blockIdx.x % KS, rest = blockIdx.x / KS;
     const int rb = (rest % groups) * 4 + (threadIdx.x >> 6), jc = rest / groups;
     if (jc >= jchunks || rb >= nrb) return;     /* no barriers below: waves are independent */
     const int r0 = rb * 16 * RG;
     const int m = r0 / ldt, i0 = r0 % ldt;
     const int j0 = jc * 64;
-    const int nf = FULL ? 4 : min(4, (nrp - j0) / 16);
+    const int nf = NF < 4 || FULL ? NF : min(4, (nrp - j0) / 16);
     const size_t ts = (size_t)ldt * ldt;
     /* this wave's k range: [kb, ke) in units of 16 */
     const int nk16 = rows / 16;
-    const int kb = (int)((long long)nk16 * ks / RES_KS) * 16, ke = (int)((long long)nk16 * (ks + 1) / RES_KS) * 16;
-    v4d acc[RG][4];
+    const int kb = (int)((long long)nk16 * ks / KS) * 16, ke = (int)((long long)nk16 * (ks + 1) / KS) * 16;
+    v4d acc[RG][NF];
 #pragma unroll
     for (int g = 0; g < RG; ++g)
 #pragma unroll
-        for (int f = 0; f < 4; ++f) acc[g][f] = zero4d();
+        for (int f = 0; f < NF; ++f) acc[g][f] = zero4d();
     /* x operands of chunk p0: X(p0 + 4 lk + q, col(f, li)), where product f
      * covers columns j0 + 16 f + li, or with FULL columns j0 + 4 li + f (a
      * lane's four columns adjacent: one 32-byte load per k) */
-    auto load_x = [&](int p0, double (&x)[4][4]) {
+    auto load_x = [&](int p0, double (&x)[4][NF]) {
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
             if constexpr (FULL) {
@@ -739,17 +742,17 @@ __global__ __launch_bounds__(256, 2) void residual_kernel(const double *A, int N
             } else {
                 const double *xr = XT + (size_t)(p0 + 4 * lk + q) * nrp + j0 + li;
 #pragma unroll
-                for (int f = 0; f < 4; ++f) x[q][f] = (f < nf) ? xr[16 * f] : 0.0;
+                for (int f = 0; f < NF; ++f) x[q][f] = (f < nf) ? xr[16 * f] : 0.0;
             }
         }
     };
-    auto mma = [&](const double (&a)[RG][4], const double (&x)[4][4]) {
+    auto mma = [&](const double (&a)[RG][4], const double (&x)[4][NF]) {
 #pragma unroll
         for (int q = 0; q < 4; ++q)
 #pragma unroll
             for (int g = 0; g < RG; ++g)
 #pragma unroll
-                for (int f = 0; f < 4; ++f)
+                for (int f = 0; f < NF; ++f)
                     if (f < nf) acc[g][f] = mfma_f64(a[g][q], x[q][f], acc[g][f]);
     };
     /* the k range, tile by tile: three loop shapes, each software-pipelined */
@@ -758,7 +761,7 @@ __global__ __launch_bounds__(256, 2) void residual_kernel(const double *A, int N
         if (nt < m) {
             /* stored tile (m, nt): element (i0 + 16 g + li, p) at T[16 g + p*ldt] */
             const double *T = A + ((size_t)nt * NT + m) * ts + i0 + li;
-            double a[RG][4], x[4][4], an[RG][4], xn[4][4];
+            double a[RG][4], x[4][NF], an[RG][4], xn[4][NF];
 #pragma unroll
             for (int g = 0; g < RG; ++g)
 #pragma unroll
@@ -776,7 +779,7 @@ __global__ __launch_bounds__(256, 2) void residual_kernel(const double *A, int N
 #pragma unroll
                     for (int g = 0; g < RG; ++g) a[g][q] = an[g][q];
 #pragma unroll
-                    for (int f = 0; f < 4; ++f) x[q][f] = xn[q][f];
+                    for (int f = 0; f < NF; ++f) x[q][f] = xn[q][f];
                 }
             }
             mma(a, x);
@@ -784,7 +787,7 @@ __global__ __launch_bounds__(256, 2) void residual_kernel(const double *A, int N
             /* transpose of stored tile (nt, m): element (i0 + 16 g + li, p) at
              * T[p + 16 g ldt] */
             const double *T = A + ((size_t)m * NT + nt) * ts + (size_t)(i0 + li) * ldt;
-            double a[RG][4], x[4][4], an[RG][4], xn[4][4];
+            double a[RG][4], x[4][NF], an[RG][4], xn[4][NF];
 #pragma unroll
             for (int g = 0; g < RG; ++g) {
                 const v4d v = *(const v4d *)(T + (size_t)16 * g * ldt + pb + 4 * lk);
@@ -806,7 +809,7 @@ __global__ __launch_bounds__(256, 2) void residual_kernel(const double *A, int N
 #pragma unroll
                     for (int g = 0; g < RG; ++g) a[g][q] = an[g][q];
 #pragma unroll
-                    for (int f = 0; f < 4; ++f) x[q][f] = xn[q][f];
+                    for (int f = 0; f < NF; ++f) x[q][f] = xn[q][f];
                 }
             }
             mma(a, x);
@@ -814,7 +817,7 @@ __global__ __launch_bounds__(256, 2) void residual_kernel(const double *A, int N
             /* diagonal tile, lower triangle stored */
             const double *T = A + ((size_t)m * NT + m) * ts;
             for (int p = pb; p < pe; p += 16) {
-                double a[RG][4], x[4][4];
+                double a[RG][4], x[4][NF];
 #pragma unroll
                 for (int g = 0; g < RG; ++g) {
                     const int ii = i0 + 16 * g + li;
@@ -840,7 +843,7 @@ __global__ __launch_bounds__(256, 2) void residual_kernel(const double *A, int N
                     v4d{acc[g][0][s], acc[g][1][s], acc[g][2][s], acc[g][3][s]};
         } else {
 #pragma unroll
-            for (int f = 0; f < 4; ++f)
+            for (int f = 0; f < NF; ++f)
                 if (f < nf) {
 #pragma unroll
                     for (int s = 0; s < 4; ++s)
@@ -850,77 +853,109 @@ __global__ __launch_bounds__(256, 2) void residual_kernel(const double *A, int N
     }
 }
 
-__global__ void residual_sum_kernel(const double *BT, const double *part, double *RT, size_t n)
+/* The end of a residual in one launch: R = B - (the KS pieces, added in a
+ * fixed order), stored in RT (times sc[r] in row r with sc: the right-hand
+ * side of a solve with the scaled factor), and the column maxima
+ * max_r |X(r, j)| into out[j] and max_r |R(r, j)| into out[nrp + j]
+ * (residual_kernel has cleared out).  Thread (g, c) takes column
+ * 64 blockIdx.y + c, c < cw = min(64, nrp), rows g, g + G, ... of this
+ * block's share: a wave's loads are adjacent.  The G row lanes meet in LDS, one
+ * atomic max per column and array per workgroup (on the bit pattern:
+ * order-free and NaN-propagating for these non-negative values). */
+__global__ __launch_bounds__(256) void residual_finish_kernel(const double *BT, const double *part, int KS, double *RT,
+                                                              const double *XT, const double *sc, int nrp, int rows,
+                                                              double *out)
 {
-    for (size_t e = (size_t)blockIdx.x * blockDim.x + threadIdx.x; e < n; e += (size_t)gridDim.x * blockDim.x) {
-        double s = 0.0;
-#pragma unroll
-        for (int k = 0; k < RES_KS; ++k) s += part[(size_t)k * n + e];
-        RT[e] = BT[e] - s;
-    }
-}
-
-size_t residual_scratch(int NT, int ldt, int nrp) { return (size_t)RES_KS * NT * ldt * nrp; }
-
-void residual(const double *A, int NT, int ldt, const double *XT, const double *BT, double *RT, int nrp, double *part,
-              hipStream_t s)
-{
-    /* two 16-row groups per wave when both lie in one tile row */
-    const int rg = (ldt % 32 == 0) ? 2 : 1;
-    const bool full = nrp % 64 == 0;
-    const long long blocks = (long long)((NT * ldt / (16 * rg) + 3) / 4) * ((nrp + 63) / 64) * RES_KS;
-    auto kern = rg == 2 ? (full ? residual_kernel<2, true> : residual_kernel<2, false>)
-                        : (full ? residual_kernel<1, true> : residual_kernel<1, false>);
-    hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(256), 0, s, A, NT, ldt, XT, nrp, part);
-    const size_t n = (size_t)NT * ldt * nrp;
-    hipLaunchKernelGGL(residual_sum_kernel, dim3(2048), dim3(256), 0, s, BT, part, RT, n);
-}
-
-/* the column maxima max_p |V(j, p)| (V transposed: element (j, p) at
- * j + p*nrp) of X into out[j] and of R into out[nrp + j], in one launch;
- * out cleared by the caller.  Lane c of wave g: column 64 blockIdx.y + c,
- * rows g, g + 4, ... of this block's share: a wave reads 64 adjacent
- * columns of a row (coalesced; one column per workgroup had each lane
- * touch its own 512-byte line), the four waves meet in LDS, one atomic max
- * per column and array per workgroup (on the bit pattern: order-free and
- * NaN-propagating for these non-negative values) */
-__global__ void colmax2_kernel(const double *X, const double *R, int nrp, int ncols, int nrows, double *out)
-{
-    __shared__ double sx[4][64], sr[4][64];
-    const int c = threadIdx.x & 63, g = threadIdx.x >> 6;
+    __shared__ double sx[256], sr[256];
+    const int cw = min(64, nrp), G = 256 / cw;
+    const int c = threadIdx.x % cw, g = threadIdx.x / cw;
     const int j = blockIdx.y * 64 + c;
+    const size_t n = (size_t)rows * nrp;
     double mx = 0.0, mr = 0.0;
-    if (j < ncols) {
-        for (int p = blockIdx.x * 4 + g; p < nrows; p += gridDim.x * 4) {
-            mx = nan_max(mx, fabs(X[j + (size_t)p * nrp]));
-            mr = nan_max(mr, fabs(R[j + (size_t)p * nrp]));
+    if (g < G && j < nrp) {
+        for (int r = blockIdx.x * G + g; r < rows; r += gridDim.x * G) {
+            const size_t e = (size_t)r * nrp + j;
+            double s = 0.0;
+            for (int k = 0; k < KS; k += 8) {
+#pragma unroll
+                for (int u = 0; u < 8; ++u) s += part[(size_t)(k + u) * n + e];
+            }
+            const double v = BT[e] - s;
+            RT[e] = sc ? v * sc[r] : v;
+            mx = nan_max(mx, fabs(XT[e]));
+            mr = nan_max(mr, fabs(v));
         }
     }
-    sx[g][c] = mx;
-    sr[g][c] = mr;
+    sx[threadIdx.x] = mx;
+    sr[threadIdx.x] = mr;
     __syncthreads();
-    if (g == 0 && j < ncols) {
-        mx = nan_max(nan_max(sx[0][c], sx[1][c]), nan_max(sx[2][c], sx[3][c]));
-        mr = nan_max(nan_max(sr[0][c], sr[1][c]), nan_max(sr[2][c], sr[3][c]));
+    if (g == 0 && j < nrp) {
+        for (int q = 1; q < G; ++q) {
+            mx = nan_max(mx, sx[q * cw + c]);
+            mr = nan_max(mr, sr[q * cw + c]);
+        }
         atomicMax(reinterpret_cast<unsigned long long *>(&out[j]), (unsigned long long)__double_as_longlong(mx));
         atomicMax(reinterpret_cast<unsigned long long *>(&out[nrp + j]), (unsigned long long)__double_as_longlong(mr));
     }
 }
 
-void colmax2(const double *X, const double *R, int nrp, int ncols, int nrows, double *out, hipStream_t s)
+/* workgroups of one piece */
+static int residual_groups(int NT, int ldt, int nrp)
 {
-    hipLaunchKernelGGL(colmax2_kernel, dim3(128, (ncols + 63) / 64), dim3(256), 0, s, X, R, nrp, ncols, nrows, out);
+    const int rg = (ldt % 32 == 0) ? 2 : 1;     /* two 16-row groups per wave when both lie in one tile row */
+    return (NT * ldt / (16 * rg) + 3) / 4 * ((nrp + 63) / 64);
 }
 
-__global__ void axpy_kernel(double *Y, const double *X, size_t n)
+/* Pieces of the row range: eight, more where those leave fewer than two
+ * workgroups to each of 256 compute units (and 64 rows or more to a piece).  A
+ * wave's chunks wait for memory one after the other, so a small system is
+ * bound by their number: one right-hand side, 8 / 16 / 32 pieces, N = 1100
+ * 10.3 / 7.8 us (18 pieces' worth of rows), 2500 20.2 / 18.6 / 14.6, 4096 28.4 /
+ * 26 / 26; at N = 8000 8 and 16 take 92 and 90 and the longer sum of the pieces
+ * (19 to 23 us) loses it again.  With nrp = 16 a wave holds the one column
+ * group it has (NF = 1: twice the wavefronts in flight; 41 us at N = 4096
+ * with the four-group kernel). */
+static int residual_pieces(int NT, int ldt, int nrp)
 {
-    for (size_t e = (size_t)blockIdx.x * blockDim.x + threadIdx.x; e < n; e += (size_t)gridDim.x * blockDim.x)
-        Y[e] += X[e];
+    const long long g = residual_groups(NT, ldt, nrp);
+    int ks = 8;
+    while (ks < 32 && g * ks < 512 && NT * ldt / (2 * ks) >= 64) ks *= 2;
+    return ks;
 }
 
-void axpy(double *Y, const double *X, size_t n, hipStream_t s)
+size_t residual_scratch(int NT, int ldt, int nrp)
 {
-    hipLaunchKernelGGL(axpy_kernel, dim3(2048), dim3(256), 0, s, Y, X, n);
+    return (size_t)residual_pieces(NT, ldt, nrp) * NT * ldt * nrp;
+}
+
+void residual(const double *A, int NT, int ldt, const double *XT, const double *BT, double *RT, int nrp, double *part,
+              double *out, const double *sc, hipStream_t s)
+{
+    const int rows = NT * ldt, ks = residual_pieces(NT, ldt, nrp);
+    auto *one = ldt % 32 == 0 ? residual_kernel<2, 1, false> : residual_kernel<1, 1, false>;
+    auto *full = ldt % 32 == 0 ? residual_kernel<2, 4, true> : residual_kernel<1, 4, true>;
+    auto *any = ldt % 32 == 0 ? residual_kernel<2, 4, false> : residual_kernel<1, 4, false>;
+    hipLaunchKernelGGL((nrp == 16 ? one : nrp % 64 == 0 ? full : any), dim3((unsigned)(residual_groups(NT, ldt, nrp) * ks)),
+                       dim3(256), 0, s, A, NT, ldt, XT, nrp, ks, part, out);
+    const int G = 256 / std::min(64, nrp);
+    hipLaunchKernelGGL(residual_finish_kernel, dim3(std::min(512, (rows + G - 1) / G), (nrp + 63) / 64), dim3(256), 0, s, BT,
+                       part, ks, RT, XT, sc, nrp, rows, out);
+}
+
+/* X += D, row r of D times sc[r] (with sc) */
+__global__ void correct_kernel(double *XT, const double *DT, int nrp, int rows, const double *sc)
+{
+    const size_t total = (size_t)nrp * rows;
+    for (size_t e = (size_t)blockIdx.x * blockDim.x + threadIdx.x; e < total; e += (size_t)gridDim.x * blockDim.x)
+        XT[e] += sc ? DT[e] * sc[e / nrp] : DT[e];
+}
+
+void correct(double *XT, const double *DT, int nrp, int rows, const double *sc, hipStream_t s)
+{
+    const size_t total = (size_t)nrp * rows;
+    if (!total) return;
+    hipLaunchKernelGGL(correct_kernel, dim3((unsigned)std::min<size_t>((total + 255) / 256, 8192)), dim3(256), 0, s, XT,
+                       DT, nrp, rows, sc);
 }
 
 /* ------------------------------------------------------------------ */
@@ -930,19 +965,21 @@ void axpy(double *Y, const double *X, size_t n, hipStream_t s)
  * tile (m, n) at (n NT + m) ldt^2; only tiles m >= n are read and written.
  * The valid part of tile (m, n) is min(mb, N - m mb) x min(mb, N - n mb);
  * of a diagonal tile only the lower triangle counts.  For tile t = n NT + m:
- *   part[2 t ldt + i]       = sum_j |S(i, j)|                  (rows)
- *   part[(2 t + 1) ldt + j] = sum_i |S(i, j)|, diagonal excluded (columns)
+ *   part[(t CQ + q) ldt + i] = sum_j |S(i, j)|, j in piece q    (rows)
+ *   part[(TT CQ + t) ldt + j] = sum_i |S(i, j)|, diagonal excluded (columns)
+ * with TT = NT^2 and the tile's columns cut in CQ pieces,
  * so logical row r = m mb + i of the symmetric matrix is the sum of the
  * tile rows i of tiles (m, 0..m) and the tile columns i of (m..NT-1, m).
- * One workgroup per tile: wave w takes rows w*128 + 512 c, two rows per
- * lane (16-byte loads), eight columns in flight; each column's sum goes
- * through a wave reduction into an LDS row of the wave's own (no atomics:
- * the result does not depend on scheduling).  ldt a multiple of 128. */
+ * One workgroup per tile and piece: wave w of nw = min(4, ldt/128) takes rows
+ * w*128 + 128 nw c, two rows per lane (16-byte loads), eight columns in flight;
+ * each column's sum goes through a wave reduction into an LDS row of the
+ * wave's own (no atomics: the result does not depend on scheduling).  ldt a
+ * multiple of 128, CQ a power of two up to ldt/32. */
 __global__ __launch_bounds__(256) void copy_lower_norm_kernel(const double *S, double *W, int NT, int ldt, int mb,
-                                                              int N, double *part, const double *sc)
+                                                              int N, int CQ, double *part, const double *sc)
 {
-    extern __shared__ double cs[];      /* [4][ldt] column sums, one row per wave */
-    const int m = blockIdx.x % NT, n = blockIdx.x / NT;
+    extern __shared__ double cs[];      /* [nw][cq] column sums, one row per wave */
+    const int m = blockIdx.x % NT, n = blockIdx.x / NT, nw = blockDim.x >> 6;
     if (m < n) return;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const size_t ts = (size_t)ldt * ldt, t = (size_t)n * NT + m;
@@ -950,16 +987,17 @@ __global__ __launch_bounds__(256) void copy_lower_norm_kernel(const double *S, d
     double *dst = W + t * ts;
     const int vm = min(mb, N - m * mb), vn = min(mb, N - n * mb);
     const bool diag = (m == n);
-    double *csw = cs + (size_t)wave * ldt;
-    for (int j = lane; j < ldt; j += 64) csw[j] = 0.0;
+    const int cq = ldt / CQ, jq = blockIdx.y * cq;
+    double *csw = cs + wave * cq;
+    for (int j = lane; j < cq; j += 64) csw[j] = 0.0;
     __syncthreads();            /* lane 0 adds below into entries other lanes cleared */
-    for (int r0 = wave * 128; r0 < ldt; r0 += 512) {
+    for (int r0 = wave * 128; r0 < ldt; r0 += 128 * nw) {
         const int i = r0 + 2 * lane;
         double rs0 = 0.0, rs1 = 0.0;
         /* with sc: the copy is S A S (element (i, j) times s_i s_j, the
          * product of the two scales first), the sums stay those of A */
         const double sr0 = sc ? sc[m * ldt + i] : 1.0, sr1 = sc ? sc[m * ldt + i + 1] : 1.0;
-        for (int j0 = 0; j0 < ldt; j0 += 8) {
+        for (int j0 = jq; j0 < jq + cq; j0 += 8) {
             double2 v[8];
 #pragma unroll
             for (int u = 0; u < 8; ++u) v[u] = *reinterpret_cast<const double2 *>(src + (size_t)(j0 + u) * ldt + i);
@@ -980,31 +1018,62 @@ __global__ __launch_bounds__(256) void copy_lower_norm_kernel(const double *S, d
                 double c = (diag && i == j ? 0.0 : a0) + (diag && i + 1 == j ? 0.0 : a1);
 #pragma unroll
                 for (int off = 32; off > 0; off >>= 1) c += __shfl_xor(c, off);
-                if (lane == 0) csw[j] += c;
+                if (lane == 0) csw[j - jq] += c;
             }
         }
-        part[2 * t * ldt + i] = rs0;
-        part[2 * t * ldt + i + 1] = rs1;
+        part[(t * CQ + blockIdx.y) * ldt + i] = rs0;
+        part[(t * CQ + blockIdx.y) * ldt + i + 1] = rs1;
     }
     __syncthreads();
-    for (int j = threadIdx.x; j < ldt; j += 256)
-        part[(2 * t + 1) * ldt + j] = ((cs[j] + cs[ldt + j]) + cs[2 * ldt + j]) + cs[3 * ldt + j];
+    for (int j = threadIdx.x; j < cq; j += blockDim.x) {
+        double c = cs[j];
+        for (int w = 1; w < nw; ++w) c += cs[w * cq + j];
+        part[((size_t)NT * NT * CQ + t) * ldt + jq + j] = c;
+    }
 }
 
 /* rowsum[r], r < N: the symmetric matrix's absolute row sums from the
- * partials of copy_lower_norm_kernel, added in a fixed order */
-__global__ void norm_rows_kernel(const double *part, int NT, int ldt, int mb, int N, double *rowsum)
+ * partials of copy_lower_norm_kernel, added in a fixed order: 64 rows to a
+ * workgroup, wave w adds partials w, w + 8, ... of each (in one thread the
+ * (m + 1) CQ + NT - m loads were a chain: 34 us at NT = 16, CQ = 8, now 4.7) */
+__global__ __launch_bounds__(512) void norm_rows_kernel(const double *part, int NT, int ldt, int mb, int N, int CQ,
+                                                        double *rowsum)
 {
-    for (int r = blockIdx.x * blockDim.x + threadIdx.x; r < N; r += gridDim.x * blockDim.x) {
-        const int m = r / mb, i = r % mb;
-        double s = 0.0;
-        for (int n = 0; n <= m; ++n) s += part[2 * ((size_t)n * NT + m) * ldt + i];
-        for (int q = m; q < NT; ++q) s += part[(2 * ((size_t)m * NT + q) + 1) * ldt + i];
+    __shared__ double sum[8][64];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const int r = blockIdx.x * 64 + lane;
+    double s = 0.0;
+    if (r < N) {
+        const int m = r / mb, nrow = (m + 1) * CQ, n = nrow + NT - m;
+        const double *P = part + r % mb, *C = P + (size_t)NT * NT * CQ * ldt;
+#pragma unroll 4
+        for (int u = w; u < n; u += 8) {
+            const size_t row = ((size_t)(u / CQ) * NT + m) * CQ + u % CQ, col = (size_t)m * NT + m + u - nrow;
+            s += u < nrow ? P[row * ldt] : C[col * ldt];
+        }
+    }
+    sum[w][lane] = s;
+    __syncthreads();
+    if (w == 0 && r < N) {
+        for (int q = 1; q < 8; ++q) s += sum[q][lane];
         rowsum[r] = s;
     }
 }
 
-size_t copy_lower_norm_scratch(int NT, int ldt) { return (size_t)2 * NT * NT * ldt; }
+/* Column pieces of a tile: one, doubled while the launch has fewer than 4096
+ * workgroups (16 to a compute unit: each wave's loads and shuffles are a chain) and
+ * a piece stays 32 columns wide.  One piece against the rule: N = 1100, 128
+ * tiles 60 -> 20 us, 4096/256 118 -> 35, 8000/256 197 -> 138, 8000/512 286 ->
+ * 142, 16000/512 615 -> 541 (4.1 TB/s, near the rate of a copy); 2048
+ * workgroups left 8000/256 at 152 and 16000/512 at 557. */
+static int copy_norm_pieces(int NT, int ldt)
+{
+    int cq = 1;
+    while (NT * (NT + 1) / 2 * cq < 4096 && ldt / (2 * cq) >= 32) cq *= 2;
+    return cq;
+}
+
+size_t copy_lower_norm_scratch(int NT, int ldt) { return (size_t)(1 + copy_norm_pieces(NT, ldt)) * NT * NT * ldt; }
 
 int copy_lower_norm(const double *S, double *W, int NT, int ldt, int mb, int N, double *part, double *rowsum,
                     hipStream_t s, const double *sc)
@@ -1012,10 +1081,11 @@ int copy_lower_norm(const double *S, double *W, int NT, int ldt, int mb, int N, 
     if (NT <= 0 || ldt % 128 != 0 || ldt > COPY_NORM_MAX_LDT || mb <= 0 || mb > ldt || N <= (NT - 1) * mb ||
         N > NT * mb)
         return -1;
-    hipLaunchKernelGGL(copy_lower_norm_kernel, dim3((unsigned)(NT * NT)), dim3(256), (size_t)4 * ldt * sizeof(double),
-                       s, S, W, NT, ldt, mb, N, part, sc);
-    hipLaunchKernelGGL(norm_rows_kernel, dim3((unsigned)std::min(2048, (N + 255) / 256)), dim3(256), 0, s, part, NT,
-                       ldt, mb, N, rowsum);
+    const int cq = copy_norm_pieces(NT, ldt), nw = std::min(4, ldt / 128);
+    hipLaunchKernelGGL(copy_lower_norm_kernel, dim3((unsigned)(NT * NT), cq), dim3(64 * nw),
+                       (size_t)nw * (ldt / cq) * sizeof(double), s, S, W, NT, ldt, mb, N, cq, part, sc);
+    hipLaunchKernelGGL(norm_rows_kernel, dim3((N + 63) / 64), dim3(512), 0, s, part, NT, ldt,
+                       mb, N, cq, rowsum);
     return 0;
 }
 

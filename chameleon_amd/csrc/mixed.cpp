@@ -63,14 +63,11 @@ double norm_inf_sym(CHAM_desc_t *A)
     return r;
 }
 
-/* column maxima of X and R (transposed, nrp x rows) on the host, one
- * launch and one round trip; dwork holds 2 nrp doubles */
-void colmax_pair_host(const double *XT, const double *RT, int nrp, int rows, double *dwork, std::vector<double> &xn,
-                      std::vector<double> &rn)
+/* the column maxima of X and R that k::residual left in dwork (2 nrp
+ * doubles), on the host */
+void colmax_pair_host(const double *dwork, int nrp, std::vector<double> &xn, std::vector<double> &rn)
 {
     hipStream_t s = ctx()->s_main;
-    k::zero_ints((int *)dwork, 4 * nrp, s);
-    k::colmax2(XT, RT, nrp, nrp, rows, dwork, s);
     std::vector<double> h(2 * (size_t)nrp);
     CHX_HIP(hipMemcpyAsync(h.data(), dwork, 2 * (size_t)nrp * sizeof(double), hipMemcpyDeviceToHost, s));
     CHX_HIP(hipStreamSynchronize(s));
@@ -166,9 +163,9 @@ int backward_error(cham_uplo_t uplo, CHAM_desc_t *A, CHAM_desc_t *X, CHAM_desc_t
     double *XT = w, *BT = w + vb, *RT = w + 2 * vb, *nw = w + 3 * vb, *part = nw + 2 * (size_t)nrp;
     k::rhs_transpose((double *)MX->d, XT, NT, ldt, MX->ldt, MX->wdt, MX->nt, 1, s);
     k::rhs_transpose((double *)MB->d, BT, NT, ldt, MB->ldt, MB->wdt, MB->nt, 1, s);
-    k::residual((const double *)MA->d, NT, ldt, XT, BT, RT, nrp, part, s);
+    k::residual((const double *)MA->d, NT, ldt, XT, BT, RT, nrp, part, nw, nullptr, s);
     std::vector<double> xn, rn;
-    colmax_pair_host(XT, RT, nrp, rows, nw, xn, rn);
+    colmax_pair_host(nw, nrp, xn, rn);
     const double eps = std::ldexp(1.0, -53);
     double worst = 0.0;
     for (int j = 0; j < X->n; ++j) {
@@ -247,7 +244,10 @@ int mixed_posv(cham_uplo_t uplo, CHAM_desc_t *A, CHAM_desc_t *B, CHAM_desc_t *X,
         if (adaptive) tile_precision_map(Aw, NT, ldt, tss, dmap, s);
 
         k::rhs_transpose((double *)MB->d, BT, NT, ldt, MB->ldt, MB->wdt, MB->nt, 1, s);
-        CHX_HIP(hipMemcpyAsync(XT, BT, vb * sizeof(double), hipMemcpyDeviceToDevice, s));
+        if (scaled)
+            k::scale_bt(XT, BT, nrp, rows, sc, s);
+        else
+            CHX_HIP(hipMemcpyAsync(XT, BT, vb * sizeof(double), hipMemcpyDeviceToDevice, s));
         PotrfPlan p;
         p.A = Aw;
         p.NT = NT;
@@ -269,11 +269,13 @@ int mixed_posv(cham_uplo_t uplo, CHAM_desc_t *A, CHAM_desc_t *B, CHAM_desc_t *X,
          * the factorisation, sized for the rate of this precision's bulk
          * update (measured on MI355X, FP64-equivalent flop/s) */
         const bool overlap = potrf_solve_eligible(ldt);
-        if (scaled) k::scale_bt(XT, nrp, rows, sc, s);
+        SolvePlan sp;
         if (overlap) {
             /* FP32, BF16, BF16x3, FP8, per-tile (sized for its FP64 tiles) */
             static const double rate[5] = {98e12, 377e12, 205e12, 400e12, 60e12};
-            potrf_solve_run(p, XT, nrp, X->n, rate[prec]);
+            /* its block inverses and products serve the corrections too */
+            p.dinv = (double *)workspace((size_t)NT * (ldt / 64) * 64 * 64 * sizeof(double));
+            sp = potrf_solve_run(p, XT, nrp, X->n, rate[prec]);
         } else {
             potrf_run(p);
         }
@@ -282,13 +284,16 @@ int mixed_posv(cham_uplo_t uplo, CHAM_desc_t *A, CHAM_desc_t *B, CHAM_desc_t *X,
         if (info != 0 || *st->h_info == LP_RANGE) {
             it_count = -3;
         } else {
-            SolvePlan sp = solve_plan(Aw, NT, ldt, nrp, st->d_info, X->n);
-            if (!overlap) solve_bt(sp, Aw, NT, ldt, XT, nrp, st->d_info);
-            if (scaled) k::scale_bt(XT, nrp, rows, sc, s);
+            if (!overlap) {
+                sp = solve_plan(Aw, NT, ldt, nrp, st->d_info, X->n);
+                solve_bt(sp, Aw, NT, ldt, XT, nrp, st->d_info);
+            }
+            if (scaled) k::scale_bt(XT, XT, nrp, rows, sc, s);
             for (int it = 0; it <= ITERMAX; ++it) {
-                k::residual((const double *)MA->d, NT, ldt, XT, BT, RT, nrp, part, s);
+                /* RT: the residual, scaled for the solve of the correction */
+                k::residual((const double *)MA->d, NT, ldt, XT, BT, RT, nrp, part, nw, scaled ? sc : nullptr, s);
                 std::vector<double> xn, rn;
-                colmax_pair_host(XT, RT, nrp, rows, nw, xn, rn);
+                colmax_pair_host(nw, nrp, xn, rn);
                 bool ok = true;
                 worst = 0.0;
                 for (int j = 0; j < X->n; ++j) {
@@ -306,10 +311,8 @@ int mixed_posv(cham_uplo_t uplo, CHAM_desc_t *A, CHAM_desc_t *B, CHAM_desc_t *X,
                     break;
                 }
                 if (it == ITERMAX) break;
-                if (scaled) k::scale_bt(RT, nrp, rows, sc, s);
                 solve_bt(sp, Aw, NT, ldt, RT, nrp, st->d_info);
-                if (scaled) k::scale_bt(RT, nrp, rows, sc, s);
-                k::axpy(XT, RT, vb, s);
+                k::correct(XT, RT, nrp, rows, scaled ? sc : nullptr, s);
             }
             /* a strip-solve wait that ran out leaves its code in the info
              * flag: the refinement result is then not trusted */

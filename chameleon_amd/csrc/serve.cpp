@@ -578,9 +578,8 @@ void mixed_step(Server *s, Slot &sl, Job *job, bool first)
     double *sc = scptr(s, f);
     if (first) {
         CHX_HIP(hipMemcpyAsync(job->BT, sl.host, vb * sizeof(double), hipMemcpyHostToDevice, st));
-        CHX_HIP(hipMemcpyAsync(job->XT, job->BT, vb * sizeof(double), hipMemcpyDeviceToDevice, st));
         k::zero_ints(sl.d_info, 1, st);
-        k::scale_bt(job->XT, job->nrp, job->rows, sc, st);
+        k::scale_bt(job->XT, job->BT, job->nrp, job->rows, sc, st);
         const long long dper = (long long)(f->ldt / 64) * 4096;
         if (job->d128)
             k::dinv128(fptr(s, f), dptr(s, f), dper, 4096, 64, f->NT, f->ldt, job->d128, st);
@@ -588,19 +587,16 @@ void mixed_step(Server *s, Slot &sl, Job *job, bool first)
             k::strip_products(fptr(s, f), dptr(s, f), dper, 4096, 64, f->NT, f->ldt, job->ef, job->eb, st);
         solve_strips_lane(&sl.lane, fptr(s, f), dptr(s, f), f->NT, f->ldt, job->XT, job->nrp, sl.d_info, job->d128,
                           q->r.nrhs, job->ef, job->eb);
-        k::scale_bt(job->XT, job->nrp, job->rows, sc, st);
+        k::scale_bt(job->XT, job->XT, job->nrp, job->rows, sc, st);
     } else {
-        /* correction: X += A_lp^-1 R */
-        k::scale_bt(job->RT, job->nrp, job->rows, sc, st);
+        /* correction: X += A_lp^-1 R (RT: R scaled for it) */
         solve_strips_lane(&sl.lane, fptr(s, f), dptr(s, f), f->NT, f->ldt, job->RT, job->nrp, sl.d_info, job->d128,
                           q->r.nrhs, job->ef, job->eb);
-        k::scale_bt(job->RT, job->nrp, job->rows, sc, st);
-        k::axpy(job->XT, job->RT, vb, st);
+        k::correct(job->XT, job->RT, job->nrp, job->rows, sc, st);
     }
     /* FP64 residual on the kept lower tiles of A, column max-norms of X and R */
-    k::residual(optr(s, f), f->NT, f->ldt, job->XT, job->BT, job->RT, job->nrp, job->part, st);
-    k::zero_ints((int *)job->nw, 4 * job->nrp, st);
-    k::colmax2(job->XT, job->RT, job->nrp, job->nrp, job->rows, job->nw, st);
+    k::residual(optr(s, f), f->NT, f->ldt, job->XT, job->BT, job->RT, job->nrp, job->part, job->nw, sc,
+                st);
     CHX_HIP(hipMemcpyAsync(sl.host + job->host_off, job->nw, 2 * job->nrp * sizeof(double), hipMemcpyDeviceToHost,
                            st));
     job->stage = 1;
