@@ -51,42 +51,70 @@ __device__ __forceinline__ float bf16_to_float(unsigned short b) { return __uint
 /* Demote tiles (m, k), m0 <= m < m1, of the FP64 mirror into the panel
  * buffer.  F32: column-major floats, tile m at P + m*ts.  BF16 / BF16X3:
  * row-major BF16 (element (i, p) at p + i*ldt), hi plane at P + m*ts and,
- * for X3, lo plane at P + (NT + m)*ts (in BF16 elements). */
-__global__ __launch_bounds__(256) void panel_demote_kernel(const double *A, int NT, int ldt, int k, int m0,
-                                                            void *P, int mode)
+ * for X3, lo plane at P + (NT + m)*ts (in BF16 elements).
+ *
+ * Bound by memory.  A workgroup takes a 64 x 64 block (ldt is a multiple of
+ * 128): columns read as 16-byte loads of 64 adjacent rows, eight in flight per
+ * thread, and the BF16 planes turned in LDS so that rows go out as 128-byte
+ * lines.  Reading along the rows of the column-major tile (8 bytes of a line at a
+ * time) took 41 us at 63 tiles of 512 (100 beside a bulk update), this
+ * 30 (68). */
+template <int MODE>
+__global__ __launch_bounds__(256) void panel_demote_kernel(const double *A, int NT, int ldt, int k, int m0, void *P)
 {
     const size_t ts = (size_t)ldt * ldt;
     const int m = m0 + blockIdx.z;
     const double *T = A + ((size_t)k * NT + m) * ts;
-    const int r0 = blockIdx.x * 32, c0 = blockIdx.y * 32;
-    const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;
-    if (mode == 0) {
+    const int r0 = blockIdx.x * 64, c0 = blockIdx.y * 64;
+    const int rr = 2 * (threadIdx.x & 31), cc = threadIdx.x >> 5;
+    double2 v[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u)
+        v[u] = *reinterpret_cast<const double2 *>(T + (size_t)(c0 + cc + 8 * u) * ldt + r0 + rr);
+    if constexpr (MODE == 0) {
         float *D = (float *)P + (size_t)m * ts;
-        for (int jj = ty; jj < 32; jj += 8) {
-            if (r0 + tx >= ldt || c0 + jj >= ldt) continue;
-            const size_t e = (r0 + tx) + (size_t)(c0 + jj) * ldt;
-            D[e] = (float)T[e];
+#pragma unroll
+        for (int u = 0; u < 8; ++u)
+            *reinterpret_cast<float2 *>(D + (size_t)(c0 + cc + 8 * u) * ldt + r0 + rr) =
+                float2{(float)v[u].x, (float)v[u].y};
+    } else {
+        /* row r of a plane from word 33 r: 32 words and one of padding, so that
+         * neither the halfwords written down a column nor the rows read
+         * back meet in a bank more than twice */
+        __shared__ unsigned pl[MODE][64 * 33];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                /* split from the FP64 value for the lo part: hi = bf16(x), lo = bf16(x - hi) */
+                const double x = h ? v[u].y : v[u].x;
+                const unsigned short hb = bf16_bits((float)x);
+                const int e = 66 * (rr + h) + cc + 8 * u;
+                reinterpret_cast<unsigned short *>(pl[0])[e] = hb;
+                if constexpr (MODE == 2)
+                    reinterpret_cast<unsigned short *>(pl[1])[e] = bf16_bits((float)(x - (double)bf16_to_float(hb)));
+            }
         }
-        return;
-    }
-    unsigned short *H = (unsigned short *)P + (size_t)m * ts;
-    unsigned short *Lo = (unsigned short *)P + ((size_t)NT + m) * ts;
-    for (int jj = ty; jj < 32; jj += 8) {
-        const int i = r0 + jj, p = c0 + tx;
-        if (i >= ldt || p >= ldt) continue;
-        /* split from the FP64 value for the lo part: hi = bf16(x), lo = bf16(x - hi) */
-        const double x = T[i + (size_t)p * ldt];
-        const unsigned short hb = bf16_bits((float)x);
-        H[p + (size_t)i * ldt] = hb;
-        if (mode == 2) Lo[p + (size_t)i * ldt] = bf16_bits((float)(x - (double)bf16_to_float(hb)));
+        __syncthreads();
+#pragma unroll
+        for (int q = 0; q < MODE; ++q) {
+            unsigned short *D = (unsigned short *)P + ((size_t)q * NT + m) * ts;
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                const int r = (threadIdx.x >> 4) + 16 * u, w = 2 * (threadIdx.x & 15);
+                *reinterpret_cast<uint2 *>(D + (size_t)(r0 + r) * ldt + c0 + 2 * w) =
+                    uint2{pl[q][33 * r + w], pl[q][33 * r + w + 1]};
+            }
+        }
     }
 }
 
 void panel_demote(const double *A, int NT, int ldt, int k, int m0, int m1, void *P, int mode, hipStream_t s)
 {
     if (m1 <= m0) return;
-    dim3 grid((ldt + 31) / 32, (ldt + 31) / 32, m1 - m0);
-    hipLaunchKernelGGL(panel_demote_kernel, grid, dim3(256), 0, s, A, NT, ldt, k, m0, P, mode);
+    dim3 grid(ldt / 64, ldt / 64, m1 - m0);
+    auto *kern = mode == 0 ? panel_demote_kernel<0> : mode == 1 ? panel_demote_kernel<1> : panel_demote_kernel<2>;
+    hipLaunchKernelGGL(kern, grid, dim3(256), 0, s, A, NT, ldt, k, m0, P);
 }
 
 /* Tile-pair decoding shared by the update kernels (same enumeration as the
