@@ -1115,12 +1115,15 @@ void panel_factor(double *T, double *P, long long ts, int S, int ldt, double *di
  * systems are in work at once), so what counts is how far ahead they are asked
  * for and how often they are read.  A wavefront takes two 16-row blocks against
  * the same 64 shared rows, keeps four slices of both in flight, and solves its
- * rows while they are in registers.  With one block, one slice and a pass of
- * its own for the solves, the 20 000 systems of orders 16 to 1023 took 24.0 ms,
- * now 16.8; 1024 of order 1024 11.4 and 8.6 ms, 2048 of order 512 4.1 and 2.9.
+ * rows while they are in registers; the rows' old values come as the slices
+ * after the last, behind the products.  With one block, one slice, a pass of
+ * its own for the solves and the old values asked for at the end, the 20 000
+ * systems of orders 16 to 1023 took 24.0 ms, now 16.6; 1024 of order 1024 11.4
+ * and 8.5 ms (about 4 TB/s), 2048 of order 512 4.1 and 2.76, 4000 of order 300
+ * 1.76 and 1.70 by the old values alone.
  * A small batch is bound by the serial (b), 18 us per block before and 9 now
- * (the steps of the panel's chain): 4000 of order 64 366 and 191 us, one of
- * order 256 198 and 124. */
+ * (the steps of the panel's chain): 4000 of order 64 366 and 178 us, one of
+ * order 256 198 and 115. */
 
 struct PotrfJobs {
     double *A;               /* job j: matrix at A + off[j] (off null: A)               */
@@ -1143,8 +1146,10 @@ struct PotrfJobs {
  * wavefronts), goes to Db; rows below are solved with M in Db and stored.  The
  * 16-deep slices of the 64 shared rows (Y) are staged in LDS, double-buffered;
  * every wavefront streams its own rows (X; DIAG reads them from Y).  C is a
- * multiple of 64, so the ring of four slices needs no test; loads past the
- * last slice repeat it.  A block past the matrix reads rows li instead, and
+ * multiple of 64, so the ring of four slices needs no test, and the four slices
+ * after the last hold the old values of the block's own columns: they are in
+ * flight behind the last products (DIAG loads those of its lower blocks at the
+ * start).  Shared rows past the last slice repeat it.  A block past the matrix reads rows li instead, and
  * shared rows past the matrix (last block column) whatever follows in it:
  * neither is used.  FP32 products leave other columns in a slot than FP64
  * ones; their shared rows are read in an order (pi) that undoes it. */
@@ -1186,7 +1191,7 @@ __device__ __forceinline__ void jobs_update(double *T, int ldt, int C, int rb0, 
         for (int h = 0; h < YH; ++h) *reinterpret_cast<v2d *>(ys + buf * 16 * OB + h * (NT / 32) * OB) = r[h];
     };
     auto xload = [&](int st, double (&r)[NB][4]) {
-        const rsrc_t b = pf_rsrc(T + (size_t)(16 * min(st, S - 1)) * ldt);
+        const rsrc_t b = pf_rsrc(T + (size_t)(16 * st) * ldt);
 #pragma unroll
         for (int u = 0; u < NB; ++u)
 #pragma unroll
@@ -1224,13 +1229,15 @@ __device__ __forceinline__ void jobs_update(double *T, int ldt, int C, int rb0, 
             }
         }
     };
-    if (S > 0) {
-        yload(0, y[0]);
+    if (S > 0) yload(0, y[0]);
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            if (!DIAG) xload(j, x[j]);
-            if (j > 0) yload(j, y[j]);
-        }
+    for (int j = 0; j < 4; ++j) {
+        if (!DIAG) xload(j, x[j]);
+        else if (j <= wave && wave < nrb) xload(S + j, x[j]);
+    }
+    if (S > 0) {
+#pragma unroll
+        for (int j = 1; j < 4; ++j) yload(j, y[j]);
         ystore(0, y[0]);
         yload(4, y[0]);
         __syncthreads();
@@ -1245,41 +1252,30 @@ __device__ __forceinline__ void jobs_update(double *T, int ldt, int C, int rb0, 
             }
         }
     }
-    /* the old values of all blocks first, all in flight; of the diagonal block
-     * the lower 16 x 16 blocks only */
     const int vt = (li + lk * ldt) * 8;
-    v4d old[NB][4];
-#pragma unroll
-    for (int u = 0; u < NB; ++u) {
-        const int rb = min(rb0 + wave + NW * u, nrb - 1);
-        const rsrc_t t = pf_rsrc(T + C + 16 * rb + (size_t)C * ldt);
-#pragma unroll
-        for (int f = 0; f < 4; ++f)
-#pragma unroll
-            for (int s = 0; s < 4; ++s) old[u][f][s] = pf_ld(t, vt, (16 * (DIAG ? min(f, rb) : f) + 4 * s) * ldt * 8);
-    }
 #pragma unroll
     for (int u = 0; u < NB; ++u) {
         const int rb = rb0 + wave + NW * u;
         if (rb >= nrb) continue;
+        v4d old[4];
 #pragma unroll
         for (int f = 0; f < 4; ++f)
 #pragma unroll
-            for (int s = 0; s < 4; ++s) old[u][f][s] -= LP ? (double)accf[u][f][s] : acc[u][f][s];
+            for (int s = 0; s < 4; ++s) old[f][s] = x[f][u][s] - (LP ? (double)accf[u][f][s] : acc[u][f][s]);
         if constexpr (DIAG) {
 #pragma unroll
             for (int f = 0; f < 4; ++f)
                 if (f <= rb) {
 #pragma unroll
-                    for (int s = 0; s < 4; ++s) Db[pf_low(rb, f) + 64 * s + lane] = old[u][f][s];
+                    for (int s = 0; s < 4; ++s) Db[pf_low(rb, f) + 64 * s + lane] = old[f][s];
                 }
         } else {
-            pf_subst(Db, lane, old[u]);
+            pf_subst(Db, lane, old);
             const rsrc_t t = pf_rsrc(T + C + 16 * rb + (size_t)C * ldt);
 #pragma unroll
             for (int f = 0; f < 4; ++f)
 #pragma unroll
-                for (int s = 0; s < 4; ++s) pf_st(old[u][f][s], t, vt, (16 * f + 4 * s) * ldt * 8);
+                for (int s = 0; s < 4; ++s) pf_st(old[f][s], t, vt, (16 * f + 4 * s) * ldt * 8);
         }
     }
 }
