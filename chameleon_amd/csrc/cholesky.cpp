@@ -130,11 +130,21 @@ void potrf_run(const PotrfPlan &p)
             int *flags = lane_flags(L, k::panel_flags(ldt), 1, &epoch);
             unsigned *ctr = lane_counters(L);
             double *ws = lane_panel_scratch(L, k::panel_scratch(ldt));
+            /* the tiles below also in the precision of the trailing products
+             * (FP8 needs each tile's largest element first: a launch of its own) */
+            k::PanelLow low;
+            if (k + 1 < NT && p.lp_mode >= 0 && p.lp_mode != CHAMAMD_PREC_FP8) {
+                void *half = p.lp_mode == CHAMAMD_PREC_ADAPTIVE ? pbuf2(k) : pbuf(k);
+                if (p.lp_mode == CHAMAMD_PREC_FP32 || p.lp_mode == CHAMAMD_PREC_ADAPTIVE)
+                    low.f32 = (float *)pbuf(k) + (size_t)(k + 1) * ts;
+                if (p.lp_mode != CHAMAMD_PREC_FP32) low.hi = (unsigned short *)half + (size_t)(k + 1) * ts;
+                if (p.lp_mode == CHAMAMD_PREC_BF16X3) low.lo = (unsigned short *)half + ((size_t)NT + k + 1) * ts;
+            }
             timed(CHAMAMD_KERNEL_PANEL, f, sm, [&] {
                 k::panel_factor(tile(k, k), tile(std::min(k + 1, NT - 1), k), (long long)ts, NT - k - 1, ldt, dk,
-                                ws, flags, ctr, epoch, p.d_info, p.nb * k, nvalid, sm);
+                                ws, flags, ctr, epoch, p.d_info, p.nb * k, nvalid, sm, low);
             });
-            if (k + 1 < NT && p.lp_mode >= 0) demote(k);
+            if (k + 1 < NT && p.lp_mode == CHAMAMD_PREC_FP8) demote(k);
             return;
         }
         const int waves = potrf_waves(k);

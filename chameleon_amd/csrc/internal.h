@@ -305,10 +305,17 @@ void lacpy_tiles(const double *src, double *dst, int mt, int nt, int ldt, int wd
                  int M, int N, int uplo, hipStream_t s);
 /* chol.hip */
 void potrf_diag(double *Akk, int ldt, double *dinv, int iinfo, int nvalid, int *info, int waves, hipStream_t s);
+/* where panel_factor leaves the tiles below in the precision of the trailing
+ * products, each null or the place of the first tile below (panel_demote's layouts) */
+struct PanelLow {
+    float *f32 = nullptr;
+    unsigned short *hi = nullptr, *lo = nullptr;
+};
 /* scratch: panel_scratch doubles, flags: panel_flags of them, used by one
  * panel at a time */
 void panel_factor(double *T, double *P, long long ts, int S, int ldt, double *dinv, double *scratch, int *flags,
-                  unsigned *ctr, int epoch, int *info, int iinfo, int nvalid, hipStream_t s);
+                  unsigned *ctr, int epoch, int *info, int iinfo, int nvalid, hipStream_t s,
+                  const PanelLow &low = PanelLow());
 size_t panel_scratch(int ldt);
 int panel_flags(int ldt);
 void trsm_right_lower_trans(double *panel, int ntiles, size_t tile_stride, int ldt, const double *Lkk,

@@ -53,6 +53,15 @@ __device__ __forceinline__ double readlane_f64(double v, int l)
     return __builtin_bit_cast(double, ((unsigned long long)hi << 32) | lo);
 }
 
+/* round-to-nearest-even FP32 -> BF16 bits (finite inputs) */
+__device__ __forceinline__ unsigned short bf16_bits(float f)
+{
+    unsigned int u = __float_as_uint(f);
+    u += 0x7fffu + ((u >> 16) & 1u);
+    return (unsigned short)(u >> 16);
+}
+__device__ __forceinline__ float bf16_to_float(unsigned short b) { return __uint_as_float(((unsigned int)b) << 16); }
+
 __device__ __forceinline__ v4d zero4d() { v4d z = {0.0, 0.0, 0.0, 0.0}; return z; }
 __device__ __forceinline__ v4f zero4f() { v4f z = {0.f, 0.f, 0.f, 0.f}; return z; }
 

@@ -38,22 +38,14 @@ __device__ __forceinline__ int xcd_remap_m(int id, int total)
     return (x < rem) ? x * (per + 1) + local : rem * (per + 1) + (x - rem) * per + local;
 }
 
-/* round-to-nearest-even FP32 -> BF16 bits (finite inputs) */
-__device__ __forceinline__ unsigned short bf16_bits(float f)
-{
-    unsigned int u = __float_as_uint(f);
-    u += 0x7fffu + ((u >> 16) & 1u);
-    return (unsigned short)(u >> 16);
-}
-__device__ __forceinline__ float bf16_to_float(unsigned short b) { return __uint_as_float(((unsigned int)b) << 16); }
-
 /* ------------------------------------------------------------------ */
 /* Demote tiles (m, k), m0 <= m < m1, of the FP64 mirror into the panel
  * buffer.  F32: column-major floats, tile m at P + m*ts.  BF16 / BF16X3:
  * row-major BF16 (element (i, p) at p + i*ldt), hi plane at P + m*ts and,
  * for X3, lo plane at P + (NT + m)*ts (in BF16 elements).
  *
- * Bound by memory.  A workgroup takes a 64 x 64 block (ldt is a multiple of
+ * The fused panel stores these itself (panel_low in panel.hip); this is for
+ * panels factored by separate launches.  Bound by memory.  A workgroup takes a 64 x 64 block (ldt is a multiple of
  * 128): columns read as 16-byte loads of 64 adjacent rows, eight in flight per
  * thread, and the BF16 planes turned in LDS so that rows go out as 128-byte
  * lines.  Reading along the rows of the column-major tile (8 bytes of a line at a

@@ -345,6 +345,7 @@ struct PanelArgs {
     int epoch;
     int *info;
     int iinfo, nvalid;
+    PanelLow low;        /* tiles below in a lower precision (panel_factor_kernel<true>)   */
 };
 
 /* Buffer accesses relative to a tile: one per-lane offset register, the
@@ -958,12 +959,58 @@ __device__ __forceinline__ void panel_diag(const PanelArgs &a, PanelLds &L, int 
     pf_publish(a, ND + r, tid);
 }
 
-/* X(u, C) of the 64 rows at Rw in a tile below, every C, left-looking.  The
+/* The finished columns of block C of a 64-row unit u below (panel_rows' y) in
+ * the precision of the trailing products, from registers: a launch that read
+ * them back took 5 us of the chain at 256-row tiles and up to 68, beside a bulk
+ * update, at 512.  FP32 in the layout of the tile; BF16 row-major, a
+ * wavefront's 16 rows turned in its own part of Xs, which is idle between the
+ * last product and the next staging. */
+__device__ __forceinline__ void panel_low(const PanelArgs &a, PanelLds &L, const v4d (&y)[4], int u, int C, int wave,
+                                          int lane)
+{
+    const int li = lane & 15, lk = lane >> 4, ldt = a.ldt;
+    const size_t tile = (size_t)(u / a.ND) * a.ts;
+    const int row = 64 * (u % a.ND) + 16 * wave;
+    if (a.low.f32) {
+        const rsrc_t r = pf_rsrc(reinterpret_cast<const double *>(a.low.f32 + tile));
+        const int vo = (row + li + lk * ldt) * 4;
+#pragma unroll
+        for (int q = 0; q < 16; ++q)
+            __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint((float)y[q >> 2][q & 3]), r, vo, (16 * C + q) * 16 * ldt, 0);
+    }
+    if (a.low.hi) {
+        /* rows of 72 halfwords, so that 16-byte pieces stay aligned */
+        unsigned short *const S = reinterpret_cast<unsigned short *>(L.Xs + 1024 * wave);
+        for (int plane = 0; plane < (a.low.lo ? 2 : 1); ++plane) {
+#pragma unroll
+            for (int q = 0; q < 16; ++q) {
+                const double v = y[q >> 2][q & 3];
+                unsigned short b = bf16_bits((float)v);
+                if (plane) b = bf16_bits((float)(v - (double)bf16_to_float(b)));
+                S[72 * li + 4 * q + lk] = b;
+            }
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            const rsrc_t r = pf_rsrc(reinterpret_cast<const double *>((plane ? a.low.lo : a.low.hi) + tile));
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                const int i = (lane >> 3) + 8 * h, c = 8 * (lane & 7);
+                v2d w;
+                __builtin_memcpy(&w, S + 72 * i + c, sizeof w);
+                pf_st2(w, r, ((row + i) * ldt + c) * 2, 64 * C * 2);
+            }
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        }
+    }
+}
+
+/* X(u, C) of the 64 rows of unit u in the tiles below, every C, left-looking.  The
  * published blocks X(C, p) go through two LDS buffers, one barrier per block;
  * the loads of a block (and of the unit's own X(u, p)) are issued before the
  * products of the one before.  64-row blocks per product: 1.7 us of MFMAs. */
-__device__ __forceinline__ void panel_rows(const PanelArgs &a, PanelLds &L, double *Rw)
+template <bool LOW>
+__device__ __forceinline__ void panel_rows(const PanelArgs &a, PanelLds &L, int u)
 {
+    double *const Rw = a.P + (size_t)(u / a.ND) * a.ts + 64 * (u % a.ND);
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int li = lane & 15, lk = lane >> 4;
     const int ldt = a.ldt, ND = a.ND;
@@ -1015,6 +1062,7 @@ __device__ __forceinline__ void panel_rows(const PanelArgs &a, PanelLds &L, doub
         pf_subst(L.B[0], lane, y);
 #pragma unroll
         for (int q = 0; q < 16; ++q) pf_st(y[q >> 2][q & 3], rR, vr, (16 * C + q) * c4);
+        if constexpr (LOW) panel_low(a, L, y, u, C, wave, lane);
     }
 }
 
@@ -1022,6 +1070,7 @@ __device__ __forceinline__ void panel_rows(const PanelArgs &a, PanelLds &L, doub
  * D(L+1) (L > 0) and the blocks (r, L), r > L+1 */
 __host__ __device__ __forceinline__ int panel_units(int ND) { return ND > 1 ? ND * (ND - 1) / 2 + ND - 2 : 0; }
 
+template <bool LOW>
 __global__ __launch_bounds__(256, 2) void panel_factor_kernel(PanelArgs a)
 {
     __shared__ PanelLds L;
@@ -1052,8 +1101,7 @@ __global__ __launch_bounds__(256, 2) void panel_factor_kernel(PanelArgs a)
                 else panel_block(a, L, lev + 1 + (u > 1 ? u - (lev > 0) : u), lev);
             }
         } else {
-            const int u = t - 1 - a.nw;
-            panel_rows(a, L, a.P + (size_t)(u / a.ND) * a.ts + 64 * (u % a.ND));
+            panel_rows<LOW>(a, L, t - 1 - a.nw);
         }
     }
     __syncthreads();
@@ -1071,9 +1119,10 @@ size_t panel_scratch(int ldt)
 int panel_flags(int ldt) { return (ldt / 64) * (ldt / 64) + 1; }
 
 void panel_factor(double *T, double *P, long long ts, int S, int ldt, double *dinv, double *scratch, int *flags,
-                  unsigned *ctr, int epoch, int *info, int iinfo, int nvalid, hipStream_t s)
+                  unsigned *ctr, int epoch, int *info, int iinfo, int nvalid, hipStream_t s, const PanelLow &low)
 {
     PanelArgs a;
+    a.low = low;
     a.T = T; a.P = P; a.ts = ts; a.S = S; a.ldt = ldt; a.ND = ldt / 64;
     a.dinv = dinv; a.W = scratch; a.XW = scratch + (size_t)a.ND * PF_W; a.flags = flags; a.ctr = ctr; a.epoch = epoch;
     a.info = info; a.iinfo = iinfo; a.nvalid = nvalid;
@@ -1094,7 +1143,7 @@ void panel_factor(double *T, double *P, long long ts, int S, int ldt, double *di
     const int room = rows + least <= ncu ? ncu - rows : rows + least <= 2 * ncu ? 2 * ncu - rows : nu;
     a.nw = nu < room ? nu : room;
     const int grid = 1 + a.nw + a.ND * S;
-    hipLaunchKernelGGL(panel_factor_kernel, dim3(grid), dim3(256), 0, s, a);
+    hipLaunchKernelGGL((low.f32 || low.hi ? panel_factor_kernel<true> : panel_factor_kernel<false>), dim3(grid), dim3(256), 0, s, a);
 }
 
 /* ================================================================== */
