@@ -483,7 +483,8 @@ __global__ __launch_bounds__(256, 2) void strip_solve_kernel(StripArgs a)
 #pragma unroll
         for (int c = 0; c < NC; ++c) x[c] = zero4d();
 #pragma unroll
-        for (int pc = 0; pc < NPC; ++pc) {
+        for (int pi = 0; pi < NPC; ++pi) {
+            const int pc = fwd ? pi : NPC - 1 - pi;     /* the diagonal's chunk, the largest terms, last */
             if (pc < pc0 || pc >= pc1) continue;
             double xd[4][NC];
 #pragma unroll
@@ -504,7 +505,15 @@ __global__ __launch_bounds__(256, 2) void strip_solve_kernel(StripArgs a)
             __syncthreads();                     /* every wave is done with Xs */
             stage_store(xv);
             __syncthreads();
-            strip_mma<NC>(ev, Xb, lane, x);
+            /* summed by themselves: added to x one by one, each of the 64 small
+             * products rounded x (seven right-hand sides at N = 7003: error
+             * 8.9e-16 so, 7.1e-16 now) */
+            v4d ex[NC];
+#pragma unroll
+            for (int c = 0; c < NC; ++c) ex[c] = zero4d();
+            strip_mma<NC>(ev, Xb, lane, ex);
+#pragma unroll
+            for (int c = 0; c < NC; ++c) x[c] += ex[c];
         }
         {
             /* publication by completion: X_s is written with device-scope
@@ -796,8 +805,8 @@ __global__ __launch_bounds__(512, 1) void strip_narrow_kernel(NarrowArgs a)
 #pragma unroll
         for (int c = 0; c < NCV; ++c) xp[c] = 0.0;
 #pragma unroll
-        for (int i = 0; i < 32; ++i) {
-            const int p = 32 * kq + i;
+        for (int h = 0; h < 32; ++h) {
+            const int i = fwd ? h : 31 - h, p = 32 * kq + i;     /* the diagonal, the largest term, last */
 #pragma unroll
             for (int c = 0; c < NCV; ++c) xp[c] = fma(dreg[i], Acc[p * NCV + c], xp[c]);
         }
