@@ -994,7 +994,7 @@ void correct(double *XT, const double *DT, int nrp, int rows, const double *sc, 
  * w*128 + 128 nw c, two rows per lane (16-byte loads), eight columns in flight;
  * each column's sum goes through a wave reduction into an LDS row of the
  * wave's own (no atomics: the result does not depend on scheduling).  ldt a
- * multiple of 128, CQ a power of two up to ldt/32. */
+ * multiple of 128, a piece (ldt / CQ) a whole number of eight columns. */
 __global__ __launch_bounds__(256) void copy_lower_norm_kernel(const double *S, double *W, int NT, int ldt, int mb,
                                                               int N, int CQ, double *part, const double *sc)
 {
@@ -1082,14 +1082,15 @@ __global__ __launch_bounds__(512) void norm_rows_kernel(const double *part, int 
 
 /* Column pieces of a tile: one, doubled while the launch has fewer than 4096
  * workgroups (16 to a compute unit: each wave's loads and shuffles are a chain) and
- * a piece stays 32 columns wide.  One piece against the rule: N = 1100, 128
+ * a piece stays 32 columns wide and a multiple of the eight that are in flight
+ * (tiles of 1152 columns stop at 72, not 36).  One piece against the rule: N = 1100, 128
  * tiles 60 -> 20 us, 4096/256 118 -> 35, 8000/256 197 -> 138, 8000/512 286 ->
  * 142, 16000/512 615 -> 541 (4.1 TB/s, near the rate of a copy); 2048
  * workgroups left 8000/256 at 152 and 16000/512 at 557. */
 static int copy_norm_pieces(int NT, int ldt)
 {
     int cq = 1;
-    while (NT * (NT + 1) / 2 * cq < 4096 && ldt / (2 * cq) >= 32) cq *= 2;
+    while (NT * (NT + 1) / 2 * cq < 4096 && ldt / (2 * cq) >= 32 && ldt % (16 * cq) == 0) cq *= 2;
     return cq;
 }
 

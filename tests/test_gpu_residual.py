@@ -69,3 +69,10 @@ def test_copy_norm(ch, n, nb, nrhs):
     assert 0 <= it.value <= 3
     assert abs(be.value - ref.value) <= 1e-12 * ref.value, (be.value, ref.value)
     assert oracle.rel_frobenius(X, want) <= 1e-12
+
+
+@pytest.mark.parametrize("n,nb,nrhs", [(1152, 1152, 1), (2500, 1152, 5), (1400, 1408, 2), (3000, 1408, 1),
+                                       (1664, 1664, 1), (4000, 1920, 17)])
+def test_copy_norm_odd_multiples_of_128(ch, n, nb, nrhs):
+    """Tiles whose column pieces stop at an odd multiple of eight columns."""
+    test_copy_norm(ch, n, nb, nrhs)
