@@ -443,9 +443,10 @@ void dinv128(const double *A, const double *D, long long dts, long long doff, in
 void solve_coop(const double *A, const double *TN, const double *TT, double *BT, double *W, int NT, int ldt, int nrhs,
                 int trans, const int *info, hipStream_t s);
 /* with info != null, nothing is copied once *info is nonzero */
-/* ldb: tile rows of B, at most ldt (the rows of BT past them are zero) */
+/* ldb, wdt: tile rows and columns of B, ldt, wbt (0: wdt) those of BT; what only
+ * one of them has is padding, zero in BT and left alone in B */
 void rhs_transpose(double *Bm, double *BT, int NT, int ldt, int ldb, int wdt, int bnt, int to_bt, hipStream_t s,
-                   const int *info = nullptr);
+                   const int *info = nullptr, int wbt = 0);
 /* forward substitution of one tile row right after its panel (dposv) */
 /* the forward tile solve addresses a tile row of the factor and of the
  * right-hand sides with 32-bit buffer offsets */

@@ -1354,25 +1354,29 @@ void fwd_update(const double *A, double *BT, int k, int NT, int ldt, int nrp, co
 
 /* ------------------------------------------------------------------ */
 /* B mirror (NT x bnt tiles of ldb x wdt) <-> BT (nrhs_p x NT*ldt), with
- * nrhs_p = bnt * wdt; rows ldb .. ldt-1 of a tile row are zero in BT. */
-__global__ void rhs_transpose_kernel(double *Bm, double *BT, int NT, int ldt, int ldb, int wdt, int bnt, int to_bt,
-                                     const int *info)
+ * nrhs_p = bnt * wbt; rows and columns of a tile past either of the two sizes
+ * are padding, zero in BT and not touched in B. */
+__global__ void rhs_transpose_kernel(double *Bm, double *BT, int NT, int ldt, int ldb, int wdt, int wbt, int bnt,
+                                     int to_bt, const int *info)
 {
     __shared__ double S[32][33];
     if (info && *info != 0) return;   /* failed factorisation: B keeps its values */
-    const int nrp = bnt * wdt;
+    const int nrp = bnt * wbt;
     const int rows = NT * ldt;
     const int r0 = blockIdx.x * 32, c0 = blockIdx.y * 32;   /* rows of B, columns (rhs) of B */
     const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;
     auto baddr = [&](int r, int c) -> size_t {
-        const int m = r / ldt, i = r % ldt, n = c / wdt, j = c % wdt;
+        const int m = r / ldt, i = r % ldt, n = c / wbt, j = c % wbt;
         return ((size_t)n * NT + m) * ldb * wdt + i + (size_t)j * ldb;
     };
-    const bool rpad = ldb < ldt;
+    const bool pad = ldb < ldt || wdt < wbt;
+    auto has = [&](int r, int c) {
+        return r < rows && c < nrp && !(pad && (r % ldt >= ldb || c % wbt >= wdt));
+    };
     if (to_bt) {
         for (int jj = ty; jj < 32; jj += 8) {
             const int r = r0 + tx, c = c0 + jj;
-            S[tx][jj] = (r < rows && c < nrp && !(rpad && r % ldt >= ldb)) ? Bm[baddr(r, c)] : 0.0;
+            S[tx][jj] = has(r, c) ? Bm[baddr(r, c)] : 0.0;
         }
         __syncthreads();
         for (int jj = ty; jj < 32; jj += 8) {
@@ -1387,17 +1391,18 @@ __global__ void rhs_transpose_kernel(double *Bm, double *BT, int NT, int ldt, in
         __syncthreads();
         for (int jj = ty; jj < 32; jj += 8) {
             const int r = r0 + tx, c = c0 + jj;
-            if (r < rows && c < nrp && !(rpad && r % ldt >= ldb)) Bm[baddr(r, c)] = S[tx][jj];
+            if (has(r, c)) Bm[baddr(r, c)] = S[tx][jj];
         }
     }
 }
 
 void rhs_transpose(double *Bm, double *BT, int NT, int ldt, int ldb, int wdt, int bnt, int to_bt, hipStream_t s,
-                   const int *info)
+                   const int *info, int wbt)
 {
-    const int rows = NT * ldt, nrp = bnt * wdt;
+    if (wbt == 0) wbt = wdt;
+    const int rows = NT * ldt, nrp = bnt * wbt;
     dim3 grid((rows + 31) / 32, (nrp + 31) / 32);
-    hipLaunchKernelGGL(rhs_transpose_kernel, grid, dim3(256), 0, s, Bm, BT, NT, ldt, ldb, wdt, bnt, to_bt, info);
+    hipLaunchKernelGGL(rhs_transpose_kernel, grid, dim3(256), 0, s, Bm, BT, NT, ldt, ldb, wdt, wbt, bnt, to_bt, info);
 }
 
 /* Per-tile transpose of a batch of square tiles (TT -> TN). */

@@ -161,8 +161,9 @@ int backward_error(cham_uplo_t uplo, CHAM_desc_t *A, CHAM_desc_t *X, CHAM_desc_t
     const size_t pv = k::residual_scratch(NT, ldt, nrp);
     double *w = (double *)workspace2((3 * vb + 2 * (size_t)nrp + pv) * sizeof(double));
     double *XT = w, *BT = w + vb, *RT = w + 2 * vb, *nw = w + 3 * vb, *part = nw + 2 * (size_t)nrp;
+    /* the two mirrors may be padded differently (see mirror_alloc) */
     k::rhs_transpose((double *)MX->d, XT, NT, ldt, MX->ldt, MX->wdt, MX->nt, 1, s);
-    k::rhs_transpose((double *)MB->d, BT, NT, ldt, MB->ldt, MB->wdt, MB->nt, 1, s);
+    k::rhs_transpose((double *)MB->d, BT, NT, ldt, MB->ldt, MB->wdt, MB->nt, 1, s, nullptr, MX->wdt);
     k::residual((const double *)MA->d, NT, ldt, XT, BT, RT, nrp, part, nw, nullptr, s);
     std::vector<double> xn, rn;
     colmax_pair_host(nw, nrp, xn, rn);
@@ -333,7 +334,12 @@ int mixed_posv(cham_uplo_t uplo, CHAM_desc_t *A, CHAM_desc_t *B, CHAM_desc_t *X,
         /* plain FP64 factorisation and solve; A holds its factor */
         CHAMELEON_Sequence_Destroy(seq);
         CHAMELEON_Sequence_Create(&seq);
-        CHX_HIP(hipMemcpyAsync(MX->d, MB->d, MB->bytes, hipMemcpyDeviceToDevice, s));
+        /* square right-hand sides: the two mirrors may be padded differently (see mirror_alloc) */
+        if (MX->ldt == MB->ldt && MX->wdt == MB->wdt)
+            CHX_HIP(hipMemcpyAsync(MX->d, MB->d, MB->bytes, hipMemcpyDeviceToDevice, s));
+        else
+            k::lacpy_tiles((const double *)MB->d, (double *)MX->d, MB->mt, MB->nt, MB->ldt, MB->wdt, MX->ldt, MX->wdt,
+                           B->mb, B->nb, B->m, B->n, ChamUpperLower, s);
         MX->state = MB->state;
         MX->diag_identity = false;
         potrf_async(uplo, A, seq);

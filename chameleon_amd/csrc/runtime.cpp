@@ -185,8 +185,12 @@ static void mirror_alloc(CHAM_desc_t *A, Mirror *M)
      * and 751, N = 1000 nb = 80 3862 and 1169, nb = 100 3309 and 925, N = 2000
      * nb = 17 29.7 and 7.6 ms, N = 4000 nb = 200 9.5 and 3.3 ms.  Matrices
      * whose mirror would pass 16 GiB keep the small padding (16-column tiles
-     * grow 16 times), and so does one that finds no memory for the large. */
-    if (A->mb == A->nb && A->m == A->n && A->dtyp == ChamRealDouble && M->ldt % 64 != 0) {
+     * grow 16 times), and so does one that finds no memory for the large
+     * (two matrices of one tiling may then be padded differently: whatever
+     * works on both goes by each one's ldt and wdt).  CHAMAMD_PAD64=0: the
+     * small padding for all. */
+    const char *pad64 = getenv("CHAMAMD_PAD64");
+    if (A->mb == A->nb && A->m == A->n && A->dtyp == ChamRealDouble && M->ldt % 64 != 0 && !(pad64 && *pad64 == '0')) {
         const int t16 = M->ldt, t64 = (M->ldt + 63) & ~63;
         size(t64, t64);
         if (M->bytes <= (size_t)16 << 30 && hipMalloc(&M->d, M->bytes) == hipSuccess) {
