@@ -6,7 +6,7 @@
  * tile order, each tile padded to ldt x wdt elements (ldt = mb rounded up to
  * a multiple of 16, wdt likewise unless the matrix is a single tile column,
  * where wdt = n rounded up to 16; square double matrices mostly round up to
- * 64, see mirror_alloc in runtime.cpp).  Padding is zero off the diagonal tiles
+ * 64, see mirror_pads64 in runtime.cpp).  Padding is zero off the diagonal tiles
  * and the identity on the padded diagonal of diagonal tiles, so the padded
  * matrix has the same Cholesky factor as the real one with identity blocks
  * in the holes; every kernel therefore works on full ldt x ldt tiles.
@@ -163,6 +163,7 @@ int *strip_flags(int n, int launches, int *epoch);
 unsigned *panel_counters();
 
 Mirror *mirror_of(const CHAM_desc_t *A);
+bool mirror_pads64(int nt, int t16);
 /* Make the device mirror of A hold its current values in orientation
  * `state` (MIRROR_NORMAL or MIRROR_TRANS); uploads from host if needed.
  * lower_need: the caller reads and writes only the tiles m >= n (a Lower

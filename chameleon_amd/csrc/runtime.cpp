@@ -153,6 +153,36 @@ static Mirror *mirror_get(CHAM_desc_t *A)
     return M;
 }
 
+/* Whether a square matrix of nt x nt tiles, t16 rows each (a multiple of 16),
+ * is padded to tiles of whole 64x64 blocks.
+ *
+ * The fused panel, the strip solves and the 64-column updates want those;
+ * other tiles take one workgroup per diagonal tile, one wavefront per 16 rows
+ * below it and cooperative solves, at 240 us or more per tile column whatever
+ * the order, and longer with the tile.  The padding costs the flops of the
+ * larger order P instead of p: (P^3 - p^3) / 3, shared by P / t64 tile columns,
+ * so the line is drawn at a value of (P^3 - p^3) / P.  Resident dposv, tiles
+ * rounded to 16 / to 64, in ms, and that value in 1e8:
+ *   nb 16:  N 2000 29.5 / 7.0 (0.6), 4000 61 / 39 (2.5), 5500 84 / 94 (4.8),
+ *           8000 129 / 275 (10), 11000 211 / 702 (19)
+ *   nb 17:  4000 63 / 33 (2.0), 5500 91 / 79 (3.8), 8000 165 / 231 (8.0)
+ *   nb 32:  8000 65 / 39 (2.2), 11000 104 / 95 (4.2), 16000 184 / 275 (9.0)
+ *   nb 33:  11000 134 / 86 (2.6), 16000 283 / 251 (5.6)
+ *   nb 40:  11000 96 / 50 (1.8), 16000 190 / 144 (3.8), 23000 419 / 413 (7.8)
+ *   nb 72:  11000 59 / 47 (2.9), 16000 120 / 134 (6.2), 23000 265 / 375 (13)
+ *   nb 80:  11000 50 / 36 (2.4), 16000 97 / 99 (5.0), 23000 208 / 277 (10)
+ *   nb 100: 4000 11.4 / 2.4 (0.4), 23000 229 / 146 (2.9)
+ *   nb 144: 23000 163 / 159 (5.5); nb 200: 23000 162 / 138 (4.0)
+ *   nb 336: 23000 143 / 101 (2.3)
+ * (nb 33 loses a little by it: its 48-row tiles take the slowest updates).
+ * A matrix whose wider mirror would pass 16 GiB keeps the small padding. */
+bool mirror_pads64(int nt, int t16)
+{
+    if (t16 % 64 == 0) return false;
+    const double P = (double)nt * ((t16 + 63) & ~63), p = (double)nt * t16;
+    return P * P * sizeof(double) <= (double)((size_t)16 << 30) && P * P - p * p * p / P <= 4.5e8;
+}
+
 static void mirror_alloc(CHAM_desc_t *A, Mirror *M)
 {
     if (M->d) return;
@@ -177,23 +207,15 @@ static void mirror_alloc(CHAM_desc_t *A, Mirror *M)
         if (M->bytes == 0) M->bytes = 256;
     };
     size(M->ldt, M->wdt);
-    /* The fused panel, the strip solves and the 64-column updates want tiles
-     * of whole 64x64 blocks; other tiles take one workgroup per diagonal tile,
-     * one wavefront per 16 rows below it and cooperative solves, whose latency
-     * costs more than the added padding at every tile size: resident dposv, 16
-     * against 64, N = 96 in one tile 487 against 211 us, N = 611 nb = 40 4310
-     * and 751, N = 1000 nb = 80 3862 and 1169, nb = 100 3309 and 925, N = 2000
-     * nb = 17 29.7 and 7.6 ms, N = 4000 nb = 200 9.5 and 3.3 ms.  Matrices
-     * whose mirror would pass 16 GiB keep the small padding (16-column tiles
-     * grow 16 times), and so does one that finds no memory for the large
-     * (two matrices of one tiling may then be padded differently: whatever
-     * works on both goes by each one's ldt and wdt).  CHAMAMD_PAD64=0: the
-     * small padding for all. */
+    /* wider padding, unless there is no memory for it (two matrices of one
+     * tiling may then be padded differently: whatever works on both goes by
+     * each one's ldt and wdt).  CHAMAMD_PAD64=0: never. */
     const char *pad64 = getenv("CHAMAMD_PAD64");
-    if (A->mb == A->nb && A->m == A->n && A->dtyp == ChamRealDouble && M->ldt % 64 != 0 && !(pad64 && *pad64 == '0')) {
+    if (A->mb == A->nb && A->m == A->n && A->dtyp == ChamRealDouble && mirror_pads64(M->nt, M->ldt) &&
+        !(pad64 && *pad64 == '0')) {
         const int t16 = M->ldt, t64 = (M->ldt + 63) & ~63;
         size(t64, t64);
-        if (M->bytes <= (size_t)16 << 30 && hipMalloc(&M->d, M->bytes) == hipSuccess) {
+        if (hipMalloc(&M->d, M->bytes) == hipSuccess) {
             M->state = MIRROR_NONE;
             return;
         }
