@@ -546,9 +546,8 @@ __device__ __forceinline__ void pf_take16(double *Db, int i, int j, int c, int l
  * pivot d and the unscaled a_kj read from the diagonal lanes: only the
  * reciprocal (estimate, two Newton steps) is between a pivot and the next,
  * and the other lane reads go on beside it; the square roots scale all
- * columns at the end.  Returns the 1-based index of the first non-positive
- * pivot, 0 if none. */
-__device__ __forceinline__ int pf_col16(double (&a)[16], int lane)
+ * columns at the end (pf_scale16).  Returns lane j's pivot j, 1 in the others. */
+__device__ __forceinline__ double pf_col16(double (&a)[16], int lane)
 {
     double dv = 1.0;                     /* lane j: pivot j */
 #pragma unroll
@@ -566,6 +565,13 @@ __device__ __forceinline__ int pf_col16(double (&a)[16], int lane)
 #pragma unroll
         for (int k = j + 1; k < 16; ++k) a[k] = fma(w, s[k], a[k]);
     }
+    return dv;
+}
+
+/* The columns of pf_col16 scaled by the square roots of its pivots; returns the
+ * 1-based index of the first non-positive pivot, 0 if none. */
+__device__ __forceinline__ int pf_scale16(double (&a)[16], double dv)
+{
     const unsigned long long bad = __ballot(!(dv > 0.0));
     const double rs = rsqrt_f64(dv);
 #pragma unroll
@@ -579,7 +585,11 @@ __device__ __forceinline__ int pf_col16(double (&a)[16], int lane)
  * their place, the inverse of L(c, c) to the diagonal one's.  Every lane has one
  * place to read from and one to write to: as three kinds of lanes each with
  * loads, selects and stores of their own, a step was 2.1 us, with 1.2 for the
- * columns; now 1.6.  Returns the failing column or 0. */
+ * columns; now 1.6.  Returns the failing column or 0.
+ * A pivot whose reciprocal leaves the range of the type (it is infinite below
+ * 2^-1024) spoils the columns after it.  With one outside [2^-1000, 2^1000), and
+ * those that are not positive among them, the step is done again on the block
+ * times 2^128 or 2^-128, whose factor is 2^64 or 2^-64 times the block's. */
 __device__ __forceinline__ int pf_step16(double *Db, double *Ld, const double *Id, int c, int nr, int lane)
 {
     const int li = lane & 15, lk = lane >> 4;
@@ -587,14 +597,35 @@ __device__ __forceinline__ int pf_step16(double *Db, double *Ld, const double *I
     const double *const src = lk < nr ? Db + low : Id;
     double *const dst = (lk == 0 ? Ld + c * PF_BLK : Db + low) + li;
     const int flip = lk == nr ? 15 : 0;      /* the inverse's element (q, li) is at 16 q + (li ^ q) */
-    double v[16];
+    double v[16], dv;
+    auto store = [&]() {
+        if (lk <= nr) {
 #pragma unroll
-    for (int q = 0; q < 16; ++q) v[q] = src[li + 16 * q];
-    const int fail = pf_col16(v, lane);
-    if (lk <= nr) {
+            for (int q = 0; q < 16; ++q) dst[16 * q + ((li ^ (q & flip)) - li)] = v[q];
+        }
+    };
+    for (int e = 0;;) {
 #pragma unroll
-        for (int q = 0; q < 16; ++q) dst[16 * q + ((li ^ (q & flip)) - li)] = v[q];
+        for (int q = 0; q < 16; ++q) v[q] = src[li + 16 * q];
+        if (e != 0 && lk < nr) {
+#pragma unroll
+            for (int q = 0; q < 16; ++q) v[q] = ldexp(v[q], 2 * e);
+        }
+        dv = pf_col16(v, lane);
+        if (e != 0) {
+            const int fail = pf_scale16(v, dv);
+#pragma unroll
+            for (int q = 0; q < 16; ++q) v[q] = ldexp(v[q], lk < nr ? -e : e);
+            store();
+            return fail;
+        }
+        /* sign, exponent and the first bits: 2^-1000 is 0x01700000, 2^1000 0x7e700000 */
+        const unsigned hi = (unsigned)__double2hiint(dv);
+        if (__builtin_expect(__ballot(hi - 0x01700000u >= 0x7e700000u - 0x01700000u) == 0, 1)) break;
+        e = __ballot(dv >= 0x1p1000) ? -64 : 64;
     }
+    const int fail = pf_scale16(v, dv);
+    store();
     return fail;
 }
 
