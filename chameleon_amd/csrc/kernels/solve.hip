@@ -998,6 +998,9 @@ void dinv128(const double *A, const double *D, long long dts, long long doff, in
 {
     const int S = NT * ldt / NSR;
     if (S <= 0) return;
+    /* the products and the backward solve read the inverses 32 bytes at a time */
+    if ((uintptr_t)D128 % 32 != 0)
+        ::chx::fatal_hip(hipErrorInvalidValue, "dinv128: inverses not on 32 bytes", __FILE__, __LINE__);
     hipLaunchKernelGGL(dinv128_kernel, dim3(S), dim3(256), 0, s, A, D, dts, doff, ldd, NT, ldt, D128);
 }
 

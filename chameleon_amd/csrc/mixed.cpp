@@ -214,9 +214,10 @@ int mixed_posv(cham_uplo_t uplo, CHAM_desc_t *A, CHAM_desc_t *B, CHAM_desc_t *X,
         /* at the end, for the first solve (beside the factorisation): with
          * few right-hand sides the 128 x 128 strip inverses and their
          * predecessor products, else those of the MFMA strip solve */
+        const size_t ntss = ((size_t)NT * NT + 31) & ~(size_t)31;      /* what follows is read 32 bytes at a time */
         const size_t n128 = k::narrow_eligible(ldt, NT, X->n) ? 3 * (size_t)NT * ldt * 128 : 2 * (size_t)NT * ldt * 64;
         char *w = (char *)workspace2(abytes + npanel * pbytes + mapbytes +
-                                     (3 * vb + 2 * (size_t)nrp + pv + rows + (size_t)NT * NT + n128) * sizeof(double));
+                                     (3 * vb + 2 * (size_t)nrp + pv + rows + ntss + n128) * sizeof(double));
         double *Aw = (double *)w;
         unsigned char *dmap = (unsigned char *)(w + abytes + npanel * pbytes);
         double *BT = (double *)(w + abytes + npanel * pbytes + mapbytes), *XT = BT + vb, *RT = XT + vb, *nw = RT + vb,
@@ -258,9 +259,9 @@ int mixed_posv(cham_uplo_t uplo, CHAM_desc_t *A, CHAM_desc_t *B, CHAM_desc_t *X,
         p.d_info = st->d_info;
         p.lp_mode = prec;
         if (k::narrow_eligible(ldt, NT, X->n))
-            p.d128 = tss + (size_t)NT * NT;
+            p.d128 = tss + ntss;
         else
-            p.epred = tss + (size_t)NT * NT;     /* predecessor products of the first solve */
+            p.epred = tss + ntss;     /* predecessor products of the first solve */
         for (int i = 0; i < 4; ++i) p.P[i] = w + abytes + i * pbytes;
         if (adaptive) {
             for (int i = 0; i < 4; ++i) p.P2[i] = w + abytes + (4 + i) * pbytes;

@@ -76,3 +76,10 @@ def test_copy_norm(ch, n, nb, nrhs):
 def test_copy_norm_odd_multiples_of_128(ch, n, nb, nrhs):
     """Tiles whose column pieces stop at an odd multiple of eight columns."""
     test_copy_norm(ch, n, nb, nrhs)
+
+
+@pytest.mark.parametrize("n,nb,nrhs", [(1500, 512, 1), (1700, 384, 2), (3500, 512, 1)])
+def test_narrow_solve_behind_odd_tile_counts(ch, n, nb, nrhs):
+    """The strip inverses of one or two columns come after NT^2 tile norms, an odd
+    number of doubles here; the launch checks that they are on 32 bytes."""
+    test_copy_norm(ch, n, nb, nrhs)
