@@ -308,11 +308,18 @@ void trailing_update(double *A, int lmt, int ldt, int k, int n0, int n1, int NT,
      *                    S 32  (33792)      5314 / 4343 / 4200
      * and one tile column, ldt 320, K 320: 250 blocks 15 / 21 (the 64 x 64
      * blocks as they were before took 22), 50 blocks 7 / 16 (18); ldt 320, S 10,
-     * K 640 (1375 blocks) 119 / 128 (133). */
+     * K 640 (1375 blocks) 119 / 128 (133).
+     * CHAMAMD_SMALL_COLS=0: launches of single columns take the largest blocks
+     * that divide a tile. */
+    static const bool small_cols = [] {
+        const char *e = getenv("CHAMAMD_SMALL_COLS");
+        return !(e && atoi(e) == 0);
+    }();
+    const bool largest = ncol > 0 && !small_cols;
     const long long b64 = ((long long)npairs * ldt / 64) * ldt / 64;
-    if (ldt % 128 == 0 && b64 >= 80LL * ncu)
+    if (ldt % 128 == 0 && (largest || b64 >= 80LL * ncu))
         launch_update<128, 128, 32, 64, 16, 1>(A, lmt, ldt, k, kp, n0, NT, ncol, npairs, info, s, pmap);
-    else if (ldt % 64 == 0 && b64 >= 6LL * ncu)
+    else if (ldt % 64 == 0 && (largest || b64 >= 6LL * ncu))
         launch_update<64, 64, 32, 32, 16, 2>(A, lmt, ldt, k, kp, n0, NT, ncol, npairs, info, s, pmap);
     else if (ldt % 32 == 0)
         launch_update<32, 32, 16, 16, 32, 2>(A, lmt, ldt, k, kp, n0, NT, ncol, npairs, info, s, pmap);

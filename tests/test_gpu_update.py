@@ -44,3 +44,37 @@ def test_factor(ch, n, nb, uplo):
     D = torch.from_numpy(A).cuda()
     P = G @ G.T if uplo == LOWER else G.T @ G
     assert float((P - D).norm() / D.norm()) <= n * np.finfo(float).eps
+
+
+SMALL_COLS = """
+import sys
+import numpy as np
+import chameleon_amd as ch
+ch.init()
+n, nb = 2560, 256
+rng = np.random.default_rng(3)
+A = rng.uniform(-0.5, 0.5, (n, n))
+A = np.asfortranarray(A + A.T)
+A[np.diag_indices(n)] += float(n)
+seq = ch.Sequence()
+with ch.Desc.from_array(A, nb) as dA:
+    ch.check(ch.lib.CHAMELEON_dpotrf_Tile_Async(122, dA.ptr, seq.ptr, seq.req))
+    assert seq.wait() == 0
+    np.save(sys.argv[1], dA.to_array(n, n))
+"""
+
+
+def test_column_blocks_switch(tmp_path):
+    """CHAMAMD_SMALL_COLS=0 (large blocks in the lookahead columns, read once per
+    process): the same sums, so the same bits."""
+    import os
+    import subprocess
+    import sys
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    out = []
+    for v in ("1", "0"):
+        path = str(tmp_path / ("factor%s.npy" % v))
+        env = dict(os.environ, CHAMAMD_SMALL_COLS=v, PYTHONPATH=root)
+        subprocess.run([sys.executable, "-c", SMALL_COLS, path], check=True, env=env, timeout=100)
+        out.append(np.load(path))
+    assert np.array_equal(out[0], out[1])

@@ -56,3 +56,24 @@ def test_padding_is_bounded(lib):
         for nt in (1, 2, 7, 30, 100, 400, 1500, 4000):
             if rule(nt, t):
                 assert t % 64 and (nt * (-(-t // 64) * 64)) ** 2 * 8 <= 16 << 30
+
+
+SWITCHES = ["CHAMELEON_TILE_SIZE", "CHAMELEON_INNER_BLOCK_SIZE", "CHAMELEON_TRANSLATION_MODE", "CHAMELEON_GERED_ACC",
+            "CHAMELEON_LOOKAHEAD", "CHAMAMD_PAIRS", "CHAMAMD_PANEL", "CHAMAMD_SMALL_COLS", "CHAMAMD_PAD64",
+            "CHAMAMD_FWD_TAIL", "CHAMAMD_SERVE_SMALL", "CHAMAMD_SERVE_LANES", "CHAMAMD_BATCH_GRAPHS",
+            "CHAMAMD_XFER_THREADS", "CHAMAMD_XFER_ZC", "CHAMAMD_ATOMIC_UPDATE"]
+
+
+@pytest.mark.parametrize("name", SWITCHES)
+def test_documented_switches_are_read(name):
+    """Every environment variable that the documents offer is named in a source."""
+    import os
+    import chameleon_amd as ch
+    src = os.path.join(os.path.dirname(ch.LIB_PATH), "csrc")
+    for folder, _, files in os.walk(src):
+        for f in files:
+            with open(os.path.join(folder, f)) as h:
+                text = h.read()
+            if '("%s"' % name in text:
+                return
+    raise AssertionError(name)
