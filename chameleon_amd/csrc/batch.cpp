@@ -80,9 +80,9 @@ struct CHAMAMD_batch_s {
     double *ra_host = nullptr, *ra_dev = nullptr;   /* pinned, and as the device addresses it            */
     size_t ra_cap = 0, ra_pos = 0;                  /* elements, and where system ra_next lies           */
     int ra_next = 0, ra_end = 0, ra_run = 0;        /* systems [ra_next, ra_end) are there; fetched in a row */
-    std::vector<long long> ra_off;                  /* per user index, packed offsets (count + 1)        */
+    /* behind the elements, in the same allocation: packed offsets (count + 1) and slots per user index */
+    long long *ra_off = nullptr, *d_raoff = nullptr;
     int *d_slot = nullptr;
-    long long *d_raoff = nullptr;
 };
 
 namespace {
@@ -228,11 +228,12 @@ bool ra_fill(CHAMAMD_batch_t *b, int i, hipStream_t s)
 {
     if (b->ra_run < RA_FROM || b->count - i < (b->ra_host ? 2 : RA_FROM)) return false;
     if (!b->ra_host) {
-        b->ra_off.resize(b->count + 1);
-        b->ra_off[0] = 0;
-        for (int u = 0; u < b->count; ++u)
-            b->ra_off[u + 1] = b->ra_off[u] + (long long)b->n[b->slot[u]] * b->nrhs[b->slot[u]];
-        const size_t bytes = std::min(RA_BYTES, (size_t)b->ra_off[b->count] * sizeof(double));
+        size_t elems = 0;
+        for (int u = 0; u < b->count; ++u) elems += (size_t)b->n[u] * b->nrhs[u];
+        elems = std::min(RA_BYTES / sizeof(double), elems);
+        /* (the device reads the tables across the bus, so that nothing is taken
+         * of its memory, which may be full) */
+        const size_t bytes = elems * sizeof(double) + (b->count + 1) * sizeof(long long) + b->count * sizeof(int);
         if (hipHostMalloc((void **)&b->ra_host, bytes, hipHostMallocMapped) != hipSuccess) {
             (void)hipGetLastError();
             b->ra_host = nullptr;
@@ -240,9 +241,14 @@ bool ra_fill(CHAMAMD_batch_t *b, int i, hipStream_t s)
             return false;
         }
         CHX_HIP(hipHostGetDevicePointer((void **)&b->ra_dev, b->ra_host, 0));
-        b->ra_cap = bytes / sizeof(double);
-        b->d_slot = upload(b->slot);
-        b->d_raoff = upload(b->ra_off);
+        b->ra_cap = elems;
+        b->ra_off = (long long *)(b->ra_host + elems);
+        b->d_raoff = (long long *)(b->ra_dev + elems);
+        b->d_slot = (int *)(b->d_raoff + b->count + 1);
+        b->ra_off[0] = 0;
+        for (int u = 0; u < b->count; ++u)
+            b->ra_off[u + 1] = b->ra_off[u] + (long long)b->n[b->slot[u]] * b->nrhs[b->slot[u]];
+        memcpy(b->ra_off + b->count + 1, b->slot.data(), b->count * sizeof(int));
     }
     int e = i;
     while (e < b->count && e - i < b->ra_run && b->ra_off[e + 1] - b->ra_off[i] <= (long long)b->ra_cap) ++e;
@@ -504,8 +510,7 @@ int CHAMAMD_Batch_Destroy(CHAMAMD_batch_t **batch)
     if (ctx()) CHX_HIP(hipStreamSynchronize(ctx()->s_main));
     drop_graphs(b);
     void *ptrs[] = {b->dA, b->dB, b->dD, b->d_np, b->d_n, b->d_nrhs, b->d_info, b->d_queue, b->d_aoff, b->d_boff,
-                    b->d_doff, b->dW, b->dX, b->dR, b->d_anrm, b->d_berr, b->d_state, b->d_iters,
-                    b->d_slot, b->d_raoff};
+                    b->d_doff, b->dW, b->dX, b->dR, b->d_anrm, b->d_berr, b->d_state, b->d_iters};
     for (void *p : ptrs)
         if (p) CHX_HIP(hipFree(p));
     if (b->ra_host) CHX_HIP(hipHostFree(b->ra_host));

@@ -80,3 +80,23 @@ def test_fetch_in_any_order(ch, count, hi, nrhs_hi):
     for i in range(count // 2, count):
         same(i)
     ch.check(L.CHAMAMD_Batch_Destroy(ctypes.byref(b)))
+
+
+def test_fetch_takes_no_device_memory(ch):
+    """The read-ahead works where the device's memory is full: none of it is taken."""
+    import torch
+    count = 200000                                           # tables of 2.4 MB
+    n = np.ones(count, dtype=np.int32)
+    ip = ctypes.POINTER(ctypes.c_int)
+    b = ctypes.c_void_p()
+    L = ch.lib
+    ch.check(L.CHAMAMD_Batch_Create(ctypes.byref(b), count, n.ctypes.data_as(ip), n.ctypes.data_as(ip)))
+    ch.check(L.CHAMAMD_dplrnt_batch(b, 5))
+    x = np.empty(100)
+    ch.check(L.CHAMAMD_Batch_GetB(b, 0, ctypes.c_void_p(x.ctypes.data), 1))
+    free = torch.cuda.mem_get_info()[0]
+    for i in range(1, 100):
+        ch.check(L.CHAMAMD_Batch_GetB(b, i, ctypes.c_void_p(x.ctypes.data + 8 * i), 1))
+    assert torch.cuda.mem_get_info()[0] == free
+    ch.check(L.CHAMAMD_Batch_Destroy(ctypes.byref(b)))
+    assert (x == [oracle.dplrnt(1, 1, 5 + i)[0, 0] for i in range(100)]).all()
