@@ -1012,11 +1012,11 @@ __device__ __forceinline__ void panel_low(const PanelArgs &a, PanelLds &L, const
     const size_t tile = (size_t)(u / a.ND) * a.ts;
     const int row = 64 * (u % a.ND) + 16 * wave;
     if (a.low.f32) {
-        const rsrc_t r = pf_rsrc(reinterpret_cast<const double *>(a.low.f32 + tile));
+        const rsrc_t r = pf_rsrc(reinterpret_cast<const double *>(a.low.f32 + tile + (size_t)64 * C * ldt));
         const int vo = (row + li + lk * ldt) * 4;
 #pragma unroll
         for (int q = 0; q < 16; ++q)
-            __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint((float)y[q >> 2][q & 3]), r, vo, (16 * C + q) * 16 * ldt, 0);
+            __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint((float)y[q >> 2][q & 3]), r, vo, q * 16 * ldt, 0);
     }
     if (a.low.hi) {
         /* rows of 72 halfwords, so that 16-byte pieces stay aligned */
@@ -1030,13 +1030,13 @@ __device__ __forceinline__ void panel_low(const PanelArgs &a, PanelLds &L, const
                 S[72 * li + 4 * q + lk] = b;
             }
             __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-            const rsrc_t r = pf_rsrc(reinterpret_cast<const double *>((plane ? a.low.lo : a.low.hi) + tile));
+            const rsrc_t r = pf_rsrc(reinterpret_cast<const double *>((plane ? a.low.lo : a.low.hi) + tile + (size_t)row * ldt));
 #pragma unroll
             for (int h = 0; h < 2; ++h) {
                 const int i = (lane >> 3) + 8 * h, c = 8 * (lane & 7);
                 v2d w;
                 __builtin_memcpy(&w, S + 72 * i + c, sizeof w);
-                pf_st2(w, r, ((row + i) * ldt + c) * 2, 64 * C * 2);
+                pf_st2(w, r, (i * ldt + c) * 2, 64 * C * 2);
             }
             __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
         }
@@ -1054,18 +1054,21 @@ __device__ __forceinline__ void panel_rows(const PanelArgs &a, PanelLds &L, int 
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int li = lane & 15, lk = lane >> 4;
     const int ldt = a.ldt, ND = a.ND;
-    const rsrc_t rR = pf_rsrc(Rw);
+    /* offsets from column block p of the rows: those from the first one would
+     * pass 32 bits in tiles beyond 16384 */
+    auto block = [&](int p) { return pf_rsrc(Rw + (size_t)64 * p * ldt); };
     const int vr = (16 * wave + li + lk * ldt) * 8, c4 = 4 * ldt * 8;
     for (int C = 0; C < ND; ++C) {
+        const rsrc_t rC = block(C);
         v4d acc[4] = {zero4d(), zero4d(), zero4d(), zero4d()}, y[4];
         double av[16];
 #pragma unroll
-        for (int q = 0; q < 16; ++q) av[q] = pf_ld(rR, vr, (16 * C + q) * c4);
+        for (int q = 0; q < 16; ++q) av[q] = pf_ld(rC, vr, q * c4);
         if (C > 0) {
             const rsrc_t ry = pf_rsrc(pf_xw(a, C, 0));
             double x[16], yst[16];
 #pragma unroll
-            for (int q = 0; q < 16; ++q) x[q] = pf_ld(rR, vr, q * c4);
+            for (int q = 0; q < 16; ++q) x[q] = pf_ld(block(0), vr, q * c4);
             /* X(C, C-2) is published after every X(C, p) before it; X(C, C-1)
              * comes last, from the chain */
             if (!pf_wait<16>(a, C * ND + max(C - 2, 0), tid, &L.s_int)) return;
@@ -1082,7 +1085,7 @@ __device__ __forceinline__ void panel_rows(const PanelArgs &a, PanelLds &L, int 
 #pragma unroll
                     for (int h = 0; h < 16; ++h) yst[h] = pf_ld<true>(ry, tid * 8, (p + 1) * PF_X * 8 + h * 2048);
 #pragma unroll
-                    for (int q = 0; q < 16; ++q) xn[q] = pf_ld(rR, vr, (16 * (p + 1) + q) * c4);
+                    for (int q = 0; q < 16; ++q) xn[q] = pf_ld(block(p + 1), vr, q * c4);
                 }
                 pf_mma(cur, lane, x, acc);
                 if (p + 1 < C) {
@@ -1101,7 +1104,7 @@ __device__ __forceinline__ void panel_rows(const PanelArgs &a, PanelLds &L, int 
         __syncthreads();
         pf_subst(L.B[0], lane, y);
 #pragma unroll
-        for (int q = 0; q < 16; ++q) pf_st(y[q >> 2][q & 3], rR, vr, (16 * C + q) * c4);
+        for (int q = 0; q < 16; ++q) pf_st(y[q >> 2][q & 3], rC, vr, q * c4);
         if constexpr (LOW) panel_low(a, L, y, u, C, wave, lane);
     }
 }
