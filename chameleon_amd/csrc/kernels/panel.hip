@@ -303,7 +303,8 @@ void trsm_right_lower_trans(double *panel, int ntiles, size_t tile_stride, int l
  * waves' share of each step is cut so that wave 0 never waits for them: it did
  * for 0.8 us in the first and 0.5 in the second step, for the stores behind
  * M(C)'s flag and for R(C+1).  With many tiles below, the FP64 MFMAs are the
- * bound (36 products of 64^3 per row unit, 1.9 us each).
+ * bound (36 products of 64^3 per row unit, 1.7 us each at the full rate of a
+ * compute unit).
  *
  * Publication: a flag set to this launch's epoch after the data was written
  * with device-scope (coherent) stores and every wave has waited for its own
@@ -1046,7 +1047,7 @@ __device__ __forceinline__ void panel_low(const PanelArgs &a, PanelLds &L, const
 /* X(u, C) of the 64 rows of unit u in the tiles below, every C, left-looking.  The
  * published blocks X(C, p) go through two LDS buffers, one barrier per block;
  * the loads of a block (and of the unit's own X(u, p)) are issued before the
- * products of the one before.  64-row blocks per product: 1.7 us of MFMAs. */
+ * products of the one before.  A product is 1.7 us of MFMAs. */
 template <bool LOW>
 __device__ __forceinline__ void panel_rows(const PanelArgs &a, PanelLds &L, int u)
 {
@@ -1407,7 +1408,8 @@ __global__ __launch_bounds__(POTRF_WAVES * 64, 2) void potrf_jobs_kernel(PotrfJo
         asm volatile("" : "+v"(tid));
         const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), li = lane & 15, lk = lane >> 4;
         const int W = min(OB, np - C), nfb = W >> 4;
-        /* a last block column narrower than 64 goes on as if identity */
+        /* of a last block column narrower than 64 the blocks past the matrix hold
+         * finite values; whatever is formed from them is masked */
         if (nfb < 4) {
             for (int e = tid; e < PF_LOW; e += NT) {
                 const int b = e >> 8, i = b < 1 ? 0 : b < 3 ? 1 : b < 6 ? 2 : 3;
