@@ -589,8 +589,9 @@ __device__ __forceinline__ int pf_scale16(double (&a)[16], double dv)
  * columns; now 1.6.  Returns the failing column or 0.
  * A pivot whose reciprocal leaves the range of the type (it is infinite below
  * 2^-1024) spoils the columns after it.  With one outside [2^-1000, 2^1000), and
- * those that are not positive among them, the step is done again on the block
- * times 2^128 or 2^-128, whose factor is 2^64 or 2^-64 times the block's. */
+ * those that are not positive among them, the step is done again on S A S and
+ * the rows below (and of the identity) times S, S the powers of two next to
+ * a_qq^-1/2: the factor is S L then, and the rows come out as they should. */
 __device__ __forceinline__ int pf_step16(double *Db, double *Ld, const double *Id, int c, int nr, int lane)
 {
     const int li = lane & 15, lk = lane >> 4;
@@ -605,25 +606,32 @@ __device__ __forceinline__ int pf_step16(double *Db, double *Ld, const double *I
             for (int q = 0; q < 16; ++q) dst[16 * q + ((li ^ (q & flip)) - li)] = v[q];
         }
     };
-    for (int e = 0;;) {
+    for (bool scaled = false;; scaled = true) {
+        int er = 0;                          /* the exponent of this row of S A S */
 #pragma unroll
         for (int q = 0; q < 16; ++q) v[q] = src[li + 16 * q];
-        if (e != 0 && lk < nr) {
+        if (scaled) {
 #pragma unroll
-            for (int q = 0; q < 16; ++q) v[q] = ldexp(v[q], 2 * e);
+            for (int q = 0; q < 16; ++q) {
+                const double d = readlane_f64(v[q], q);
+                const int e = d > 0.0 && d < __builtin_inf() ? -(__builtin_amdgcn_frexp_exp(d) >> 1) : 0;
+                v[q] = ldexp(v[q], e);
+                if (lane == q) er = e;
+            }
+#pragma unroll
+            for (int q = 0; q < 16; ++q) v[q] = ldexp(v[q], er);
         }
         dv = pf_col16(v, lane);
-        if (e != 0) {
+        if (scaled) {
             const int fail = pf_scale16(v, dv);
 #pragma unroll
-            for (int q = 0; q < 16; ++q) v[q] = ldexp(v[q], lk < nr ? -e : e);
+            for (int q = 0; q < 16; ++q) v[q] = ldexp(v[q], -er);
             store();
             return fail;
         }
         /* sign, exponent and the first bits: 2^-1000 is 0x01700000, 2^1000 0x7e700000 */
         const unsigned hi = (unsigned)__double2hiint(dv);
         if (__builtin_expect(__ballot(hi - 0x01700000u >= 0x7e700000u - 0x01700000u) == 0, 1)) break;
-        e = __ballot(dv >= 0x1p1000) ? -64 : 64;
     }
     const int fail = pf_scale16(v, dv);
     store();

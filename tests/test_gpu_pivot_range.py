@@ -74,6 +74,29 @@ def test_one_tiny_pivot(ch, last):
     assert np.abs(F / np.sqrt(np.diag(d)).max(axis=0) - np.eye(n)).max() <= 1e-15
 
 
+@pytest.mark.parametrize("n,nb,uplo", [(60, 64, LOWER), (150, 64, UPPER), (300, 200, LOWER)])
+def test_rows_of_every_scale(ch, n, nb, uplo):
+    """D L0 L0^T D with powers of two from 2^-512 to 2^507 in D: both ends of the range in one
+    16-column step, each row as exact as without D."""
+    print("[case] rows of every scale", n, nb, uplo, flush=True)
+    _, _, L0, _ = matrix(n, 0)
+    rng = np.random.default_rng(2 * n)
+    k = rng.integers(-512, 508, n)
+    k[[3, 9]] = 507, -512
+    X = rng.integers(-3, 4, (n, 2)).astype(float)
+    A = np.asfortranarray(np.ldexp(L0 @ L0.T, k[:, None] + k))
+    B = np.asfortranarray(np.ldexp(L0 @ (L0.T @ X), k[:, None]))
+    seq = ch.Sequence()
+    with ch.Desc.from_array(A, nb) as dA, ch.Desc.from_array(B, nb) as dB:
+        ch.check(ch.lib.CHAMELEON_dposv_Tile_Async(uplo, dA.ptr, dB.ptr, seq.ptr, seq.req))
+        assert seq.wait() == 0
+        F, Y = dA.to_array(n, n), dB.to_array(n, 2)
+    seq.destroy()
+    F = np.tril(F) if uplo == LOWER else np.triu(F).T
+    assert np.abs(np.ldexp(F, -k[:, None]) - L0).max() <= 4.0 * 1e-13
+    assert np.abs(np.ldexp(Y, k[:, None]) - X).max() <= 3.0 * 1e-12
+
+
 def test_not_positive_after_a_tiny_pivot(ch):
     n, nb = 100, 100
     d = np.full(n, 2.0 ** -1040)
